@@ -34,17 +34,16 @@ class ConvEngine {
   void transform_green(const zd* G, bool g0, hipStream_t s);
   // chi(Nk,Nw,Nchi,Nchi) <- bubble of the transformed Fg (and, if tail, minus
   // the G0 bubble plus the analytic tau reference).  Thresholds at 1e-9.
-  void chi0(zd* chi, double temp, bool tail, const double* eig_d, const zd* uni_d, const double* eig_h,
-            const zd* uni_h, const int64_t* invk, double mu, hipStream_t s, bool apply_threshold = true);
+  void chi0(zd* chi, double temp, bool tail, const double* eig_d, const zd* uni_d, double mu, hipStream_t s,
+            bool apply_threshold = true);
   // The tail-corrected chi0 of an FP32 engine: conv[G] - conv[G0] at grid
   // precision, the analytic tau reference and its sawtooth term through an
   // FP64 engine (tau_reference), combined in FP64 in (q, i nu)
-  void chi0_split_tail(zd* chi, double temp, const double* eig_d, const zd* uni_d, const double* eig_h,
-                       const zd* uni_h, const int64_t* invk, double mu, hipStream_t s);
+  void chi0_split_tail(zd* chi, double temp, const double* eig_d, const zd* uni_d, double mu, hipStream_t s);
   // chi(pair) += -(1/(T Nkall)) ref[G0](pair) + J(pair) sawc for every
   // irreducible pair (no partner copies), at this engine's precision
-  void tau_reference(zd* chi, double temp, const double* eig_d, const zd* uni_d, double mu, const std::vector<zd>& J,
-                     const zd* sawc_d, hipStream_t s);
+  void tau_reference(zd* chi, double temp, const double* eig_d, const zd* uni_d, double mu, const zd* J, const zd* sawc_d,
+                     hipStream_t s);
   // sigma(Nk,Nw,No,No) <- (T/Nkall) sum_pairs V (*) G, using Fg; thresholds at 1e-9
   void sigma(zd* sig, const zd* V, const double* S_h, const double* C_h, double temp, hipStream_t s,
              bool apply_threshold = true);
@@ -63,9 +62,10 @@ class ConvEngine {
   void tau_grids(cpx<R>* ta, cpx<R>* tb, int a, int b, const double* eig_d, const zd* uni_d, double mu, double mu2,
                  bool diff, double temp, hipStream_t s);
 
-  // tail constants J (per chi pair, [l + Nchi*m]) at mu and the sawtooth table (built once)
-  void tail_constants(double temp, const double* eig_h, const zd* uni_h, const int64_t* invk, double mu,
-                      std::vector<zd>& J, DBuf<zd>& sawc_d, hipStream_t s) const;
+  // tail constants J (per chi pair, [l + Nchi*m]) at mu and the sawtooth
+  // table (built once), in device memory
+  void tail_constants(double temp, const double* eig_d, const zd* uni_d, double mu, DBuf<zd>& J, DBuf<zd>& sawc_d,
+                      hipStream_t s) const;
 
   // ---- increments from a fixed reference (mixed-precision FLEX): the
   // transforms of a reference iterate are held at grid precision and every
@@ -84,7 +84,7 @@ class ConvEngine {
   // transformed differences in Fd (F0d, TAd, TBd).
   void chi0_increment(zd* chi, const zd* chi_base, const zd* G, const zd* Gref, const zd* G0, const zd* G0ref,
                       double temp, bool tail, const double* eig_d, const zd* uni_d, double mu, double mu_ref,
-                      const std::vector<zd>& dJ, const zd* sawc_d, hipStream_t s);
+                      const zd* dJ, const zd* sawc_d, hipStream_t s);
   // sig <- sig_base + Sigma[V, G] - Sigma[Vref, Gref] (unthresholded); uses
   // Fr/Fd of the preceding chi0_increment and FVr.
   // dv_ready: the FP32 vertex difference V - Vref is already in dv_buffer()
@@ -113,6 +113,9 @@ class ConvEngine {
   const FFTPlan<R>* p3;
   DBuf<cpx<R>> Fg, F0g, TA, TB, work, tmp, acc, Vft, Ff;
   DBuf<cpx<R>> Fr, Fd, F0r, F0d, TAr, TBr, TAd, TBd, FVr;  // increment mode (r: reference, d: difference)
+  DBuf<zd> rhobar;         // BZ-averaged free density matrix of the tail constants
+  std::vector<int> ol_h;   // orbital pairs (o1, o2) per chi index, and their device copy
+  DBuf<int> ol_d;
   DBuf<cpx<R>> Mg;  // mirrored Fg (G(-r,-t)): the second factor of the bubble, read in place
   DBuf<cpx<R>> Lff;  // the two legs of one anomalous-bubble pair
   // Sigma through the accumulating last pass: the sources of one output
@@ -133,7 +136,7 @@ class ConvEngine {
   double tlive_frac = 1.0;
   bool tlive_built = false;
   // the gather of a spatial-first inverse transform
-  GatherStore<R> gather_sf(zd* dst, double w, zd J, const zd* sawc, int acc, hipStream_t s);
+  GatherStore<R> gather_sf(zd* dst, double w, const zd* J, const zd* sawc, int acc, hipStream_t s);
   std::vector<std::array<int, 2>> gap_pairs;
   std::vector<SocBosonLoad<R>> soc_vload;  // per gap pair of a spinful basis
   bool vft_cached = false;

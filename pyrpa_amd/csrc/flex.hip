@@ -89,7 +89,7 @@ static void chi0_driver(zd* chi_h, const zd* Gk, const int64_t* kmap, const int6
   if (tail) { up(eig_d, eig, (size_t)No * Nk); up(uni_d, uni, (size_t)No * No * Nk); }
   ConvEngine<R> eng(mesh, op);
   eng.transform_green(G.p, false, s);
-  eng.chi0(chi.p, temp, tail, eig_d.p, uni_d.p, eig, uni, invk, mu, s);
+  eng.chi0(chi.p, temp, tail, eig_d.p, uni_d.p, mu, s);
   if (stoner) {
     up(S_d, S, (size_t)Nchi * Nchi);
     *stoner = stoner_factor(chi.p, Nk, Nw, Nchi, S_d.p, s, 0.0, alpha);
@@ -200,7 +200,7 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
   // mu_ref, Jref).  In the increment iterations the vertex overwrites
   // chi_acc in place, and chi_ref takes over the buffer `chi` held.
   DBuf<zd> chi_acc, chi_ref, Vref, sig_acc, sig_ref, Gref, G0, G0ref, sawc_d;
-  std::vector<zd> Jref, Jcur, dJ;
+  DBuf<zd> Jref, Jcur, dJ;
   double mu_ref = 0.0;
   long head = 1;
   if (const char* e = getenv("GMOD_MIXED_HEAD")) head = std::max(1L, atol(e));
@@ -367,7 +367,8 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
     mu_ref = mu;
     if (A.sw_tail) {
       green0(G0ref.p, eig_d.p, uni_d.p, mu, T, Nk, (int)Nw, No, s);
-      Jref = Jcur;
+      if (Jref.n != Jcur.n) Jref.alloc(Jcur.n);
+      copy(Jref.p, Jcur.p, Jcur.n, s);
     }
     e32->set_reference(Gref.p, G0ref.p, A.sw_tail, eig_d.p, uni_d.p, mu_ref, T, s);
     e32->set_vertex_reference(Vref.p, A.Smat, A.Cmat, s);
@@ -392,18 +393,18 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
     const bool rebase = inc && rebase_c > 0.0 && it > 1 && esterr < rebase_c * dist_ref;
     if (!inc) {
       eng->transform_green(G.p, false, s);
-      eng->chi0(mixed ? chi_acc.p : chi.p, T, A.sw_tail, eig_d.p, uni_d.p, A.eig, A.uni, A.invk, mu, s, false);
+      eng->chi0(mixed ? chi_acc.p : chi.p, T, A.sw_tail, eig_d.p, uni_d.p, mu, s, false);
     } else {
       if (A.sw_tail) {
         green0(G0.p, eig_d.p, uni_d.p, mu, T, Nk, (int)Nw, No, s);
-        e32->tail_constants(T, A.eig, A.uni, A.invk, mu, Jcur, sawc_d, s);
-        dJ.resize(Jcur.size());
-        for (size_t i = 0; i < Jcur.size(); ++i) dJ[i] = Jcur[i] - Jref[i];
+        e32->tail_constants(T, eig_d.p, uni_d.p, mu, Jcur, sawc_d, s);
+        if (dJ.n != Jcur.n) dJ.alloc(Jcur.n);
+        lincomb(dJ.p, Jcur.p, 1.0, Jref.p, -1.0, Jcur.n, s);
       }
       // slots the gather does not keep hold the last vertex: restore them
       if (!mesh.complete) copy(chi_acc.p, chi_ref.p, nC, s);
       e32->chi0_increment(chi_acc.p, chi_ref.p, G.p, Gref.p, G0.p, G0ref.p, T, A.sw_tail, eig_d.p, uni_d.p, mu,
-                          mu_ref, dJ, sawc_d.p, s);
+                          mu_ref, dJ.p, sawc_d.p, s);
       if (rebase) copy(chi_ref.p, chi_acc.p, nC, s);  // chi0 of the new reference, before the vertex overwrites it
     }
     stoner = stoner_factor(chi_src, Nk, Nw, Nchi, S_d.p, s, 1e-9, A.soc ? -1.0 : 1.0);
@@ -448,7 +449,7 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
         threshold_copy(sig.p, sig_acc.p, nS, 1e-9, s);
         if (it >= head) {
           if (verbose) printf("[FLEX] switching to FP32 increments\n");
-          if (A.sw_tail) eng->tail_constants(T, A.eig, A.uni, A.invk, mu, Jcur, sawc_d, s);
+          if (A.sw_tail) eng->tail_constants(T, eig_d.p, uni_d.p, mu, Jcur, sawc_d, s);
           eng.reset();  // FP64 grids are no longer needed
           e32.reset(new ConvEngine<float>(mesh, op));
           // chi_ref takes the buffer of the vertex, which is copied to Vref first
@@ -957,7 +958,7 @@ static void nonlin_eliash_driver(const NonlinIn& A, zd* delta_io, zd* sigma_out,
   // VS <- chi0_S, VD <- chi0_C from G and F (ffeliash.f90:459-489)
   auto chi0sc = [&]() {
     eng.transform_green(G.p, false, s);
-    eng.chi0(VS.p, T, false, nullptr, nullptr, nullptr, nullptr, nullptr, 0.0, s, true);
+    eng.chi0(VS.p, T, false, nullptr, nullptr, 0.0, s, true);
     eng.chi0_ff(VD.p, F.p, A.prt, singlet, T, s);
     sum_diff(VS.p, VD.p, (long)nC, s);
   };
@@ -1824,7 +1825,7 @@ extern "C" void get_chi0sc_(gmod_z* Vsigma, gmod_z* Vdelta, const gmod_z* Gk, co
   up(F, (const zd*)fk, nS);
   auto run = [&](auto eng) {
     eng->transform_green(G.p, false, s);
-    eng->chi0(cs.p, *temp, false, nullptr, nullptr, nullptr, nullptr, nullptr, 0.0, s, true);
+    eng->chi0(cs.p, *temp, false, nullptr, nullptr, 0.0, s, true);
     eng->chi0_ff(cc.p, F.p, prt, *sw_pair, *temp, s);
   };
   if (ctx().precision >= 1) run(std::make_unique<ConvEngine<float>>(mesh, op));

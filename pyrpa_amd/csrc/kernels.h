@@ -587,7 +587,7 @@ template <typename R>
 struct GatherStore {
   zd* dst;
   double w;
-  zd J;
+  const zd* J;  // read when sawc is set (device memory)
   const zd* sawc;
   int acc;
   MeshDev m;
@@ -615,7 +615,8 @@ struct GatherStore {
     const zd sw = (sawc ? sawc : dst)[sawc ? tt : 0];
     q.old = acc ? old : zd(0, 0);
     q.bv = base ? bv : zd(0, 0);
-    q.js = sawc ? J * sw : zd(0, 0);
+    const zd jv = (sawc ? J : dst)[0];
+    q.js = sawc ? jv * sw : zd(0, 0);
     return q;
   }
   __device__ void commit(unsigned, unsigned, const Pre& q, cpx<R> v) const {
@@ -651,6 +652,15 @@ void mul_acc(cpx<R>* acc, const cpx<R>* A, const cpx<R>* B, bool first, long n, 
 template <typename R>
 void tau_ref_grids(cpx<R>* ta, cpx<R>* tb, const double* eig, const zd* uni, int a, int b, int No, double mu,
                    double mu2, bool diff, double beta, double dtau, const MeshDev& m, hipStream_t s);
+
+// Tail constants of chi0 (fchi.f90:731-772), on the device: rb[m + No l] =
+// the full-zone average of sum_n U_mn conj(U_ln) f_n(mu) (transposed at -k);
+// J[l + Nchi m] of every orbital pair (ol: o1, o2 per chi index); the sawtooth
+// correction i / nu_j - dtau sum_s e^{i nu_j tau_s} (1/2 - s/M), j < Nw
+void tail_density(zd* rb, const double* eig, const zd* uni, int No, double mu, double beta, const MeshDev& m,
+                  hipStream_t s);
+void tail_jumps(zd* J, const zd* rb, const int* ol, int No, int Nchi, hipStream_t s);
+void sawtooth(zd* sawc, int Nw, double temp, hipStream_t s);
 
 // ---- elementwise
 void conj_copy(zd* dst, const zd* src, long n, hipStream_t s);

@@ -194,6 +194,82 @@ template void tau_ref_grids<float>(cpx<float>*, cpx<float>*, const double*, cons
 template void tau_ref_grids<double>(cpx<double>*, cpx<double>*, const double*, const zd*, int, int, int, double,
                                     double, bool, double, double, const MeshDev&, hipStream_t);
 
+// ------------------------------------------------------------------ tail constants
+// One work-group per density-matrix element, summed over the full zone in a
+// fixed order.  Latency-bound (No^2 groups); it replaces a host loop of
+// Nkall No^2 + Nk No^3 steps and a direct sawtooth sum of Nw x 2 Nw phases
+// that kept the GPU idle in every iteration (1 orbital, 64x64 x 1024: 32.1 ms
+// an iteration, now 2.4 ms; 32x32 x 256: 2.7 ms, now 0.9 ms).
+__global__ void __launch_bounds__(256)
+k_tail_density(zd* __restrict__ rb, const double* __restrict__ eig, const zd* __restrict__ U, int No, double mu,
+               double beta, MeshDev m) {
+  __shared__ double sr[256], si[256];
+  const int a = blockIdx.x % No, b = blockIdx.x / No;
+  zd acc(0, 0);
+  for (long sp = threadIdx.x; sp < m.Nkall; sp += 256) {
+    const int kf = m.kf_s[sp];
+    const long k = kf >> 1;
+    zd v(0, 0);
+    for (int n = 0; n < No; ++n) {
+      const double xi = eig[n + No * k] - mu, e = exp(-beta * fabs(xi));
+      const double f = (xi >= 0 ? e : 1.0) / (1.0 + e);
+      v += U[a + No * (n + No * k)] * conj(U[b + No * (n + No * k)]) * f;
+    }
+    acc += (kf & 1) ? conj(v) : v;
+  }
+  sr[threadIdx.x] = acc.re;
+  si[threadIdx.x] = acc.im;
+  __syncthreads();
+  for (int o = 128; o > 0; o >>= 1) {
+    if ((int)threadIdx.x < o) {
+      sr[threadIdx.x] += sr[threadIdx.x + o];
+      si[threadIdx.x] += si[threadIdx.x + o];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) rb[blockIdx.x] = zd(sr[0] / (double)m.Nkall, si[0] / (double)m.Nkall);
+}
+void tail_density(zd* rb, const double* eig, const zd* uni, int No, double mu, double beta, const MeshDev& m,
+                  hipStream_t s) {
+  hipLaunchKernelGGL(k_tail_density, dim3((unsigned)(No * No)), dim3(256), 0, s, rb, eig, uni, No, mu, beta, m);
+  GMOD_CHECK_LAUNCH();
+}
+
+__global__ void k_tail_jumps(zd* J, const zd* rb, const int* ol, int No, int Nchi) {
+  for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < Nchi * Nchi; e += gridDim.x * blockDim.x) {
+    const int l = e % Nchi, m = e / Nchi;
+    const int a13 = ol[2 * l], b13 = ol[2 * m], a42 = ol[2 * m + 1], b42 = ol[2 * l + 1];
+    zd v(0, 0);
+    if (a13 == b13) v += rb[a42 + No * b42];
+    if (a42 == b42) v -= rb[a13 + No * b13];
+    J[e] = v;
+  }
+}
+void tail_jumps(zd* J, const zd* rb, const int* ol, int No, int Nchi, hipStream_t s) {
+  hipLaunchKernelGGL(k_tail_jumps, dim3(nblocks((long)Nchi * Nchi)), dim3(TPB), 0, s, J, rb, ol, No, Nchi);
+  GMOD_CHECK_LAUNCH();
+}
+
+// sum_s e^{i x s} (1/2 - s/M) = -1 / (e^{i x} - 1) = 1/2 + (i/2) cot(x/2) for
+// x = 2 pi j / M, j > 0, so the correction is -dtau/2 + (i dtau/2) (1/y - cot y)
+// with y = pi j / M; the difference by its power series where it cancels
+__global__ void k_sawtooth(zd* out, int Nw, double beta) {
+  const double h = beta / (4.0 * (double)Nw);  // dtau / 2
+  for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < Nw; j += gridDim.x * blockDim.x) {
+    const double y = 3.141592653589793238462643383279 * (double)j / (2.0 * (double)Nw), q = y * y;
+    double d;
+    if (y < 0.25)
+      d = y * (1.0 / 3 + q * (1.0 / 45 + q * (2.0 / 945 + q * (1.0 / 4725 + q * (2.0 / 93555 + q * (1382.0 / 638512875))))));
+    else
+      d = 1.0 / y - cos(y) / sin(y);
+    out[j] = zd(-h, h * d);
+  }
+}
+void sawtooth(zd* sawc, int Nw, double temp, hipStream_t s) {
+  hipLaunchKernelGGL(k_sawtooth, dim3(nblocks(Nw)), dim3(TPB), 0, s, sawc, Nw, 1.0 / temp);
+  GMOD_CHECK_LAUNCH();
+}
+
 // ------------------------------------------------------------------ elementwise
 __global__ void k_conj_copy(zd* dst, const zd* src, long n) {
   for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x)

@@ -128,7 +128,7 @@ extern "C" void gmod_regrid_sigma(gmod_z* sig_f, const gmod_z* sig_c, const int6
                            (int)Nx_f, (int)Ny_f, (int)Nz_f, nslot, (double)Nkall_f / (double)Nkall_c);
         GMOD_CHECK_LAUNCH();
         pf.exec_fused(GridLoad<double>{gf.p, (unsigned)Nkall_f},
-                      GatherStore<double>{df.p + NkNw_f * (a + (long)No * b), 1.0, zd(0, 0), nullptr, 0, mdf}, gf.p,
+                      GatherStore<double>{df.p + NkNw_f * (a + (long)No * b), 1.0, nullptr, nullptr, 0, mdf}, gf.p,
                       tmp.p, +1, 1.0 / (double)Nkall_f, s);
       }
     // the outermost coarse frequency is replaced by the tail unless the fine
