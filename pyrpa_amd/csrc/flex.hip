@@ -23,10 +23,7 @@ struct Seed {
 static Seed g_seed;
 static double g_stats[16];
 
-static void check_err(DBuf<int>& err, hipStream_t s, const char* where) {
-  int h = 0;
-  err.download(&h, 1, s);
-  GMOD_HIP(hipStreamSynchronize(s));
+static void raise_err(int h, const char* where) {
   if (h) {
     std::string w = where;
     if (h & 1) throw Error(w + ": zgesv failed (singular RPA denominator)");
@@ -36,6 +33,31 @@ static void check_err(DBuf<int>& err, hipStream_t s, const char* where) {
     throw Error(w + ": device error");
   }
 }
+
+static void check_err(DBuf<int>& err, hipStream_t s, const char* where) {
+  int h = 0;
+  err.download(&h, 1, s);
+  GMOD_HIP(hipStreamSynchronize(s));
+  raise_err(h, where);
+}
+
+// device time between two points of the stream, read after a wait
+struct EventPair {
+  hipEvent_t a = nullptr, b = nullptr;
+  EventPair() {
+    GMOD_HIP(hipEventCreate(&a));
+    GMOD_HIP(hipEventCreate(&b));
+  }
+  ~EventPair() {
+    if (a) (void)hipEventDestroy(a);
+    if (b) (void)hipEventDestroy(b);
+  }
+  double seconds() const {
+    float ms = 0;
+    GMOD_HIP(hipEventElapsedTime(&ms, a, b));
+    return 1e-3 * ms;
+  }
+};
 
 struct Upload {
   hipStream_t s;
@@ -49,27 +71,30 @@ struct Upload {
 // Stoner factor: max_q max Re eig(chi0(q,0) S) (fchi.f90:352-399); thr > 0:
 // of the thresholded chi0 (the first frequency slice is copied with it)
 // (spinful basis: max Re eig(-chi0(q,0) V), fchi0withsoc.f90:156-198, alpha = -1)
+// err (optional): the caller's error flag instead of one of its own; a bit
+// that an earlier Dyson inverse left in it is raised first
 static double stoner_factor(const zd* chi, long Nk, long Nw, int Nchi, const double* S_d, hipStream_t s,
-                            double thr = 0.0, double alpha = 1.0) {
+                            double thr = 0.0, double alpha = 1.0, int* err = nullptr) {
   DBuf<double> out(Nk);
-  DBuf<int> err(1);
-  err.zero(s);
+  DBuf<int> own;
+  if (!err) {
+    own.alloc(1);
+    own.zero(s);
+    err = own.p;
+  }
   DBuf<zd> slice;
   if (thr > 0.0) {
     slice.alloc((size_t)Nk * Nchi * Nchi);
     threshold_slice(slice.p, chi, Nk, Nk * Nw, (long)Nchi * Nchi, thr, s);
-    max_re_eig(out.p, slice.p, BatchLayout{1, Nk}, Nk, Nchi, S_d, alpha, err.p, s);
+    max_re_eig(out.p, slice.p, BatchLayout{1, Nk}, Nk, Nchi, S_d, alpha, err, s);
   } else {
-    max_re_eig(out.p, chi, BatchLayout{1, Nk * Nw}, Nk, Nchi, S_d, alpha, err.p, s);
+    max_re_eig(out.p, chi, BatchLayout{1, Nk * Nw}, Nk, Nchi, S_d, alpha, err, s);
   }
-  check_err(err, s, "ckchi");
-  std::vector<double> h(Nk);
-  out.download(h.data(), Nk, s);
-  GMOD_HIP(hipStreamSynchronize(s));
-  double best = -1.0e5;
-  for (long i = 0; i < Nk; ++i)
-    if (h[i] > best) best = h[i];
-  return best;
+  int h = 0;
+  const double best = max_value(out.p, Nk, s, err, &h);
+  raise_err(h & 4, "getinv");
+  raise_err(h, "ckchi");
+  return std::max(best, -1.0e5);
 }
 
 template <typename R>
@@ -190,9 +215,12 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
   DBuf<zd> G(nS), sig(nS), sig0(nS), sd(nS), chi(nC);
   DBuf<int> err(1);
   err.zero(s);
-  std::vector<DBuf<zd>> xout(A.m_diis), res(A.m_diis);  // DIIS history (unused for m_diis = 1)
-  if (A.m_diis > 1)
-    for (long i = 0; i < A.m_diis; ++i) { xout[i].alloc(nS); res[i].alloc(nS); }
+  DBuf<zd> xout, res;  // DIIS history (unused for m_diis = 1), entry i at i nS
+  std::vector<double> gram((size_t)(A.m_diis * A.m_diis), 0.0);  // Re <res_i, res_j>
+  if (A.m_diis > 1) {
+    xout.alloc((size_t)A.m_diis * nS);
+    res.alloc((size_t)A.m_diis * nS);
+  }
   std::unique_ptr<ConvEngine<R>> eng(new ConvEngine<R>(mesh, op));
   std::unique_ptr<ConvEngine<float>> e32;
   // mixed-precision state: chi0 and Sigma of the current iterate (chi_acc,
@@ -377,6 +405,7 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
 
   double stoner = 0.0;
   double t_chi = 0, t_vert = 0, t_sig = 0, t_mu = 0;
+  EventPair vert;
   int iters = 0;
   for (long it = 1; it <= A.scf_loop; ++it) {
     iters = (int)it;
@@ -407,7 +436,7 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
                           mu_ref, dJ.p, sawc_d.p, s);
       if (rebase) copy(chi_ref.p, chi_acc.p, nC, s);  // chi0 of the new reference, before the vertex overwrites it
     }
-    stoner = stoner_factor(chi_src, Nk, Nw, Nchi, S_d.p, s, 1e-9, A.soc ? -1.0 : 1.0);
+    stoner = stoner_factor(chi_src, Nk, Nw, Nchi, S_d.p, s, 1e-9, A.soc ? -1.0 : 1.0, err.p);
     t_chi += secs(t0);
     if (verbose) printf("SDW max eig(chi0 S) = %12.8f\n", stoner);
     const bool rescale = A.sw_rescale && stoner >= 1.0;
@@ -421,6 +450,7 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
       scale(Vout, nC, rescale_t / stoner, s);
     }
     t0 = clk::now();
+    GMOD_HIP(hipEventRecord(vert.a, s));
     // the FP32 vertex difference V - Vref comes out of the vertex kernel in
     // the increment iterations (unless chi0 was rescaled)
     const bool dv_fused = inc && !rescale;
@@ -437,11 +467,10 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
                          dv_fused ? Vref.p : nullptr, dv_fused ? e32->dv_buffer(nC) : nullptr, err.p, s,
                          !dv_fused || rebase || verbose);
     }
-    check_err(err, s, A.soc ? "get_V_soc_flex" : "get_vsigma_flex_nosoc");
-    t_vert += secs(t0);
+    GMOD_HIP(hipEventRecord(vert.b, s));
+    if (verbose) check_err(err, s, A.soc ? "get_V_soc_flex" : "get_vsigma_flex_nosoc");
     if (verbose)
       printf("Re V_sigma: max:%12.4E min:%12.4E\n", max_real(Vout, nC, s), min_real(Vout, nC, s));
-    t0 = clk::now();
     if (!inc) {
       if (A.soc) eng->sigma(sig.p, chi.p, soc_stat.data(), T, s, true);
       else eng->sigma(mixed ? sig_acc.p : sig.p, chi.p, A.Smat, A.Cmat, T, s, !mixed);
@@ -465,34 +494,38 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
         take_reference(chi_ref.p, Vout);
         ++n_rebase;
       } else {
-        dist_ref = max_rel_err(sig_ref.p, sig_acc.p, nS, 1.0e-10, s, nullptr);
+        dist_ref = max_rel_err(sig_ref.p, sig_acc.p, nS, 1.0e-10, s);
       }
       ++n_inc;
     }
     if (A.sub_sigma > 0) subtract_static(sig.p, Nk, (int)Nw, No, (int)A.sub_sigma, s);
-    // ---- compare_sigma
+    // ---- compare_sigma (the vertex's error flag is read with the measure)
+    int herr = 0;
     if (m == 1) {
       // one history entry: the DIIS system [[r.r + 1e-12, 1], [1, 0]] c =
       // [0, 1] gives c0 = 1 exactly (either pivot order divides a number by
       // itself or by 1), so the extrapolated Sigma is Sigma itself and the
       // step is the linear mixing; the same values without the history
       // copy, the residual, its norm and the scaling
-      esterr = max_rel_err(sig0.p, sig.p, nS, 1.0e-10, s, nullptr);
+      esterr = max_rel_err(sig0.p, sig.p, nS, 1.0e-10, s, err.p, &herr);
       lincomb(sig.p, sig.p, A.pp, sig0.p, 1.0 - A.pp, nS, s);
     } else {
       i_hist = i_hist % m + 1;
       n_hist = std::min(n_hist + 1, m);
-      copy(xout[i_hist - 1].p, sig.p, nS, s);
-      lincomb(res[i_hist - 1].p, sig.p, 1.0, sig0.p, -1.0, nS, s);
+      const int cur = i_hist - 1;
+      copy(xout.p + cur * nS, sig.p, nS, s);
+      lincomb(res.p + cur * nS, sig.p, 1.0, sig0.p, -1.0, nS, s);
       const int n = n_hist;
       std::vector<int> idx(n);
       for (int ih = 1; ih <= n; ++ih) idx[ih - 1] = ((i_hist - n + ih - 1) % m + m) % m;
+      // the new residual's row of the Gram matrix (n entries 0 .. n-1 are in
+      // use); the others stand from the iterations before
+      std::vector<zd> row(n);
+      dots(row.data(), res.p + cur * nS, res.p, (long)nS, n, nullptr, (long)nS, 1, s);
+      for (int i = 0; i < n; ++i) gram[cur + m * i] = gram[i + m * cur] = row[i].re;
       std::vector<double> B((n + 1) * (n + 1), 0.0), c(n + 1, 0.0);
       for (int a = 0; a < n; ++a) {
-        for (int b = a; b < n; ++b) {
-          double v = dot_w(res[idx[a]].p, res[idx[b]].p, nullptr, (long)nS, 1, s).re;
-          B[a + (n + 1) * b] = B[b + (n + 1) * a] = v;
-        }
+        for (int b = 0; b < n; ++b) B[a + (n + 1) * b] = gram[idx[a] + m * idx[b]];
         B[a + (n + 1) * n] = B[n + (n + 1) * a] = 1.0;
       }
       for (int a = 0; a < n; ++a) B[a + (n + 1) * a] += 1.0e-12;
@@ -502,14 +535,15 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
         std::fill(c.begin(), c.end(), 0.0);
         c[n - 1] = 1.0;
       }
-      copy(sd.p, xout[idx[0]].p, nS, s);
-      scale(sd.p, nS, c[0], s);
-      for (int a = 1; a < n; ++a) axpy(sd.p, xout[idx[a]].p, zd(c[a], 0), nS, s);
-      esterr = max_rel_err(sig0.p, sd.p, nS, 1.0e-10, s, nullptr);
+      combine(sd.p, xout.p, (long)nS, idx, std::vector<double>(c.begin(), c.begin() + n), nS, s);
+      esterr = max_rel_err(sig0.p, sd.p, nS, 1.0e-10, s, err.p, &herr);
       if (n >= 2) copy(sig.p, sd.p, nS, s);
       else lincomb(sig.p, sd.p, A.pp, sig0.p, 1.0 - A.pp, nS, s);
     }
-    t_sig += secs(t0);
+    raise_err(herr, A.soc ? "get_V_soc_flex" : "get_vsigma_flex_nosoc");
+    const double dt_vert = vert.seconds();
+    t_vert += dt_vert;
+    t_sig += secs(t0) - dt_vert;
     if (verbose) printf("esterr=%9.2E\n", esterr);
     if (esterr < A.eps) break;
     t0 = clk::now();
@@ -518,7 +552,7 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
       ProfScope ps(PROF_DYSON, (double)nS * 2 * sizeof(zd), s);
       dyson(G.p, sig.p, ham_d.p, mu, T, Nk, (int)Nw, No, err.p, s);
     }
-    check_err(err, s, "getinv");
+    if (verbose) check_err(err, s, "getinv");  // else read with the next Stoner factor
     copy(sig0.p, sig.p, nS, s);
     t_mu += secs(t0);
   }
@@ -614,9 +648,10 @@ struct EliashIn {
 // the pass-1 Ritz vector, and takes its largest Ritz value.  apply(w, v):
 // w = A v; norm, inner: the gap's norm and inner product; init(v): the unit
 // initial gap.  D receives the unit eigenvector; returns lambda.
+// The inner product is 2 sum kw conj(u) v over (Nk, n / Nk) (kw null: weights 1).
 template <class Apply, class Norm, class Inner, class Init>
 static double arnoldi_two_pass(int md, size_t n, zd* D, Apply apply, Norm norm, Inner inner, Init init,
-                               hipStream_t s, int verbose) {
+                               const double* kw, long Nk, hipStream_t s, int verbose) {
   std::vector<DBuf<zd>> V(md);
   for (auto& v : V) v.alloc(n);
   DBuf<zd> d1(n), nd(n);
@@ -625,22 +660,19 @@ static double arnoldi_two_pass(int md, size_t n, zd* D, Apply apply, Norm norm, 
     m_act = md;
     for (int j = 0; j < md; ++j) {
       apply(nd.p, V[j].p);
+      std::vector<const zd*> vs;
       if (defl) {
         axpy(nd.p, V[j].p, zd(shift, 0), n, s);
-        zd h = inner(d1.p, nd.p);
-        axpy(nd.p, d1.p, zd(0, 0) - h, n, s);
+        vs.push_back(d1.p);
       }
-      for (int ii = 0; ii <= j; ++ii) {
-        zd h = inner(V[ii].p, nd.p);
-        Hm[ii + (md + 1) * j] = h;
-        axpy(nd.p, V[ii].p, zd(0, 0) - h, n, s);
-      }
-      double beta = norm(nd.p);
+      for (int ii = 0; ii <= j; ++ii) vs.push_back(V[ii].p);
+      std::vector<zd> h(vs.size());
+      const double beta = gram_schmidt(nd.p, vs, h.data(), 2.0, kw, Nk, (long)n / Nk, s);
+      for (int ii = 0; ii <= j; ++ii) Hm[ii + (md + 1) * j] = h[ii + (defl ? 1 : 0)];
       Hm[j + 1 + (md + 1) * j] = zd(beta, 0);
       if (beta < 1.0e-14) { m_act = j + 1; break; }
       if (j < md - 1) {
-        copy(V[j + 1].p, nd.p, n, s);
-        scale(V[j + 1].p, n, 1.0 / beta, s);
+        scale_copy(V[j + 1].p, nd.p, 1.0 / beta, n, s);
       }
     }
   };
@@ -732,7 +764,7 @@ static double eliash_driver(const EliashIn& A, zd* delta_out) {
   double lam_out = 0.0;
   if (A.arnoldi_m > 0) {
     auto init = [&](zd* v) { initial_delta(v, A.init_delta, A.uni, mesh, No, A.gap_sym, s); };
-    lam_out = arnoldi_two_pass((int)A.arnoldi_m, nS, D.p, apply, norm, inner, init, s, verbose);
+    lam_out = arnoldi_two_pass((int)A.arnoldi_m, nS, D.p, apply, norm, inner, init, mesh.kw.p, Nk, s, verbose);
   } else {
     // power method with shift + deflation (feliash.f90:67-140)
     double lam1 = 0.0, lam_phys = 0.0, lam_rq = 0.0, inorm = 1.0;
@@ -752,15 +784,15 @@ static double eliash_driver(const EliashIn& A, zd* delta_out) {
           double proj = inner(d1.p, nd.p).re;
           axpy(nd.p, d1.p, zd(-proj, 0), nS, s);
         }
-        double nrm = norm(nd.p);
+        double pd[3];
+        power_dots(pd, nd.p, D.p, mesh.kw.p, Nk, rest, s);
+        const double nn = 2.0 * pd[0], xr = 2.0 * pd[1], dd = 2.0 * pd[2];
+        const double nrm = std::sqrt(nn);
         if (nrm <= 0.0) throw Error("Error: norm <= 0 in iter_loop");
         inorm = 1.0 / nrm;
-        lam_rq = inner(D.p, nd.p).re;
+        lam_rq = xr;
         lam_phys = lam_rq + lam1;
         // vec_err = sqrt(2 min(|nd/|nd| - D|^2, |nd/|nd| + D|^2))
-        double nn = 2.0 * dot_w(nd.p, nd.p, mesh.kw.p, Nk, rest, s).re;
-        double dd = 2.0 * dot_w(D.p, D.p, mesh.kw.p, Nk, rest, s).re;
-        double xr = 2.0 * dot_w(nd.p, D.p, mesh.kw.p, Nk, rest, s).re;
         double tpos = 0.5 * (nn * inorm * inorm + dd - 2.0 * inorm * xr);
         double tneg = 0.5 * (nn * inorm * inorm + dd + 2.0 * inorm * xr);
         double verr = std::sqrt(2.0 * std::max(0.0, std::min(tpos, tneg)));
@@ -768,8 +800,7 @@ static double eliash_driver(const EliashIn& A, zd* delta_out) {
         if (lam_phys < 0.0 && verr < A.eps) break;
         if (verr < A.eps && std::fabs(lam_phys - lam_prev) < A.eps * (std::fabs(lam_phys) + 1.0e-10)) break;
         lam_prev = lam_phys;
-        copy(D.p, nd.p, nS, s);
-        scale(D.p, nS, inorm, s);
+        scale_copy(D.p, nd.p, inorm, nS, s);
       }
       if (i_eig == 1) {
         if (lam_phys > 0.0) { lam_out = lam_phys; break; }
@@ -858,7 +889,7 @@ static double eliash_soc_driver(const EliashSocIn& A, zd* delta_out) {
   };
   double lam = 0.0;
   if (A.arnoldi_m > 0) {
-    lam = arnoldi_two_pass((int)A.arnoldi_m, nF, D.p, apply, norm, inner, init, s, verbose);
+    lam = arnoldi_two_pass((int)A.arnoldi_m, nF, D.p, apply, norm, inner, init, nullptr, NW, s, verbose);
   } else {
     // shifted power method (feliashwithsoc.f90:59-110): newdelta = A delta +
     // norm2 delta, norm2 = 0 for the first eigenvalue, then the norm of the
@@ -870,12 +901,14 @@ static double eliash_soc_driver(const EliashSocIn& A, zd* delta_out) {
       for (long it = 1; it <= A.itemax; ++it) {
         apply(nd.p, D.p);
         if (norm2 != 0.0) axpy(nd.p, D.p, zd(norm2, 0), nF, s);
-        nrm = norm(nd.p);
+        double pd[3];
+        power_dots(pd, nd.p, D.p, nullptr, NW, rest, s);
+        const double nn = pd[0], xr = pd[1], dd = pd[2];
+        nrm = std::sqrt(2.0 * nn);
         if (nrm <= 0.0) throw Error("lin_eliash_soc: norm <= 0 in iter_loop");
         const double inorm = 1.0 / nrm;
-        lam_rq = inner(D.p, nd.p).re;
+        lam_rq = 2.0 * xr;
         // vec_err = sqrt(2 min(sum|nd/|nd| - D|^2, sum|nd/|nd| + D|^2))
-        const double nn = dot(nd.p, nd.p).re, dd = dot(D.p, D.p).re, xr = dot(nd.p, D.p).re;
         const double tpos = nn * inorm * inorm + dd - 2.0 * inorm * xr;
         const double tneg = nn * inorm * inorm + dd + 2.0 * inorm * xr;
         const double verr = std::sqrt(2.0 * std::max(0.0, std::min(tpos, tneg)));
@@ -886,8 +919,7 @@ static double eliash_soc_driver(const EliashSocIn& A, zd* delta_out) {
           if (verr < A.eps * 1.0e-2) ++count;
           if (count > 30) break;
         }
-        copy(D.p, nd.p, nF, s);
-        scale(D.p, nF, inorm, s);
+        scale_copy(D.p, nd.p, inorm, nF, s);
       }
       lam = lam_rq - norm2;
       if (verbose) printf("eliash=%16.8E\n", lam);

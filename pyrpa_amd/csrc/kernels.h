@@ -682,13 +682,31 @@ void diff_to_f32(cpx<float>* dst, const zd* a, const zd* b, long n, hipStream_t 
 template <typename R>
 void add_inplace(cpx<R>* y, const cpx<R>* x, long n, hipStream_t s);  // y += x
 
-// ---- deterministic reductions (two-stage, fixed order)
+// y = x f;  y = sum_i c_i (x + idx_i stride)
+void scale_copy(zd* y, const zd* x, double f, long n, hipStream_t s);
+void combine(zd* y, const zd* x, long stride, const std::vector<int>& idx, const std::vector<double>& c, long n,
+             hipStream_t s);
+// a, b <- a + b, a - b
+void sum_diff(zd* a, zd* b, long n, hipStream_t s);
+
+// ---- deterministic reductions (fixed order), each waiting for its result
 // sum over k-space arrays laid out (Nk, rest): weights kw[k] (or 1)
 zd dot_w(const zd* u, const zd* v, const double* kw, long Nk, long rest, hipStream_t s);  // sum kw conj(u) v
-double max_rel_err(const zd* s0, const zd* sd, long n, double floor, hipStream_t s, long* where);
+// the same with nv vectors v + i stride
+void dots(zd* out, const zd* u, const zd* v, long stride, int nv, const double* kw, long Nk, long rest,
+          hipStream_t s);
+// sum kw |nd|^2, Re sum kw conj(D) nd, sum kw |D|^2
+void power_dots(double out[3], const zd* nd, const zd* D, const double* kw, long Nk, long rest, hipStream_t s);
+// modified Gram-Schmidt: for each v in turn h_i = f sum kw conj(v) x, x -= h_i v;
+// returns the norm sqrt(f sum kw |x|^2) of what is left
+double gram_schmidt(zd* x, const std::vector<const zd*>& vs, zd* h, double f, const double* kw, long Nk, long rest,
+                    hipStream_t s);
+// max |s0 - sd| / |sd| over |sd| > floor; err (device): an error flag read along
+double max_rel_err(const zd* s0, const zd* sd, long n, double floor, hipStream_t s, const int* err = nullptr,
+                   int* err_out = nullptr);
+double max_value(const double* a, long n, hipStream_t s, const int* err = nullptr, int* err_out = nullptr);
 double max_real(const zd* a, long n, hipStream_t s);
 double max_abs_diff(const zd* a, const zd* b, long n, hipStream_t s);                      // max |a - b| (b null: max |a|)
-void sum_diff(zd* a, zd* b, long n, hipStream_t s);                                        // a, b <- a + b, a - b
 double min_real(const zd* a, long n, hipStream_t s);
 
 }  // namespace gmod

@@ -3,6 +3,7 @@
 #include <cmath>
 
 #include "kernels.h"
+#include "reduce.h"
 
 namespace gmod {
 
@@ -424,147 +425,339 @@ void sum_diff(zd* a, zd* b, long n, hipStream_t s) {
 }
 
 // ------------------------------------------------------------------ reductions
-constexpr int RED_BLOCKS = 1024;
+// Latency-bound (a few MB at most): one launch and one wait per result.  The
+// earlier form summed the 1024 partial results of a dot product in one thread
+// of a second launch (90 us, a dependent load per term) and copied the sum
+// back: 110 us on the device, now 15 with the wait.
+static void wait(hipStream_t s) { GMOD_HIP(hipStreamSynchronize(s)); }
 
-__device__ inline double block_sum(double v, double* sh) {
-  sh[threadIdx.x] = v;
+// The gap equation's norms and inner products are summed in one fixed order
+// whatever the launch: element e belongs to work-group (e / 256) mod 1024, a
+// work-group sums its threads by halves, the 1024 partial results are added in
+// turn.  (A few Krylov steps or a slowly converging power iteration amplify a
+// different rounding of these sums to the fourth digit of the gap.)
+constexpr int ORD_BLOCKS = 1024;
+static_assert(ORD_BLOCKS * 4 <= PIN_DOUBLES, "partial results of power_dots");
+static int ord_blocks(long n) { return (int)std::max<long>(1, std::min<long>(ORD_BLOCKS, (n + RED_TPB - 1) / RED_TPB)); }
+
+// sum over the work-group's 256 threads by halves, on thread 0
+template <int W>
+__device__ __forceinline__ void halves_sum(double (&v)[W], double* sh) {
+#pragma unroll
+  for (int c = 0; c < W; ++c) sh[c * RED_TPB + threadIdx.x] = v[c];
   __syncthreads();
-  for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
-    __syncthreads();
+  if (threadIdx.x < 128) {
+#pragma unroll
+    for (int c = 0; c < W; ++c) sh[c * RED_TPB + threadIdx.x] += sh[c * RED_TPB + threadIdx.x + 128];
   }
-  double r = sh[0];
   __syncthreads();
-  return r;
+  if (threadIdx.x < 64) {
+#pragma unroll
+    for (int c = 0; c < W; ++c) {
+      double x = sh[c * RED_TPB + threadIdx.x] + sh[c * RED_TPB + threadIdx.x + 64];
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) x += __shfl_down(x, o);
+      v[c] = x;
+    }
+  }
+  __syncthreads();
 }
 
-__global__ void k_dot_w(const zd* u, const zd* v, const double* kw, long Nk, long n, double* part) {
-  __shared__ double sh[TPB];
-  double re = 0, im = 0;
-  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x) {
-    zd p = conj(u[e]) * v[e];
-    double w = kw ? kw[e % Nk] : 1.0;
-    re += w * p.re;
-    im += w * p.im;
+__global__ void __launch_bounds__(RED_TPB)
+k_dot_w(const zd* __restrict__ u, const zd* __restrict__ v, const double* __restrict__ kw, long Nk, long n,
+        double* part) {
+  __shared__ double sh[2 * RED_TPB];
+  double r[2] = {0, 0};
+  for (long e = blockIdx.x * (long)RED_TPB + threadIdx.x; e < n; e += (long)ORD_BLOCKS * RED_TPB) {
+    const zd p = conj(u[e]) * v[e];
+    const double w = kw ? kw[e % Nk] : 1.0;
+    r[0] += w * p.re;
+    r[1] += w * p.im;
   }
-  re = block_sum(re, sh);
-  im = block_sum(im, sh);
-  if (threadIdx.x == 0) { part[2 * blockIdx.x] = re; part[2 * blockIdx.x + 1] = im; }
-}
-
-__global__ void k_finish_sum(const double* part, int nb, int width, double* out) {
-  // one thread per component, fixed order
-  int c = threadIdx.x;
-  if (c < width) {
-    double s = 0;
-    for (int b = 0; b < nb; ++b) s += part[width * b + c];
-    out[c] = s;
-  }
+  halves_sum<2>(r, sh);
+  if (threadIdx.x == 0) { part[2 * blockIdx.x] = r[0]; part[2 * blockIdx.x + 1] = r[1]; }
 }
 
 zd dot_w(const zd* u, const zd* v, const double* kw, long Nk, long rest, hipStream_t s) {
   const long n = Nk * rest;
-  DBuf<double> part(2 * RED_BLOCKS + 2);
-  hipLaunchKernelGGL(k_dot_w, dim3(RED_BLOCKS), dim3(TPB), 0, s, u, v, kw, Nk, n, part.p);
+  const int nb = ord_blocks(n);
+  const double* p = ctx().pin;
+  hipLaunchKernelGGL(k_dot_w, dim3(nb), dim3(RED_TPB), 0, s, u, v, kw, Nk, n, ctx().pin);
   GMOD_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_finish_sum, dim3(1), dim3(64), 0, s, part.p, RED_BLOCKS, 2, part.p + 2 * RED_BLOCKS);
-  GMOD_CHECK_LAUNCH();
-  double h[2];
-  GMOD_HIP(hipMemcpyAsync(h, part.p + 2 * RED_BLOCKS, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
-  GMOD_HIP(hipStreamSynchronize(s));
-  return zd(h[0], h[1]);
-}
-
-__global__ void k_max_rel(const zd* s0, const zd* sd, long n, double floor, double* part) {
-  __shared__ double sh[TPB];
-  double best = 0.0;
-  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x) {
-    zd d = sd[e];
-    double ad = hypot(d.re, d.im);
-    if (ad > floor) {
-      zd df = s0[e] - d;
-      double r = hypot(df.re, df.im) / ad;
-      if (r > best) best = r;
-    }
-  }
-  sh[threadIdx.x] = best;
-  __syncthreads();
-  for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + o]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
-}
-
-__global__ void k_minmax_re(const zd* a, long n, int want_max, double* part) {
-  __shared__ double sh[TPB];
-  double best = want_max ? -HUGE_VAL : HUGE_VAL;
-  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x)
-    best = want_max ? fmax(best, a[e].re) : fmin(best, a[e].re);
-  sh[threadIdx.x] = best;
-  __syncthreads();
-  for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o)
-      sh[threadIdx.x] = want_max ? fmax(sh[threadIdx.x], sh[threadIdx.x + o]) : fmin(sh[threadIdx.x], sh[threadIdx.x + o]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
-}
-
-static double host_reduce(const double* dpart, int nb, hipStream_t s, int mode) {
-  std::vector<double> h(nb);
-  GMOD_HIP(hipMemcpyAsync(h.data(), dpart, nb * sizeof(double), hipMemcpyDeviceToHost, s));
-  GMOD_HIP(hipStreamSynchronize(s));
-  double r = h[0];
-  for (int i = 1; i < nb; ++i) r = mode == 0 ? std::max(r, h[i]) : std::min(r, h[i]);
+  wait(s);
+  zd r(0, 0);
+  for (int b = 0; b < nb; ++b) r += zd(p[2 * b], p[2 * b + 1]);
   return r;
 }
 
-double max_rel_err(const zd* s0, const zd* sd, long n, double floor, hipStream_t s, long* where) {
-  DBuf<double> part(RED_BLOCKS);
-  hipLaunchKernelGGL(k_max_rel, dim3(RED_BLOCKS), dim3(TPB), 0, s, s0, sd, n, floor, part.p);
+// the sums of a power step: kw |nd|^2, Re kw conj(D) nd, kw |D|^2
+__global__ void __launch_bounds__(RED_TPB)
+k_power_dots(const zd* __restrict__ nd, const zd* __restrict__ D, const double* __restrict__ kw, long Nk, long n,
+             double* part) {
+  __shared__ double sh[3 * RED_TPB];
+  double r[3] = {0, 0, 0};
+  for (long e = blockIdx.x * (long)RED_TPB + threadIdx.x; e < n; e += (long)ORD_BLOCKS * RED_TPB) {
+    const zd a = nd[e], d = D[e];
+    const zd aa = conj(a) * a, da = conj(d) * a, dd = conj(d) * d;
+    const double w = kw ? kw[e % Nk] : 1.0;
+    r[0] += w * aa.re;
+    r[1] += w * da.re;
+    r[2] += w * dd.re;
+  }
+  halves_sum<3>(r, sh);
+  if (threadIdx.x == 0)
+    for (int c = 0; c < 3; ++c) part[3 * blockIdx.x + c] = r[c];
+}
+void power_dots(double out[3], const zd* nd, const zd* D, const double* kw, long Nk, long rest, hipStream_t s) {
+  const int nb = ord_blocks(Nk * rest);
+  const double* p = ctx().pin;
+  hipLaunchKernelGGL(k_power_dots, dim3(nb), dim3(RED_TPB), 0, s, nd, D, kw, Nk, Nk * rest, ctx().pin);
   GMOD_CHECK_LAUNCH();
-  if (where) *where = -1;
-  return host_reduce(part.p, RED_BLOCKS, s, 0);
+  wait(s);
+  for (int c = 0; c < 3; ++c) {
+    out[c] = 0.0;
+    for (int b = 0; b < nb; ++b) out[c] += p[3 * b + c];
+  }
+}
+
+// the nb partial results (re, im) added in turn, by threads 0 and 1 from LDS:
+// s[0], s[1] (1024 dependent additions, 4 us)
+__device__ __forceinline__ void turn_sum(double (&s)[2], const double* __restrict__ part, int nb, double* sh) {
+  for (int i = threadIdx.x; i < 2 * nb; i += RED_TPB) sh[i] = part[i];
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    double t = 0.0;
+    int b = 0;
+    for (; b + 8 <= nb; b += 8) {
+      double x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = sh[2 * (b + i) + threadIdx.x];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) t += x[i];
+    }
+    for (; b < nb; ++b) t += sh[2 * b + threadIdx.x];
+    s[0] = t;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) sh[threadIdx.x] = s[0];
+  __syncthreads();
+  s[0] = sh[0];
+  s[1] = sh[1];
+  __syncthreads();
+}
+
+// One step of a modified Gram-Schmidt chain without a host wait: h = f times
+// the sum of the previous launch's nb partial results (every work-group forms
+// it), x -= h v, and the partial results of the next inner product,
+// conj(vn) x (vn null: |x|^2), in pout.  v null: no update (the chain's
+// start).  h goes to hout.
+__global__ void __launch_bounds__(RED_TPB)
+k_mgs(zd* __restrict__ x, const zd* __restrict__ v, const zd* __restrict__ vn, const double* __restrict__ kw, long Nk,
+      long n, double f, const double* __restrict__ pin_, double* __restrict__ pout, double* hout) {
+  __shared__ double sh[2 * ORD_BLOCKS];
+  const int nb = gridDim.x;
+  zd h(0, 0);
+  if (v) {
+    double t[2];
+    turn_sum(t, pin_, nb, sh);
+    h = zd(t[0] * f, t[1] * f);
+    if (hout && blockIdx.x == 0 && threadIdx.x == 0) {
+      hout[0] = h.re;
+      hout[1] = h.im;
+    }
+    h = zd(0, 0) - h;
+  }
+  double r[2] = {0, 0};
+  for (long e = blockIdx.x * (long)RED_TPB + threadIdx.x; e < n; e += (long)ORD_BLOCKS * RED_TPB) {
+    zd a = x[e];
+    if (v) {
+      a = a + h * v[e];
+      x[e] = a;
+    }
+    const zd p = conj(vn ? vn[e] : a) * a;
+    const double w = kw ? kw[e % Nk] : 1.0;
+    r[0] += w * p.re;
+    r[1] += w * p.im;
+  }
+  halves_sum<2>(r, sh);
+  if (threadIdx.x == 0) {
+    pout[2 * blockIdx.x] = r[0];
+    pout[2 * blockIdx.x + 1] = r[1];
+  }
+}
+
+double gram_schmidt(zd* x, const std::vector<const zd*>& vs, zd* h, double f, const double* kw, long Nk, long rest,
+                    hipStream_t s) {
+  const long n = Nk * rest;
+  Context& c = ctx();
+  const int nb = ord_blocks(n), m = (int)vs.size();
+  double* pnorm = c.pin;  // the last step's partial results go to the host, behind them the h
+  double* hp = c.pin + 2 * ORD_BLOCKS;
+  constexpr int ROOM = (PIN_DOUBLES - 2 * ORD_BLOCKS) / 2;
+  double* part[2] = {c.red, c.red + 2 * ORD_BLOCKS};
+  for (int i = -1; i < m; ++i) {
+    const zd* vn = i + 1 < m ? vs[i + 1] : nullptr;
+    hipLaunchKernelGGL(k_mgs, dim3(nb), dim3(RED_TPB), 0, s, x, i < 0 ? (const zd*)nullptr : vs[i], vn, kw, Nk, n, f,
+                       (const double*)part[(i + 1) & 1], i + 1 < m ? part[i & 1] : pnorm,
+                       i < 0 ? (double*)nullptr : hp + 2 * (i % ROOM));
+    GMOD_CHECK_LAUNCH();
+    if (i + 1 == m || i % ROOM == ROOM - 1) {
+      wait(s);
+      for (int j = i < 0 ? 0 : i - i % ROOM; j <= i; ++j) h[j] = zd(hp[2 * (j % ROOM)], hp[2 * (j % ROOM) + 1]);
+    }
+  }
+  double t = 0.0;
+  for (int b = 0; b < nb; ++b) t += pnorm[2 * b];
+  return std::sqrt(f * t);
+}
+
+// sum kw conj(u) v_y of the nv vectors v + y stride (blockIdx.y = y)
+__global__ void __launch_bounds__(RED_TPB)
+k_dots(const zd* __restrict__ u, const zd* __restrict__ v, long stride, const double* __restrict__ kw, long Nk,
+       long n, double* part, unsigned* ticket, double* out) {
+  const zd* __restrict__ vy = v + (long)blockIdx.y * stride;
+  double r[2] = {0, 0};
+  for (long e = blockIdx.x * (long)RED_TPB + threadIdx.x; e < n; e += (long)gridDim.x * RED_TPB) {
+    const zd p = conj(u[e]) * vy[e];
+    const double w = kw ? kw[e % Nk] : 1.0;
+    r[0] += w * p.re;
+    r[1] += w * p.im;
+  }
+  finish_reduce<RedSum, 2>(r, blockIdx.x, gridDim.x, part + (long)blockIdx.y * 2 * RED_MAX_BLOCKS,
+                           ticket + blockIdx.y, out + 2 * blockIdx.y);
+}
+
+void dots(zd* out, const zd* u, const zd* v, long stride, int nv, const double* kw, long Nk, long rest,
+          hipStream_t s) {
+  const long n = Nk * rest;
+  Context& c = ctx();
+  for (int v0 = 0; v0 < nv; v0 += 64) {  // as many as there are ticket counters
+    const int m = std::min(64, nv - v0);
+    hipLaunchKernelGGL(k_dots, dim3(red_blocks(n), m), dim3(RED_TPB), 0, s, u, v + v0 * stride, stride, kw, Nk, n,
+                       c.red, c.ticket, c.pin);
+    GMOD_CHECK_LAUNCH();
+    wait(s);
+    for (int i = 0; i < m; ++i) out[v0 + i] = zd(c.pin[2 * i], c.pin[2 * i + 1]);
+  }
+}
+
+__global__ void __launch_bounds__(RED_TPB)
+k_max_rel(const zd* __restrict__ s0, const zd* __restrict__ sd, long n, double floor, double* part, unsigned* ticket,
+          double* out, const int* err) {
+  double best[1] = {0.0};
+  for (long e = blockIdx.x * (long)RED_TPB + threadIdx.x; e < n; e += (long)gridDim.x * RED_TPB) {
+    const zd d = sd[e];
+    const double ad = hypot(d.re, d.im);
+    if (ad > floor) {
+      const zd df = s0[e] - d;
+      const double r = hypot(df.re, df.im) / ad;
+      if (r > best[0]) best[0] = r;
+    }
+  }
+  finish_reduce<RedMax, 1>(best, blockIdx.x, gridDim.x, part, ticket, out, err);
+}
+double max_rel_err(const zd* s0, const zd* sd, long n, double floor, hipStream_t s, const int* err, int* err_out) {
+  Context& c = ctx();
+  hipLaunchKernelGGL(k_max_rel, dim3(red_blocks(n)), dim3(RED_TPB), 0, s, s0, sd, n, floor, c.red, c.ticket, c.pin,
+                     err);
+  GMOD_CHECK_LAUNCH();
+  wait(s);
+  if (err) *err_out = (int)c.pin[1];
+  return c.pin[0];
+}
+
+template <class Op>
+__global__ void __launch_bounds__(RED_TPB)
+k_extreme(const double* __restrict__ a, long stride, long n, double* part, unsigned* ticket, double* out,
+          const int* err) {
+  double best[1] = {Op::id()};
+  for (long e = blockIdx.x * (long)RED_TPB + threadIdx.x; e < n; e += (long)gridDim.x * RED_TPB)
+    best[0] = Op::op(best[0], a[e * stride]);
+  finish_reduce<Op, 1>(best, blockIdx.x, gridDim.x, part, ticket, out, err);
+}
+double max_value(const double* a, long n, hipStream_t s, const int* err, int* err_out) {
+  Context& c = ctx();
+  hipLaunchKernelGGL(k_extreme<RedMax>, dim3(red_blocks(n)), dim3(RED_TPB), 0, s, a, 1L, n, c.red, c.ticket, c.pin,
+                     err);
+  GMOD_CHECK_LAUNCH();
+  wait(s);
+  if (err) *err_out = (int)c.pin[1];
+  return c.pin[0];
+}
+double max_real(const zd* a, long n, hipStream_t s) {
+  Context& c = ctx();
+  hipLaunchKernelGGL(k_extreme<RedMax>, dim3(red_blocks(n)), dim3(RED_TPB), 0, s, (const double*)a, 2L, n, c.red,
+                     c.ticket, c.pin, (const int*)nullptr);
+  GMOD_CHECK_LAUNCH();
+  wait(s);
+  return c.pin[0];
+}
+double min_real(const zd* a, long n, hipStream_t s) {
+  Context& c = ctx();
+  hipLaunchKernelGGL(k_extreme<RedMin>, dim3(red_blocks(n)), dim3(RED_TPB), 0, s, (const double*)a, 2L, n, c.red,
+                     c.ticket, c.pin, (const int*)nullptr);
+  GMOD_CHECK_LAUNCH();
+  wait(s);
+  return c.pin[0];
 }
 
 // max |a - b| (b null: max |a|)
-__global__ void k_max_absdiff(const zd* a, const zd* b, long n, double* part) {
-  __shared__ double sh[TPB];
-  double best = 0.0;
-  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x) {
+__global__ void __launch_bounds__(RED_TPB)
+k_max_absdiff(const zd* __restrict__ a, const zd* __restrict__ b, long n, double* part, unsigned* ticket,
+              double* out) {
+  double best[1] = {0.0};
+  for (long e = blockIdx.x * (long)RED_TPB + threadIdx.x; e < n; e += (long)gridDim.x * RED_TPB) {
     const zd d = b ? a[e] - b[e] : a[e];
     const double r = hypot(d.re, d.im);
-    if (r > best) best = r;
+    if (r > best[0]) best[0] = r;
   }
-  sh[threadIdx.x] = best;
-  __syncthreads();
-  for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + o]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
+  finish_reduce<RedMax, 1>(best, blockIdx.x, gridDim.x, part, ticket, out);
 }
-
 double max_abs_diff(const zd* a, const zd* b, long n, hipStream_t s) {
-  DBuf<double> part(RED_BLOCKS);
-  hipLaunchKernelGGL(k_max_absdiff, dim3(RED_BLOCKS), dim3(TPB), 0, s, a, b, n, part.p);
+  Context& c = ctx();
+  hipLaunchKernelGGL(k_max_absdiff, dim3(red_blocks(n)), dim3(RED_TPB), 0, s, a, b, n, c.red, c.ticket, c.pin);
   GMOD_CHECK_LAUNCH();
-  return host_reduce(part.p, RED_BLOCKS, s, 0);
+  wait(s);
+  return c.pin[0];
 }
 
-double max_real(const zd* a, long n, hipStream_t s) {
-  DBuf<double> part(RED_BLOCKS);
-  hipLaunchKernelGGL(k_minmax_re, dim3(RED_BLOCKS), dim3(TPB), 0, s, a, n, 1, part.p);
-  GMOD_CHECK_LAUNCH();
-  return host_reduce(part.p, RED_BLOCKS, s, 0);
+// y = sum_i c_i x_i over up to COMBINE vectors x + idx_i stride (add: onto y)
+constexpr int COMBINE = 8;
+struct CombineArgs {
+  double c[COMBINE];
+  long off[COMBINE];
+  int n;
+};
+__global__ void k_combine(zd* __restrict__ y, const zd* __restrict__ x, CombineArgs a, int add, long n) {
+  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x) {
+    zd r = add ? y[e] : zd(0, 0);
+#pragma unroll
+    for (int i = 0; i < COMBINE; ++i)
+      if (i < a.n) r += x[a.off[i] + e] * a.c[i];
+    y[e] = r;
+  }
+}
+void combine(zd* y, const zd* x, long stride, const std::vector<int>& idx, const std::vector<double>& c, long n,
+             hipStream_t s) {
+  for (size_t i0 = 0; i0 < idx.size(); i0 += COMBINE) {
+    CombineArgs a{};
+    a.n = (int)std::min<size_t>(COMBINE, idx.size() - i0);
+    for (int i = 0; i < a.n; ++i) {
+      a.c[i] = c[i0 + i];
+      a.off[i] = idx[i0 + i] * stride;
+    }
+    hipLaunchKernelGGL(k_combine, dim3(nblocks(n)), dim3(TPB), 0, s, y, x, a, i0 > 0 ? 1 : 0, n);
+    GMOD_CHECK_LAUNCH();
+  }
 }
 
-double min_real(const zd* a, long n, hipStream_t s) {
-  DBuf<double> part(RED_BLOCKS);
-  hipLaunchKernelGGL(k_minmax_re, dim3(RED_BLOCKS), dim3(TPB), 0, s, a, n, 0, part.p);
+__global__ void k_scale_copy(zd* y, const zd* x, double f, long n) {
+  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x)
+    y[e] = x[e] * f;
+}
+void scale_copy(zd* y, const zd* x, double f, long n, hipStream_t s) {
+  hipLaunchKernelGGL(k_scale_copy, dim3(nblocks(n)), dim3(TPB), 0, s, y, x, f, n);
   GMOD_CHECK_LAUNCH();
-  return host_reduce(part.p, RED_BLOCKS, s, 1);
 }
 
 // ------------------------------------------------------------------ Sigma reference-vertex term

@@ -45,10 +45,8 @@ void max_re_eig_ws(double* out, const zd* A, BatchLayout La, long batch, int n, 
 // Dyson: G = [(i w_j + mu) I - H(k) - Sigma(k, i w_j)]^-1   (fself.f90:43-83, 131-157)
 void dyson(zd* G, const zd* sigma, const zd* hamk, double mu, double temp, long Nk, int Nw, int No, int* err,
            hipStream_t s);
-// n(mu) pieces (fself.f90:687-714): returns {sum_k,n f(e), sum_{k,j} Re[Tr(z-H-Sigma)^-1 - sum_n 1/(z-e_n)]}
-void filling_parts(double out[2], const zd* sigma, const zd* hamk, const double* eig, double rmu, double temp,
-                   long Nk, int Nw, int No, int* err, hipStream_t s);
-// The same n(mu) pieces through the characteristic polynomials of H + Sigma:
+// n(mu) pieces (fself.f90:687-714): {sum_k,n f(e), sum_{k,j} Re[Tr(z-H-Sigma)^-1
+// - sum_n 1/(z-e_n)]} through the characteristic polynomials of H + Sigma:
 // filling_charpoly writes coef(NkNw, No) once per Sigma, filling_parts_cp
 // evaluates Tr (z - H - Sigma)^-1 = p'(z)/p(z) at any mu
 void filling_charpoly(zd* coef, const zd* sigma, const zd* hamk, long Nk, int Nw, int No, hipStream_t s);

@@ -4,13 +4,14 @@
 //   matrix and both right-hand sides live in LDS; the LU with partial pivoting
 //   (pivot = max |Re|+|Im|, as LAPACK's izamax) updates the trailing block with
 //   one lane per element.
-// * dyson / filling_parts / green0 / anomalous_f: one lane per (k, i w) with
+// * dyson / filling_charpoly / green0 / anomalous_f: one lane per (k, i w) with
 //   the No x No matrix held in registers (No <= 8).
 // * max_re_eig: one lane per matrix; Hessenberg reduction + shifted complex QR.
 #include <cfloat>
 #include <cmath>
 
 #include "linalg.h"
+#include "reduce.h"
 #include "kernels.h"
 
 namespace gmod {
@@ -1312,7 +1313,7 @@ __device__ inline bool gj_inverse(zd (&a)[NO][NO]) {
 }
 
 // The per-(k, w) register kernels below declare the block size they are
-// launched with (128 threads; 256 for the filling reductions): the bound
+// launched with (128 threads; 256 for the filling reduction): the bound
 // lets the compiler keep their No x No complex matrices in registers
 // (without it, it plans for 1024-thread blocks, caps a thread at 128
 // registers and spills the matrices to scratch memory).
@@ -1338,51 +1339,6 @@ __global__ void __launch_bounds__(128) k_dyson(zd* G, const zd* sig, const zd* H
 #pragma unroll
       for (int q = 0; q < NO; ++q) G[e + tot * (p + NO * q)] = a[p][q];
   }
-}
-
-template <int NO>
-__global__ void __launch_bounds__(256) k_filling(const zd* sig, const zd* H, const double* eig, double rmu, double temp, long Nk, int Nw,
-                          double* part, int* err) {
-  __shared__ double sh[2][256];
-  const long tot = Nk * (long)Nw;
-  double fsum = 0.0, dsum = 0.0;
-  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < tot; e += (long)gridDim.x * blockDim.x) {
-    long k = e % Nk;
-    long j = e / Nk;
-    zd z(rmu, (double)(2 * j + 1) * PI_D * temp);
-    zd a[NO][NO];
-#pragma unroll
-    for (int p = 0; p < NO; ++p)
-#pragma unroll
-      for (int q = 0; q < NO; ++q) {
-        zd v = zd(0, 0) - (H[p + NO * (q + NO * k)] + sig[e + tot * (p + NO * q)]);
-        if (p == q) v += z;
-        a[p][q] = v;
-      }
-    if (!gj_inverse<NO>(a)) atomicOr(err, 8);
-    double d = 0.0;
-#pragma unroll
-    for (int n = 0; n < NO; ++n) {
-      d += a[n][n].re;
-      d -= (zd(1.0, 0) / (z - zd(eig[n + NO * k], 0))).re;
-    }
-    dsum += d;
-    if (j == 0) {
-#pragma unroll
-      for (int n = 0; n < NO; ++n) fsum += 0.5 * (1.0 - tanh(0.5 * (eig[n + NO * k] - rmu) / temp));
-    }
-  }
-  sh[0][threadIdx.x] = fsum;
-  sh[1][threadIdx.x] = dsum;
-  __syncthreads();
-  for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) {
-      sh[0][threadIdx.x] += sh[0][threadIdx.x + o];
-      sh[1][threadIdx.x] += sh[1][threadIdx.x + o];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) { part[2 * blockIdx.x] = sh[0][0]; part[2 * blockIdx.x + 1] = sh[1][0]; }
 }
 
 // Characteristic polynomial of M = H(k) + Sigma(k, i w_j) per (k, j):
@@ -1432,14 +1388,15 @@ __global__ void __launch_bounds__(128) k_charpoly(zd* coef, const zd* sig, const
   }
 }
 
-// n(mu) pieces from the characteristic polynomials (see k_charpoly)
+// n(mu) pieces from the characteristic polynomials (see k_charpoly), summed
+// in the same launch (latency-bound: with a copy of the partial sums to the
+// host a trial mu took 24 us at 1 orbital, 32x32 x 256)
 template <int NO>
-__global__ void __launch_bounds__(256) k_filling_cp(const zd* coef, const double* eig, double rmu, double temp, long Nk, int Nw,
-                             double* part) {
-  __shared__ double sh[2][256];
+__global__ void __launch_bounds__(RED_TPB) k_filling_cp(const zd* coef, const double* eig, double rmu, double temp,
+                                                        long Nk, int Nw, double* part, unsigned* ticket, double* out) {
   const long tot = Nk * (long)Nw;
-  double fsum = 0.0, dsum = 0.0;
-  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < tot; e += (long)gridDim.x * blockDim.x) {
+  double r[2] = {0.0, 0.0};
+  for (long e = blockIdx.x * (long)RED_TPB + threadIdx.x; e < tot; e += (long)gridDim.x * RED_TPB) {
     const long k = e % Nk;
     const long j = e / Nk;
     const zd z(rmu, (double)(2 * j + 1) * PI_D * temp);
@@ -1452,23 +1409,13 @@ __global__ void __launch_bounds__(256) k_filling_cp(const zd* coef, const double
     double d = (dp / p).re;
 #pragma unroll
     for (int n = 0; n < NO; ++n) d -= (zd(1.0, 0) / (z - zd(eig[n + NO * k], 0))).re;
-    dsum += d;
+    r[1] += d;
     if (j == 0) {
 #pragma unroll
-      for (int n = 0; n < NO; ++n) fsum += 0.5 * (1.0 - tanh(0.5 * (eig[n + NO * k] - rmu) / temp));
+      for (int n = 0; n < NO; ++n) r[0] += 0.5 * (1.0 - tanh(0.5 * (eig[n + NO * k] - rmu) / temp));
     }
   }
-  sh[0][threadIdx.x] = fsum;
-  sh[1][threadIdx.x] = dsum;
-  __syncthreads();
-  for (int o = blockDim.x / 2; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) {
-      sh[0][threadIdx.x] += sh[0][threadIdx.x + o];
-      sh[1][threadIdx.x] += sh[1][threadIdx.x + o];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) { part[2 * blockIdx.x] = sh[0][0]; part[2 * blockIdx.x + 1] = sh[1][0]; }
+  finish_reduce<RedSum, 2>(r, blockIdx.x, gridDim.x, part, ticket, out);
 }
 
 template <int NO>
@@ -1660,21 +1607,6 @@ void dyson(zd* G, const zd* sigma, const zd* hamk, double mu, double temp, long 
   GMOD_CHECK_LAUNCH();
 }
 
-void filling_parts(double out[2], const zd* sigma, const zd* hamk, const double* eig, double rmu, double temp,
-                   long Nk, int Nw, int No, int* err, hipStream_t s) {
-  constexpr int NB = 1024;
-  DBuf<double> part(2 * NB);
-  long tot = Nk * (long)Nw;
-  LAUNCH_NO(No, k_filling, dim3(NB), dim3(256), sigma, hamk, eig, rmu, temp, Nk, Nw, part.p, err);
-  GMOD_CHECK_LAUNCH();
-  (void)tot;
-  std::vector<double> h(2 * NB);
-  GMOD_HIP(hipMemcpyAsync(h.data(), part.p, 2 * NB * sizeof(double), hipMemcpyDeviceToHost, s));
-  GMOD_HIP(hipStreamSynchronize(s));
-  out[0] = out[1] = 0.0;
-  for (int b = 0; b < NB; ++b) { out[0] += h[2 * b]; out[1] += h[2 * b + 1]; }
-}
-
 void filling_charpoly(zd* coef, const zd* sigma, const zd* hamk, long Nk, int Nw, int No, hipStream_t s) {
   const long tot = Nk * (long)Nw;
   LAUNCH_NO(No, k_charpoly, dim3(nblk(tot, 128)), dim3(128), coef, sigma, hamk, Nk, Nw);
@@ -1683,15 +1615,13 @@ void filling_charpoly(zd* coef, const zd* sigma, const zd* hamk, long Nk, int Nw
 
 void filling_parts_cp(double out[2], const zd* coef, const double* eig, double rmu, double temp, long Nk, int Nw,
                       int No, hipStream_t s) {
-  constexpr int NB = 1024;
-  DBuf<double> part(2 * NB);
-  LAUNCH_NO(No, k_filling_cp, dim3(NB), dim3(256), coef, eig, rmu, temp, Nk, Nw, part.p);
+  Context& c = ctx();
+  LAUNCH_NO(No, k_filling_cp, dim3(red_blocks(Nk * (long)Nw)), dim3(RED_TPB), coef, eig, rmu, temp, Nk, Nw, c.red,
+            c.ticket, c.pin);
   GMOD_CHECK_LAUNCH();
-  std::vector<double> h(2 * NB);
-  GMOD_HIP(hipMemcpyAsync(h.data(), part.p, 2 * NB * sizeof(double), hipMemcpyDeviceToHost, s));
   GMOD_HIP(hipStreamSynchronize(s));
-  out[0] = out[1] = 0.0;
-  for (int b = 0; b < NB; ++b) { out[0] += h[2 * b]; out[1] += h[2 * b + 1]; }
+  out[0] = c.pin[0];
+  out[1] = c.pin[1];
 }
 
 void green0(zd* G, const double* eig, const zd* uni, double mu, double temp, long Nk, int Nw, int No,
