@@ -57,10 +57,10 @@ class ConvEngine {
   // T/Nkall, the partner slot conjugated; thresholds at 1e-9
   void chi0_ff(zd* chi, const zd* F, const double* prt, bool singlet, double temp, hipStream_t s);
 
-  // the spatial transforms of the tau reference kernels TA, TB of pair (a, b)
-  // at mu, or (diff) of their change from mu2 to mu (fchi.f90:703-812)
-  void tau_grids(cpx<R>* ta, cpx<R>* tb, int a, int b, const double* eig_d, const zd* uni_d, double mu, double mu2,
-                 bool diff, double temp, hipStream_t s);
+  // the spatial transforms of the tau reference kernels TA, TB of every
+  // orbital pair at mu, or (diff) of their change from mu2 to mu (fchi.f90:703-812)
+  void tau_grids(cpx<R>* ta, cpx<R>* tb, const double* eig_d, const zd* uni_d, double mu, double mu2, bool diff,
+                 double temp, hipStream_t s);
 
   // tail constants J (per chi pair, [l + Nchi*m]) at mu and the sawtooth
   // table (built once), in device memory
@@ -97,8 +97,9 @@ class ConvEngine {
   }
   // Eliashberg: cache FFT[V_Delta] of the qualifying pairs (feliash.f90:540)
   void prepare_gap(const zd* Vd, const double* S_h, const double* C_h, bool singlet, hipStream_t s);
-  // newdelta (un-weighted, Hermitised) <- sum V_Delta (*) F  (feliash.f90:486-635)
-  void gap(zd* nd, const zd* F, const double* prt, bool singlet, hipStream_t s);
+  // newdelta (Hermitised) <- weight sum V_Delta (*) F  (feliash.f90:486-635)
+  void gap(zd* nd, const zd* F, const double* prt, bool singlet, double weight, hipStream_t s);
+  BosonBatch<R> gap_boson(const zd* Vd) const;  // the gap's vertex pairs
   // Eliashberg in a spinful basis (feliashwithsoc.f90:520-612): the pairs
   // mkdelta_soc convolves for gap_sym and FFT[V_Delta] of each (cached when
   // memory allows); gap_soc: nd(Nkall,Nw,No,No) <- the sum over them of
@@ -132,31 +133,58 @@ class ConvEngine {
   DBuf<cpx<float>> dgbuf;                                  // G - Gref (then G0 - G0ref), k space
   // boxes of p4's forward last pass (it spans the t axis) that hold a kept
   // spatial point: a spatial-first gather skips the others
-  DBuf<unsigned char> tlive;
-  double tlive_frac = 1.0;
+  // ([1]: the same for the plan's small boxes)
+  DBuf<unsigned char> tlive[2];
+  double tlive_frac[2] = {1.0, 1.0};
   bool tlive_built = false;
+  // Tables of the batched passes: per computed chi pair the orbital pairs of
+  // its product (ProductBatch) and its slices (GatherBatch).  all / self /
+  // other: every pair, those that are their own partner (conjugated), the
+  // rest with their partners; _plain: without conjugation and partner.
+  struct PairTab {
+    int n = 0;
+    DualTab<int> prod, gat;
+  };
+  PairTab pairs_all, pairs_self, pairs_other, all_plain, self_plain, other_plain;
+  DualTab<int> orb_gat;      // GatherBatch of the No^2 outputs
+  DualTab<int> soc_inv;      // spinful basis
+  DualTab<double> soc_spin;
+  DualTab<int> fv_heads, dv_heads, all_heads;  // vertex pairs (BosonBatch)
+  DualTab<double> fv_stat;
+  DualTab<int> gap_heads, gap_off, gap_ta, gap_tb, gap_gat;
+  DualTab<double> gap_stat, gap_prt;
+  cpx<R>* work_grids(int n);  // the work buffer with room for n grids
   // the gather of a spatial-first inverse transform
   GatherStore<R> gather_sf(zd* dst, double w, const zd* J, const zd* sawc, int acc, hipStream_t s);
   std::vector<std::array<int, 2>> gap_pairs;
   std::vector<SocBosonLoad<R>> soc_vload;  // per gap pair of a spinful basis
   bool vft_cached = false;
   const zd* Vd_dev = nullptr;
-  std::vector<double> S_cache, C_cache;
   cpx<R>* grid(DBuf<cpx<R>>& b, int a, int c) { return b.p + (long)(a + op.No * c) * N; }
-  // The Sigma outputs in the order their accumulating passes run: an output
-  // (m1, l1) and its transpose (l1, m1) back to back, sharing the head passes
-  // (the spatial transforms) of their vertex sources when `share`: the
-  // bosonic grid of pair (l, m) is conj B_ml(x, -t) in every slot but slot
-  // 0, so its head passes are conj X_ml(-r, -t) plus, at t = 0, the spatial
-  // transform of the slot-0 mismatch (slot0_corr), read through the
-  // accumulating pass's source map.
-  struct SigmaPlan {
-    std::vector<int> outs;                               // m1 + No l1
-    std::vector<std::vector<std::array<int, 3>>> src;    // per output: (m, l, source-map entry)
-    std::vector<std::vector<std::array<int, 3>>> heads;  // per output, run before it: (m, l, slot)
-    int nmax = 0;                                        // head slots
+  // The Sigma outputs in groups that are run at once: an output (m1, l1) and
+  // its transpose (l1, m1) back to back, sharing the head passes (the spatial
+  // transforms) of their vertex sources when `share`: the bosonic grid of
+  // pair (l, m) is conj B_ml(x, -t) in every slot but slot 0, so its head
+  // passes are conj X_ml(-r, -t) plus, at t = 0, the spatial transform of the
+  // slot-0 mismatch (slot0_corr), read through the accumulating pass's source
+  // map.  A group holds at most `outs` outputs and `slots` heads (or one such
+  // pair of outputs).
+  struct SigmaGroup {
+    std::vector<int> outs;                             // m1 + No l1
+    std::vector<std::vector<std::array<int, 3>>> src;  // per output: (m, l, source-map entry)
+    std::vector<std::array<int, 2>> heads;             // (m, l) per head slot
+    int first_off = 0, first_src = 0, first_head = 0, first_out = 0, nsrc = 0;  // its part of sigma()'s tables
   };
-  SigmaPlan plan_sigma(bool share) const;
+  std::vector<SigmaGroup> plan_sigma(bool share, int outs, int slots) const;
+  void sigma_tables(const double* stat_h, hipStream_t s);
+  std::vector<SigmaGroup> sig_groups;
+  std::vector<double> sig_stat;
+  const cpx<R>* sig_fg = nullptr;
+  bool sig_fused = false, sig_unfused = false;
+  int sig_slots = 0, sig_outs = 0;
+  DualTab<int> sig_off, sig_map, sig_heads, sig_ta, sig_tb, sig_gat;
+  DualTab<double> sig_hstat;
+  DualTab<long> sig_hoffs;
   DBuf<int> srcmap_d;
   // The contraction form of the Sigma increment: the full transforms of the
   // vertex differences (DVt) and of the reference vertex (FVr) are stored
@@ -185,12 +213,11 @@ class ConvEngine {
   bool fv_shared = false;     // FVr holds one transform per transposed pair
   DBuf<cpx<R>> DVt;
   DBuf<int> ctab_d;
-  // an inverse transform whose first pass forms a product of 1-3 terms (PL:
-  // ProductLoad or IncProductLoad), the term count fixed at compile time so
-  // the operand pointers stay in scalar registers (a run-time term index puts
-  // the functor in scratch memory)
-  template <class PL, class ST>
-  void product_pass(const PL& pl, const ST& st, hipStream_t s);
+  // inverse transforms whose first pass forms a product of 1-3 terms (the
+  // term count fixed at compile time, so the operand pointers stay in scalar
+  // registers)
+  template <class PL>
+  void product_batches(const PL& pl, const GatherBatch<R>& gat, int n, hipStream_t s);
   void fft(cpx<R>* g, int sign, bool spatial_only, hipStream_t s);
 };
 

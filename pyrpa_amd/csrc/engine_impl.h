@@ -55,6 +55,54 @@ ConvEngine<R>::ConvEngine(const Mesh& m, const OrbPairs& p) : mesh(m), op(p) {
   }
   ol_d.alloc(ol_h.size());
   ol_d.upload(ol_h.data(), ol_h.size(), ctx().stream);
+  if (p.soc) {
+    soc_inv.set(std::vector<int>(p.inv.begin(), p.inv.end()), ctx().stream);
+    soc_spin.set(p.spin, ctx().stream);
+  }
+  // the tables of the computed pairs: all of them, and apart those that are
+  // their own partner (the tail conjugates their sum half way)
+  auto table = [&](PairTab& t, int which, bool partners) {  // 0 all, 1 self-partner, 2 the others
+    std::vector<int> pr, ga;
+    for (auto& lm : p.irr) {
+      const int l = lm[0], mm = lm[1];
+      const auto q = p.partner[mm + p.Nchi * l];
+      const bool self = q[0] == mm && q[1] == l;
+      if ((which == 1 && !self) || (which == 2 && self)) continue;
+      pr.push_back(p.ol[l][0] + p.No * p.ol[mm][0]);
+      pr.push_back(p.ol[mm][1] + p.No * p.ol[l][1]);
+      ga.push_back(mm + p.Nchi * l);
+      ga.push_back(partners && q[0] >= 0 ? q[0] + p.Nchi * q[1] : -1);
+      ga.push_back(l + p.Nchi * mm);
+      ga.push_back((which == 1 ? 1 : 0) + (p.psign[mm + p.Nchi * l] < 0 ? 2 : 0));
+    }
+    t.n = (int)pr.size() / 2;
+    t.prod.set(std::move(pr), ctx().stream);
+    t.gat.set(std::move(ga), ctx().stream);
+  };
+  table(pairs_all, 0, true);
+  table(pairs_self, 1, false);
+  table(pairs_other, 2, true);
+  // without the conjugation and the partner: the second sum of a self-partner
+  // pair, and the plain store of every pair
+  auto plain = [&](const PairTab& from, PairTab& to) {
+    to.n = from.n;
+    to.prod.set(from.prod.h, ctx().stream);
+    std::vector<int> ga = from.gat.h;
+    for (int i = 0; i < to.n; ++i) {
+      ga[4 * i + 1] = -1;
+      ga[4 * i + 3] = 0;
+    }
+    to.gat.set(std::move(ga), ctx().stream);
+  };
+  plain(pairs_self, self_plain);
+  plain(pairs_all, all_plain);
+  plain(pairs_other, other_plain);
+  std::vector<int> ga;
+  for (int o = 0; o < p.No * p.No; ++o) {
+    const int e[4] = {o, -1, 0, 0};
+    ga.insert(ga.end(), e, e + 4);
+  }
+  orb_gat.set(std::move(ga), ctx().stream);
 }
 
 template <typename R>
@@ -70,57 +118,62 @@ void ConvEngine<R>::transform_green(const zd* G, bool g0, hipStream_t s) {
   const int No = op.No;
   if (dst.n != (size_t)(No * No) * N) dst.alloc((size_t)No * No * N);
   const MeshDev md = mesh_dev(mesh);
-  for (int b = 0; b < No; ++b)
-    for (int a = 0; a < No; ++a) {
-      cpx<R>* g = grid(dst, a, b);
-      if (op.soc) {
-        const SocGreenLoad<R> ld{G, a, b, op.inv[a], op.inv[b], No, op.spin[a] * op.spin[b], md};
-        p4->exec_fused(ld, GridStore<R>{g, (unsigned)mesh.Nkall}, g, tmp.p, -1, (R)1, s);
-      } else {
-        p4->exec_fused(GreenLoad<R>{G, a, b, No, md}, GridStore<R>{g, (unsigned)mesh.Nkall}, g, tmp.p, -1, (R)1, s);
-      }
-    }
+  const GridStore<R> gs{dst.p, (unsigned)mesh.Nkall, N};
+  if (op.soc)
+    p4->exec_batch(SocGreenBatch<R>{G, No, soc_inv.ptr(), soc_spin.ptr(), md}, gs, dst.p, No * No, tmp.p, -1, (R)1, s);
+  else
+    p4->exec_batch(GreenBatch<R>{G, No, md}, gs, dst.p, No * No, tmp.p, -1, (R)1, s);
 }
 
 template <typename R>
-template <class PL, class ST>
-void ConvEngine<R>::product_pass(const PL& pl, const ST& st, hipStream_t s) {
+cpx<R>* ConvEngine<R>::work_grids(int n) {
+  if (work.n < (size_t)n * N) work.alloc((size_t)n * N);
+  return work.p;
+}
+
+// n inverse transforms of products (PL: a batch of ProductLoad or
+// IncProductLoad), item i gathered by item i of gat, in batches
+template <typename R>
+template <class PL>
+void ConvEngine<R>::product_batches(const PL& pl, const GatherBatch<R>& gat, int n, hipStream_t s) {
   const R invN = (R)(1.0 / (double)p4->transformed_points());
-  switch (pl.nterm) {
-    case 1: p4->exec_fused(pl.template fixed<1>(), st, work.p, tmp.p, +1, invN, s, true); break;
-    case 2: p4->exec_fused(pl.template fixed<2>(), st, work.p, tmp.p, +1, invN, s, true); break;
-    case 3: p4->exec_fused(pl.template fixed<3>(), st, work.p, tmp.p, +1, invN, s, true); break;
-    default: p4->exec_fused(pl, st, work.p, tmp.p, +1, invN, s, true); break;
+  const int step = p4->batch_items(n);
+  for (int i0 = 0; i0 < n; i0 += step) {
+    const int m = std::min(step, n - i0);
+    p4->exec_batch(pl.from(i0), gat.from(i0), work_grids(std::min(step, n)), m, tmp.p, +1, invN, s, true);
   }
 }
 
-// TA, TB written out by an elementwise kernel (the exponentials advance by a
-// factor per slot, at full occupancy) and then transformed; above 8 orbitals
-// the functions are evaluated inside the transform's first pass instead
+// TA, TB of every orbital pair written out by an elementwise kernel (the
+// exponentials advance by a factor per slot, at full occupancy) and then
+// transformed; above 8 orbitals the functions are evaluated inside the
+// transform's first pass instead
 template <typename R>
-void ConvEngine<R>::tau_grids(cpx<R>* ta, cpx<R>* tb, int a, int b, const double* eig_d, const zd* uni_d, double mu,
-                              double mu2, bool diff, double temp, hipStream_t s) {
+void ConvEngine<R>::tau_grids(cpx<R>* ta, cpx<R>* tb, const double* eig_d, const zd* uni_d, double mu, double mu2,
+                              bool diff, double temp, hipStream_t s) {
   const int No = op.No;
   const double beta = 1.0 / temp, dtau = beta / (double)mesh.M;
   const MeshDev md = mesh_dev(mesh);
   const unsigned S = (unsigned)mesh.Nkall;
   if (No <= 8) {
-    tau_ref_grids<R>(ta, tb, eig_d, uni_d, a, b, No, mu, mu2, diff, beta, dtau, md, s);
-    p3->exec(ta, tmp.p, -1, (R)1, s);
-    p3->exec(tb, tmp.p, -1, (R)1, s);
+    tau_ref_grids<R>(ta, tb, eig_d, uni_d, No, mu, mu2, diff, beta, dtau, md, s);
+    p3->exec_many(ta, No * No, tmp.p, -1, (R)1, s);
+    p3->exec_many(tb, No * No, tmp.p, -1, (R)1, s);
     return;
   }
-  for (int which = 0; which < 2; ++which) {
-    cpx<R>* t = which == 0 ? ta : tb;
-    if (diff) {
-      const TauRefLoad<double> cur{eig_d, uni_d, a, b, No, which, mu, beta, dtau, md};
-      const TauRefLoad<double> prev{eig_d, uni_d, a, b, No, which, mu2, beta, dtau, md};
-      p3->exec_fused(TauRefDiffLoad<R>{cur, prev}, GridStore<R>{t, S}, t, tmp.p, -1, (R)1, s);
-    } else {
-      p3->exec_fused(TauRefLoad<R>{eig_d, uni_d, a, b, No, which, mu, beta, dtau, md}, GridStore<R>{t, S}, t, tmp.p, -1,
-                     (R)1, s);
+  for (int ab = 0; ab < No * No; ++ab)
+    for (int which = 0; which < 2; ++which) {
+      const int a = ab % No, b = ab / No;
+      cpx<R>* t = (which == 0 ? ta : tb) + (long)ab * N;
+      if (diff) {
+        const TauRefLoad<double> cur{eig_d, uni_d, a, b, No, which, mu, beta, dtau, md};
+        const TauRefLoad<double> prev{eig_d, uni_d, a, b, No, which, mu2, beta, dtau, md};
+        p3->exec_fused(TauRefDiffLoad<R>{cur, prev}, GridStore<R>{t, S}, t, tmp.p, -1, (R)1, s);
+      } else {
+        p3->exec_fused(TauRefLoad<R>{eig_d, uni_d, a, b, No, which, mu, beta, dtau, md}, GridStore<R>{t, S}, t, tmp.p,
+                       -1, (R)1, s);
+      }
     }
-  }
 }
 
 // Tail constants of chi0 at chemical potential mu (fchi.f90:731-772):
@@ -142,18 +195,23 @@ void ConvEngine<R>::tail_constants(double temp, const double* eig_d, const zd* u
 template <typename R>
 GatherStore<R> ConvEngine<R>::gather_sf(zd* dst, double w, const zd* J, const zd* sawc, int acc, hipStream_t s) {
   if (!tlive_built) {
-    const std::vector<unsigned char> h = p4->fwd_last_live(mesh.kgat_host, &tlive_frac);
-    if (!h.empty()) {
-      tlive.alloc(h.size());
-      tlive.upload(h.data(), h.size(), s);
-      GMOD_HIP(hipStreamSynchronize(s));  // h is released at return
+    for (int small = 0; small < 2; ++small) {
+      const std::vector<unsigned char> h = p4->fwd_last_live(mesh.kgat_host, &tlive_frac[small], small != 0);
+      if (h.empty()) continue;
+      tlive[small].alloc(h.size());
+      tlive[small].upload(h.data(), h.size(), s);
+      GMOD_HIP(hipStreamSynchronize(s));  // h is released here
     }
     tlive_built = true;
   }
   GatherStore<R> g{dst, w, J, sawc, acc, mesh_dev(mesh)};
-  if (tlive.n) {
-    g.live = tlive.p;
-    g.live_frac = tlive_frac;
+  if (tlive[0].n) {
+    g.live = tlive[0].p;
+    g.live_frac = tlive_frac[0];
+  }
+  if (tlive[1].n) {
+    g.live_s = tlive[1].p;
+    g.live_s_frac = tlive_frac[1];
   }
   return g;
 }
@@ -162,87 +220,59 @@ template <typename R>
 void ConvEngine<R>::chi0(zd* chi, double temp, bool tail, const double* eig_d, const zd* uni_d, double mu,
                          hipStream_t s, bool apply_threshold) {
   const int No = op.No, Nchi = op.Nchi;
-  const long Nk = mesh.Nk, Nw = mesh.Nw, M = mesh.M, Nkall = mesh.Nkall;
-  const long NkNw = Nk * Nw;
-  const double w = temp / (double)Nkall;
+  const long NkNw = mesh.Nk * (long)mesh.Nw;
+  const double w = temp / (double)mesh.Nkall;
   if (tail && sizeof(R) < sizeof(double)) {
     // the tail subtraction stays FP64 when the transforms are FP32
     chi0_split_tail(chi, temp, eig_d, uni_d, mu, s);
     if (apply_threshold) threshold(chi, NkNw * Nchi * Nchi, 1e-9, s);
     return;
   }
-  DBuf<zd> Jt, sawc_d;
-  if (tail) {
-    DBuf<zd> G0((size_t)NkNw * No * No);
-    green0(G0.p, eig_d, uni_d, mu, temp, Nk, (int)Nw, No, s);
-    transform_green(G0.p, true, s);
-    if (TA.n != (size_t)(No * No) * N) { TA.alloc((size_t)No * No * N); TB.alloc((size_t)No * No * N); }
-    for (int b = 0; b < No; ++b)
-      for (int a = 0; a < No; ++a) tau_grids(grid(TA, a, b), grid(TB, a, b), a, b, eig_d, uni_d, mu, mu, false, temp, s);
-    tail_constants(temp, eig_d, uni_d, mu, Jt, sawc_d, s);
-  }
-  const double wref = 1.0 / (temp * (double)Nkall);
   const MeshDev md = mesh_dev(mesh);
-  const R invN = (R)(1.0 / (double)p4->transformed_points());
   if (!mesh.complete) GMOD_HIP(hipMemsetAsync(chi, 0, NkNw * Nchi * Nchi * sizeof(zd), s));
-  // without the tail every product is G13(r,t) G42(-r,-t): the mirrored G
-  // grids are formed once (coalesced) and then read in place.  The inverse
-  // transforms run spatial-first, so a (-r,-t) operand that is not mirrored
-  // (the tail terms) is read as whole reversed planes.
+  // the partner copies are written by the gather on a complete mesh (every
+  // slot of a slice is written), else apart
+  const bool fuse = mesh.complete;
+  auto gather = [&](const PairTab& t, double wt, const zd* J, const zd* saw, int acc) {
+    return GatherBatch<R>{chi, NkNw, t.gat.ptr(), gather_sf(chi, wt, J, saw, acc, s)};
+  };
   if (!tail) {
+    // every product is G13(r,t) G42(-r,-t): the mirrored G grids are formed
+    // once (coalesced) and then read in place.  The inverse transforms run
+    // spatial-first, so a (-r,-t) operand that is not mirrored (the tail
+    // terms) is read as whole reversed planes.
     if (Mg.n != Fg.n) Mg.alloc(Fg.n);
-    for (int b = 0; b < No; ++b)
-      for (int a = 0; a < No; ++a) mirror_grid(grid(Mg, a, b), grid(Fg, a, b), mesh.Nx, mesh.Ny, mesh.Nz, mesh.M, s);
-  }
-  for (auto& lm : op.irr) {
-    const int l = lm[0], m = lm[1];
-    const int a13 = op.ol[l][0], b13 = op.ol[m][0], a42 = op.ol[m][1], b42 = op.ol[l][1];
-    auto pr = op.partner[m + Nchi * l];
+    mirror_grid(Mg.p, Fg.p, mesh.Nx, mesh.Ny, mesh.Nz, mesh.M, No * No, s);
+    const PairTab& t = fuse ? pairs_all : all_plain;
+    product_batches(ProductBatch<R, 1>{{Fg.p}, {Mg.p}, {(R)-1}, {1}, N, t.prod.ptr(), md, 1},
+                    gather(t, w, nullptr, nullptr, 0), t.n, s);
+    if (!fuse) partner_copies(chi, pairs_all.gat.d.p, pairs_all.n, NkNw, s);
+  } else {
+    DBuf<zd> Jt, sawc_d;
+    {
+      DBuf<zd> G0((size_t)NkNw * No * No);  // its block may be reused in stream order
+      green0(G0.p, eig_d, uni_d, mu, temp, mesh.Nk, (int)mesh.Nw, No, s);
+      transform_green(G0.p, true, s);
+    }
+    if (TA.n != (size_t)(No * No) * N) { TA.alloc((size_t)No * No * N); TB.alloc((size_t)No * No * N); }
+    tau_grids(TA.p, TB.p, eig_d, uni_d, mu, mu, false, temp, s);
+    tail_constants(temp, eig_d, uni_d, mu, Jt, sawc_d, s);
+    const R wr = (R)(-1.0 / (temp * (double)mesh.Nkall));
+    // conv[G] - conv[G0] + ref in one product
+    const PairTab& t = fuse ? pairs_other : other_plain;
+    product_batches(ProductBatch<R, 3>{{Fg.p, F0g.p, TA.p}, {Fg.p, F0g.p, TB.p}, {(R)(-w), (R)w, wr}, {1, 1, 0}, N,
+                                       t.prod.ptr(), md},
+                    gather(t, 1.0, Jt.p, sawc_d.p, 0), t.n, s);
+    if (!fuse) partner_copies(chi, pairs_other.gat.d.p, pairs_other.n, NkNw, s);
     // A self-partner slice (partner == itself) is conjugated in place after each
     // of the reference's three accumulation passes (fchi.f90:610, 846); the net
     // result is conj(conv[G] + ref) - conv[G0].  It equals conj of the plain sum
     // whenever TRS holds; keep the reference's order so results match it on any
     // input.
-    const bool self_tail = tail && pr[0] == m && pr[1] == l;
-    ProductLoad<R> pl{};
-    pl.m = md;
-    if (!tail) {
-      pl.nterm = 1;
-      pl.A[0] = grid(Fg, a13, b13); pl.B[0] = grid(Mg, a42, b42); pl.coef[0] = (R)-1; pl.revt[0] = 1;
-      pl.bmir = 1;
-    } else {
-      int t = 0;
-      pl.A[t] = grid(Fg, a13, b13); pl.B[t] = grid(Fg, a42, b42); pl.coef[t] = (R)(-w); pl.revt[t++] = 1;
-      if (!self_tail) {
-        pl.A[t] = grid(F0g, a13, b13); pl.B[t] = grid(F0g, a42, b42); pl.coef[t] = (R)w; pl.revt[t++] = 1;
-      }
-      pl.A[t] = grid(TA, a13, b13); pl.B[t] = grid(TB, a42, b42); pl.coef[t] = (R)(-wref); pl.revt[t++] = 0;
-      pl.nterm = t;
-    }
-    const zd* J = tail ? Jt.p + l + Nchi * m : nullptr;
-    zd* dst = chi + NkNw * (m + (long)Nchi * l);
-    GatherStore<R> gst = gather_sf(dst, tail ? 1.0 : w, J, tail ? sawc_d.p : nullptr, 0, s);
-    // the partner copy written by the gather (a complete mesh: every slot of
-    // the slice is written)
-    const bool fuse_pr = !self_tail && pr[0] >= 0 && mesh.complete;
-    if (fuse_pr) {
-      gst.pdst = chi + NkNw * (pr[0] + (long)Nchi * pr[1]);
-      gst.psign = op.psign[m + Nchi * l];
-    }
-    product_pass(pl, gst, s);
-    if (self_tail) {
-      conj_copy(dst, dst, NkNw, s);
-      ProductLoad<R> p0{};
-      p0.m = md;
-      p0.nterm = 1;
-      p0.A[0] = grid(F0g, a13, b13); p0.B[0] = grid(F0g, a42, b42); p0.coef[0] = (R)w; p0.revt[0] = 1;
-      p4->exec_fused(p0.template fixed<1>(), gather_sf(dst, 1.0, nullptr, nullptr, 1, s), work.p, tmp.p, +1, invN, s,
-                     true);
-      continue;
-    }
-    // the spinful partner carries the sign s_l1 s_l2 s_m1 s_m2 (fchi0withsoc.f90:107)
-    if (pr[0] >= 0 && !fuse_pr)
-      conj_copy(chi + NkNw * (pr[0] + (long)Nchi * pr[1]), dst, NkNw, op.psign[m + Nchi * l], s);
+    product_batches(ProductBatch<R, 2>{{Fg.p, TA.p}, {Fg.p, TB.p}, {(R)(-w), wr}, {1, 0}, N, pairs_self.prod.ptr(), md},
+                    gather(pairs_self, 1.0, Jt.p, sawc_d.p, 0), pairs_self.n, s);
+    product_batches(ProductBatch<R, 1>{{F0g.p}, {F0g.p}, {(R)w}, {1}, N, self_plain.prod.ptr(), md},
+                    gather(self_plain, 1.0, nullptr, nullptr, 1), self_plain.n, s);
   }
   if (apply_threshold) threshold(chi, NkNw * Nchi * Nchi, 1e-9, s);
 }
@@ -273,7 +303,8 @@ void ConvEngine<R>::chi0_ff(zd* chi, const zd* F, const double* prt, bool single
     pl.m = md;
     pl.add(A, B, (R)-1, 1);
     zd* dst = chi + NkNw * (m + (long)Nchi * l);
-    product_pass(pl, gather_sf(dst, w, nullptr, nullptr, 0, s), s);
+    p4->exec_fused(pl.template fixed<1>(), gather_sf(dst, w, nullptr, nullptr, 0, s), work.p, tmp.p, +1,
+                   (R)(1.0 / (double)p4->transformed_points()), s, true);
     auto pr = op.partner[m + Nchi * l];
     if (pr[0] >= 0) conj_copy(chi + NkNw * (pr[0] + (long)Nchi * pr[1]), dst, NkNw, s);
   }
@@ -283,24 +314,13 @@ void ConvEngine<R>::chi0_ff(zd* chi, const zd* F, const double* prt, bool single
 template <typename R>
 void ConvEngine<R>::tau_reference(zd* chi, double temp, const double* eig_d, const zd* uni_d, double mu,
                                   const zd* J, const zd* sawc_d, hipStream_t s) {
-  const int No = op.No, Nchi = op.Nchi;
+  const int No = op.No;
   const long NkNw = mesh.Nk * (long)mesh.Nw;
   if (TA.n != (size_t)(No * No) * N) { TA.alloc((size_t)No * No * N); TB.alloc((size_t)No * No * N); }
-  const MeshDev md = mesh_dev(mesh);
-  for (int b = 0; b < No; ++b)
-    for (int a = 0; a < No; ++a) tau_grids(grid(TA, a, b), grid(TB, a, b), a, b, eig_d, uni_d, mu, mu, false, temp, s);
+  tau_grids(TA.p, TB.p, eig_d, uni_d, mu, mu, false, temp, s);
   const double wref = 1.0 / (temp * (double)mesh.Nkall);
-  const R invN = (R)(1.0 / (double)p4->transformed_points());
-  for (auto& lm : op.irr) {
-    const int l = lm[0], m = lm[1];
-    const int a13 = op.ol[l][0], b13 = op.ol[m][0], a42 = op.ol[m][1], b42 = op.ol[l][1];
-    ProductLoad<R> pl{};
-    pl.m = md;
-    pl.add(grid(TA, a13, b13), grid(TB, a42, b42), (R)(-wref), 0);
-    zd* dst = chi + NkNw * (m + (long)Nchi * l);
-    p4->exec_fused(pl.template fixed<1>(), gather_sf(dst, 1.0, J + l + Nchi * m, sawc_d, 1, s), work.p, tmp.p, +1,
-                   invN, s, true);
-  }
+  product_batches(ProductBatch<R, 1>{{TA.p}, {TB.p}, {(R)(-wref)}, {0}, N, all_plain.prod.ptr(), mesh_dev(mesh)},
+                  GatherBatch<R>{chi, NkNw, all_plain.gat.ptr(), gather_sf(chi, 1.0, J, sawc_d, 1, s)}, all_plain.n, s);
 }
 
 template <typename R>
@@ -318,24 +338,15 @@ void ConvEngine<R>::chi0_split_tail(zd* chi, double temp, const double* eig_d, c
   DBuf<zd> J, sawc_d;
   tail_constants(temp, eig_d, uni_d, mu, J, sawc_d, s);
   const MeshDev md = mesh_dev(mesh);
-  const R invN = (R)(1.0 / (double)p4->transformed_points());
   if (!mesh.complete) GMOD_HIP(hipMemsetAsync(chi, 0, NkNw * Nchi * Nchi * sizeof(zd), s));
-  auto is_self = [&](int l, int m) {
-    auto pr = op.partner[m + Nchi * l];
-    return pr[0] == m && pr[1] == l;
+  auto gather = [&](const PairTab& t, int acc) {
+    return GatherBatch<R>{chi, NkNw, t.gat.ptr(), gather_sf(chi, 1.0, nullptr, nullptr, acc, s)};
   };
   // 1) -w conv[G] + w conv[G0] at grid precision (a self-partner pair: -w conv[G] only)
-  for (auto& lm : op.irr) {
-    const int l = lm[0], m = lm[1];
-    const int a13 = op.ol[l][0], b13 = op.ol[m][0], a42 = op.ol[m][1], b42 = op.ol[l][1];
-    ProductLoad<R> pl{};
-    pl.m = md;
-    pl.add(grid(Fg, a13, b13), grid(Fg, a42, b42), (R)(-w), 1);
-    if (!is_self(l, m)) pl.add(grid(F0g, a13, b13), grid(F0g, a42, b42), (R)w, 1);
-    zd* dst = chi + NkNw * (m + (long)Nchi * l);
-    const GatherStore<R> gst = gather_sf(dst, 1.0, nullptr, nullptr, 0, s);
-    product_pass(pl, gst, s);
-  }
+  product_batches(ProductBatch<R, 2>{{Fg.p, F0g.p}, {Fg.p, F0g.p}, {(R)(-w), (R)w}, {1, 1}, N, other_plain.prod.ptr(), md},
+                  gather(other_plain, 0), other_plain.n, s);
+  product_batches(ProductBatch<R, 1>{{Fg.p}, {Fg.p}, {(R)(-w)}, {1}, N, self_plain.prod.ptr(), md},
+                  gather(self_plain, 0), self_plain.n, s);
   // 2) + the tau reference and the sawtooth term, FP64
   {
     ConvEngine<double> e64(mesh, op);
@@ -344,23 +355,13 @@ void ConvEngine<R>::chi0_split_tail(zd* chi, double temp, const double* eig_d, c
   }
   // 3) the reference's order for a self-partner pair, conj(conv[G] + ref) -
   //    conv[G0] (fchi.f90:610, 846, 886); partner copies of the others
-  for (auto& lm : op.irr) {
-    const int l = lm[0], m = lm[1];
-    const int a13 = op.ol[l][0], b13 = op.ol[m][0];
-    const int a42 = op.ol[m][1], b42 = op.ol[l][1];
-    zd* dst = chi + NkNw * (m + (long)Nchi * l);
-    if (is_self(l, m)) {
-      conj_copy(dst, dst, NkNw, s);
-      ProductLoad<R> p0{};
-      p0.m = md;
-      p0.add(grid(F0g, a13, b13), grid(F0g, a42, b42), (R)w, 1);
-      p4->exec_fused(p0.template fixed<1>(), gather_sf(dst, 1.0, nullptr, nullptr, 1, s), work.p, tmp.p, +1, invN,
-                     s, true);
-      continue;
-    }
-    auto pr = op.partner[m + Nchi * l];
-    if (pr[0] >= 0) conj_copy(chi + NkNw * (pr[0] + (long)Nchi * pr[1]), dst, NkNw, s);
+  for (int i = 0; i < pairs_self.n; ++i) {
+    zd* dst = chi + NkNw * pairs_self.gat.h[4 * i];
+    conj_copy(dst, dst, NkNw, s);
   }
+  product_batches(ProductBatch<R, 1>{{F0g.p}, {F0g.p}, {(R)w}, {1}, N, self_plain.prod.ptr(), md},
+                  gather(self_plain, 1), self_plain.n, s);
+  partner_copies(chi, pairs_other.gat.d.p, pairs_other.n, NkNw, s);
 }
 
 template <typename R>
@@ -427,9 +428,9 @@ bool ConvEngine<R>::contract_form() const {
 }
 
 template <typename R>
-typename ConvEngine<R>::SigmaPlan ConvEngine<R>::plan_sigma(bool share) const {
+std::vector<typename ConvEngine<R>::SigmaGroup> ConvEngine<R>::plan_sigma(bool share, int outs, int slots) const {
   const int No = op.No, Nchi = op.Nchi;
-  SigmaPlan P;
+  std::vector<SigmaGroup> P;
   std::vector<char> done((size_t)No * No, 0);
   for (int l1 = 0; l1 < No; ++l1)
     for (int m1 = 0; m1 < No; ++m1) {
@@ -437,10 +438,11 @@ typename ConvEngine<R>::SigmaPlan ConvEngine<R>::plan_sigma(bool share) const {
       if (done[o]) continue;
       std::vector<int> batch{o};
       if (share && m1 != l1) batch.push_back(l1 + No * m1);
+      SigmaGroup B;
       std::map<std::pair<int, int>, int> slot;  // (m, l) -> head slot of this batch
       for (int ob : batch) {
         const int bm1 = ob % No, bl1 = ob / No;
-        std::vector<std::array<int, 3>> srcl, heads;
+        std::vector<std::array<int, 3>> srcl;
         for (int l = 0; l < Nchi; ++l)
           for (int m = 0; m < Nchi; ++m) {
             if (op.ol[m][0] != bm1 || op.ol[l][0] != bl1) continue;
@@ -453,17 +455,30 @@ typename ConvEngine<R>::SigmaPlan ConvEngine<R>::plan_sigma(bool share) const {
             } else {
               const int sl = (int)slot.size();
               slot[{m, l}] = sl;
-              heads.push_back({m, l, sl});
+              B.heads.push_back({m, l});
               e = 2 * sl;
             }
             srcl.push_back({m, l, e});
           }
-        P.outs.push_back(ob);
-        P.src.push_back(srcl);
-        P.heads.push_back(heads);
+        B.outs.push_back(ob);
+        B.src.push_back(srcl);
         done[ob] = 1;
       }
-      P.nmax = std::max(P.nmax, (int)slot.size());
+      // joined to the last group while that stays within its outputs and slots
+      // (outputs without a source stay apart: they are only zeroed)
+      if (!P.empty() && !B.heads.empty() && !P.back().heads.empty() &&
+          (int)(P.back().outs.size() + B.outs.size()) <= std::max(outs, 1) &&
+          (int)(P.back().heads.size() + B.heads.size()) <= slots) {
+        SigmaGroup& G = P.back();
+        const int base = (int)G.heads.size();
+        for (auto& sl : B.src)
+          for (auto& e : sl) e[2] += 2 * base;
+        G.outs.insert(G.outs.end(), B.outs.begin(), B.outs.end());
+        G.src.insert(G.src.end(), B.src.begin(), B.src.end());
+        G.heads.insert(G.heads.end(), B.heads.begin(), B.heads.end());
+      } else {
+        P.push_back(std::move(B));
+      }
     }
   return P;
 }
@@ -478,92 +493,114 @@ void ConvEngine<R>::sigma(zd* sig, const zd* V, const double* S_h, const double*
   sigma(sig, V, stat.data(), temp, s, apply_threshold);
 }
 
+// The tables of sigma() for one static part: built on first use and when it
+// or the transformed G's place changes
+template <typename R>
+void ConvEngine<R>::sigma_tables(const double* stat_h, hipStream_t s) {
+  const int No = op.No, Nchi = op.Nchi;
+  const std::vector<double> st(stat_h, stat_h + (size_t)Nchi * Nchi);
+  const bool unfused = sigma_unfused();
+  if (!sig_groups.empty() && st == sig_stat && sig_fg == Fg.p && sig_unfused == unfused) return;
+  sig_stat = st;
+  sig_fg = Fg.p;
+  sig_unfused = unfused;
+  // the accumulating last pass sums the pairs of one output in registers;
+  // shapes it does not cover (and GMOD_SIGMA_UNFUSED=1) transform every
+  // source whole and sum them in one streaming kernel
+  sig_fused = p4->accum_ok(-1) && !unfused;
+  // transposed outputs share their sources' head passes when the static
+  // slot is symmetric (the conjugate-reversal relation of the sources, with
+  // the slot-0 correction)
+  bool share = sig_fused && p4->accum_last_is_t(-1) && p4->reversal_ok();
+  for (int l = 0; l < Nchi && share; ++l)
+    for (int m = 0; m < Nchi; ++m)
+      if (stat_h[m + Nchi * l] != stat_h[l + Nchi * m]) { share = false; break; }
+  // as many outputs at once as give the CUs several rounds of boxes, their
+  // sources within 4 GB
+  const long slots = std::max<long>(1, (4L << 30) / (N * (long)sizeof(cpx<R>)));
+  sig_groups = plan_sigma(share, p4->batch_items(No * No), (int)std::min<long>(slots, 1 << 20));
+  std::vector<int> smap, off, heads, ta, tb, gat;
+  std::vector<double> hstat;
+  std::vector<long> hoffs;
+  accum_tab_h.clear();
+  sig_slots = 0;
+  sig_outs = 0;
+  for (auto& g : sig_groups) {
+    g.first_off = (int)off.size();
+    g.first_src = (int)smap.size();
+    g.first_head = (int)heads.size() / 2;
+    g.first_out = (int)gat.size() / 4;
+    off.push_back(0);
+    int c = 0;
+    for (size_t i = 0; i < g.outs.size(); ++i) {
+      for (auto& e : g.src[i]) {
+        const int ab = op.ol[e[0]][1] + No * op.ol[e[1]][1];
+        accum_tab_h.push_back(Fg.p + (long)ab * N);
+        smap.push_back(e[2]);
+        ta.push_back(e[2] >> 1);
+        tb.push_back(ab);
+        ++c;
+      }
+      off.push_back(c);
+      const int gt[4] = {g.outs[i], -1, 0, 0};
+      gat.insert(gat.end(), gt, gt + 4);
+    }
+    g.nsrc = c;
+    for (auto& h : g.heads) {
+      heads.push_back(h[0] + Nchi * h[1]);
+      heads.push_back(h[1] + Nchi * h[0]);
+      hstat.push_back(stat_h[h[0] + Nchi * h[1]]);
+      head_offsets(hoffs, h[0], h[1]);
+    }
+    sig_slots = std::max(sig_slots, (int)g.heads.size());
+    sig_outs = std::max(sig_outs, (int)g.outs.size());
+  }
+  sig_off.set(std::move(off), s);
+  sig_map.set(std::move(smap), s);
+  sig_heads.set(std::move(heads), s);
+  sig_hstat.set(std::move(hstat), s);
+  sig_hoffs.set(std::move(hoffs), s);
+  sig_ta.set(std::move(ta), s);
+  sig_tb.set(std::move(tb), s);
+  sig_gat.set(std::move(gat), s);
+  accum_tab.alloc(accum_tab_h.size());
+  accum_tab.upload(accum_tab_h.data(), accum_tab_h.size(), s);
+  GMOD_HIP(hipStreamSynchronize(s));
+}
+
 template <typename R>
 void ConvEngine<R>::sigma(zd* sig, const zd* V, const double* stat_h, double temp, hipStream_t s,
                           bool apply_threshold) {
-  const int No = op.No, Nchi = op.Nchi;
+  const int No = op.No;
   const long NkNw = mesh.Nk * (long)mesh.Nw;
-  if (acc.n != (size_t)N) acc.alloc(N);
   const MeshDev md = mesh_dev(mesh);
+  const unsigned S = (unsigned)mesh.Nkall;
   const R invN = (R)(1.0 / (double)p4->transformed_points());
-  const long NC = NkNw;
-  // the accumulating last pass sums the pairs of one output in registers
-  // (GMOD_SIGMA_UNFUSED=1: one pass per pair, accumulating through memory)
-  const bool fused = p4->accum_ok(-1) && !sigma_unfused();
-  auto gather_out = [&](int m1, int l1, bool any) {
-    zd* dst = sig + NkNw * (m1 + (long)No * l1);
-    if (!any) {
-      GMOD_HIP(hipMemsetAsync(dst, 0, NkNw * sizeof(zd), s));
-      return;
+  sigma_tables(stat_h, s);
+  if (srcs.n < (size_t)sig_slots * N) srcs.alloc((size_t)sig_slots * N);
+  if (acc.n < (size_t)sig_outs * N) acc.alloc((size_t)sig_outs * N);
+  if (!mesh.complete) GMOD_HIP(hipMemsetAsync(sig, 0, NkNw * No * No * sizeof(zd), s));
+  const GatherBatch<R> gat{sig, NkNw, sig_gat.ptr(),
+                           GatherStore<R>{sig, temp / (double)mesh.Nkall, nullptr, nullptr, 0, md}};
+  const BosonBatch<R> heads{V, NkNw, sig_heads.ptr(), sig_hstat.ptr(), md};
+  for (const SigmaGroup& g : sig_groups) {
+    const int nh = (int)g.heads.size(), no = (int)g.outs.size();
+    if (g.nsrc == 0) {
+      for (int o : g.outs) GMOD_HIP(hipMemsetAsync(sig + NkNw * o, 0, NkNw * sizeof(zd), s));
+      continue;
     }
-    if (!mesh.complete) GMOD_HIP(hipMemsetAsync(dst, 0, NkNw * sizeof(zd), s));
-    p4->exec_fused(GridLoad<R>{acc.p, (unsigned)mesh.Nkall},
-                   GatherStore<R>{dst, temp / (double)mesh.Nkall, nullptr, nullptr, 0, md}, acc.p, tmp.p, +1, invN, s);
-  };
-  if (fused) {
-    // transposed outputs share their sources' head passes when the static
-    // slot is symmetric (the conjugate-reversal relation of the sources, with
-    // the slot-0 correction)
-    bool share = p4->accum_last_is_t(-1) && p4->reversal_ok();
-    for (int l = 0; l < Nchi && share; ++l)
-      for (int m = 0; m < Nchi; ++m)
-        if (stat_h[m + Nchi * l] != stat_h[l + Nchi * m]) { share = false; break; }
-    const SigmaPlan P = plan_sigma(share);
-    accum_tab_h.clear();
-    std::vector<int> smap;
-    for (size_t i = 0; i < P.outs.size(); ++i)
-      for (auto& e : P.src[i]) {
-        accum_tab_h.push_back(grid(Fg, op.ol[e[0]][1], op.ol[e[1]][1]));
-        smap.push_back(e[2]);
-      }
-    if (srcs.n != (size_t)P.nmax * N) srcs.alloc((size_t)P.nmax * N);
-    accum_tab.alloc(accum_tab_h.size());
-    accum_tab.upload(accum_tab_h.data(), accum_tab_h.size(), s);
-    srcmap_d.alloc(smap.size());
-    srcmap_d.upload(smap.data(), smap.size(), s);
-    std::vector<long> hoffs;
-    for (auto& hs : P.heads)
-      for (auto& h : hs) head_offsets(hoffs, h[0], h[1]);
-    if (dh_offs.n < hoffs.size()) dh_offs.alloc(hoffs.size());
-    if (!hoffs.empty()) dh_offs.upload(hoffs.data(), hoffs.size(), s);
-    if (dhD.n < (size_t)P.nmax * mesh.Nkall) dhD.alloc((size_t)P.nmax * mesh.Nkall);
-    GMOD_HIP(hipStreamSynchronize(s));
-    long off = 0, hoff = 0;
-    for (size_t i = 0; i < P.outs.size(); ++i) {
-      for (auto& h : P.heads[i]) {
-        const int m = h[0], l = h[1];
-        const zd stat(stat_h[m + Nchi * l], 0);
-        p4->exec_head(BosonLoad<R>{V, NC * (m + (long)Nchi * l), NC * (l + (long)Nchi * m), stat, md},
-                      srcs.p + (long)h[2] * N, tmp.p, -1, s);
-      }
-      // the heads of one output take consecutive slots
-      if (!P.heads[i].empty())
-        slot0_corr(dhD.p + (size_t)P.heads[i][0][2] * mesh.Nkall, V, dh_offs.p + 2 * hoff, (int)P.heads[i].size(),
-                   s);
-      hoff += (long)P.heads[i].size();
-      const int nsrc = (int)P.src[i].size();
-      if (nsrc > 0)
-        p4->exec_accum_last(srcs.p, N, nsrc, MulAccAccum<R>{accum_tab.p + off, acc.p, (unsigned)mesh.Nkall}, -1,
-                            (R)1, s, srcmap_d.p + off, dhD.p);
-      off += nsrc;
-      gather_out(P.outs[i] % No, P.outs[i] / No, nsrc > 0);
+    if (sig_fused) {
+      p4->exec_head(heads.from(g.first_head), srcs.p, nh, tmp.p, -1, s);
+      if (dhD.n < (size_t)nh * S) dhD.alloc((size_t)nh * S);
+      slot0_corr(dhD.p, V, sig_hoffs.d.p + 2 * (long)g.first_head, nh, s);
+      p4->exec_accum_last(srcs.p, N, g.nsrc, MulAccAccum<R>{accum_tab.p + g.first_src, acc.p, S, N}, -1, (R)1, s,
+                          sig_map.d.p + g.first_src, dhD.p, sig_off.d.p + g.first_off, no);
+    } else {
+      p4->exec_batch(heads.from(g.first_head), GridStore<R>{srcs.p, S, N}, srcs.p, nh, tmp.p, -1, (R)1, s);
+      contract<R>(acc.p, srcs.p, Fg.p, sig_off.d.p + g.first_off, sig_ta.d.p + g.first_src, sig_tb.d.p + g.first_src,
+                  no, N, s);
     }
-  } else {
-    for (int l1 = 0; l1 < No; ++l1)
-      for (int m1 = 0; m1 < No; ++m1) {
-        bool first = true;
-        for (int l = 0; l < Nchi; ++l)
-          for (int m = 0; m < Nchi; ++m) {
-            if (op.ol[m][0] != m1 || op.ol[l][0] != l1) continue;
-            const zd stat(stat_h[m + Nchi * l], 0);
-            BosonLoad<R> bl{V, NC * (m + (long)Nchi * l), NC * (l + (long)Nchi * m), stat, md};
-            p4->exec_fused(bl, MulAccStore<R>{acc.p, grid(Fg, op.ol[m][1], op.ol[l][1]), first ? 1 : 0,
-                                              (unsigned)mesh.Nkall},
-                           work.p, tmp.p, -1, (R)1, s);
-            first = false;
-          }
-        gather_out(m1, l1, !first);
-      }
+    p4->exec_batch(GridLoad<R>{acc.p, S, N}, gat.from(g.first_out), acc.p, no, tmp.p, +1, invN, s);
   }
   if (apply_threshold) threshold(sig, NkNw * No * No, 1e-9, s);
 }
@@ -576,62 +613,86 @@ void ConvEngine<R>::prepare_gap(const zd* Vd, const double* S_h, const double* C
   for (int l = 0; l < Nchi; ++l)
     for (int m = 0; m < Nchi; ++m)
       if (op.ol[l][0] >= op.ol[m][1]) gap_pairs.push_back({l, m});
-  S_cache.assign(S_h, S_h + Nchi * Nchi);
-  C_cache.assign(C_h, C_h + Nchi * Nchi);
+  {
+    std::vector<int> heads, off{0}, ta, tb, gat;
+    std::vector<double> stat;
+    for (auto& p : gap_pairs) {
+      const int l = p[0], m = p[1];
+      heads.push_back(m + Nchi * l);
+      heads.push_back(l + Nchi * m);
+      stat.push_back(0.5 * (S_h[m + Nchi * l] + sgn * C_h[m + Nchi * l]));
+    }
+    for (int m2 = 0; m2 < op.No; ++m2)
+      for (int l1 = 0; l1 < op.No; ++l1) {
+        for (size_t q = 0; q < gap_pairs.size(); ++q) {
+          const int l = gap_pairs[q][0], m = gap_pairs[q][1];
+          if (op.ol[l][0] != l1 || op.ol[m][1] != m2) continue;
+          ta.push_back((int)q);
+          tb.push_back(op.ol[l][1] + op.No * op.ol[m][0]);
+        }
+        if ((int)ta.size() == off.back()) continue;
+        off.push_back((int)ta.size());
+        const int g[4] = {l1 + op.No * m2, -1, 0, 0};
+        gat.insert(gat.end(), g, g + 4);
+      }
+    gap_heads.set(std::move(heads), s);
+    gap_stat.set(std::move(stat), s);
+    gap_off.set(std::move(off), s);
+    gap_ta.set(std::move(ta), s);
+    gap_tb.set(std::move(tb), s);
+    gap_gat.set(std::move(gat), s);
+  }
   Vd_dev = Vd;
   size_t free_b = 0, total_b = 0;
   GMOD_HIP(hipMemGetInfo(&free_b, &total_b));
   const double need = (double)gap_pairs.size() * N * sizeof(cpx<R>);
   vft_cached = need < 0.5 * (double)free_b;
   if (!vft_cached) return;
-  Vft.alloc(gap_pairs.size() * (size_t)N);
-  const MeshDev md = mesh_dev(mesh);
-  const long NC = mesh.Nk * (long)mesh.Nw;
-  for (size_t q = 0; q < gap_pairs.size(); ++q) {
-    int l = gap_pairs[q][0], m = gap_pairs[q][1];
-    zd stat(0.5 * (S_h[m + Nchi * l] + sgn * C_h[m + Nchi * l]), 0);
-    cpx<R>* g = Vft.p + q * N;
-    p4->exec_fused(BosonLoad<R>{Vd, NC * (m + (long)Nchi * l), NC * (l + (long)Nchi * m), stat, md}, GridStore<R>{g, (unsigned)mesh.Nkall},
-                   g, tmp.p, -1, (R)1, s);
+  if (Vft.n != gap_pairs.size() * (size_t)N) Vft.alloc(gap_pairs.size() * (size_t)N);
+  const int n = (int)gap_pairs.size(), step = p4->batch_items(n);
+  for (int i0 = 0; i0 < n; i0 += step) {
+    cpx<R>* g = Vft.p + (long)i0 * N;
+    p4->exec_batch(gap_boson(Vd).from(i0), GridStore<R>{g, (unsigned)mesh.Nkall, N}, g, std::min(step, n - i0), tmp.p,
+                   -1, (R)1, s);
   }
 }
 
 template <typename R>
-void ConvEngine<R>::gap(zd* nd, const zd* F, const double* prt, bool singlet, hipStream_t s) {
-  const int No = op.No, Nchi = op.Nchi;
+BosonBatch<R> ConvEngine<R>::gap_boson(const zd* Vd) const {
+  return BosonBatch<R>{Vd, mesh.Nk * (long)mesh.Nw, gap_heads.ptr(), gap_stat.ptr(), mesh_dev(mesh)};
+}
+
+template <typename R>
+void ConvEngine<R>::gap(zd* nd, const zd* F, const double* prt, bool singlet, double weight, hipStream_t s) {
+  const int No = op.No;
   const long NkNw = mesh.Nk * (long)mesh.Nw;
   const double sgn = singlet ? 1.0 : -1.0, dprt = sgn;
   if (Ff.n != (size_t)(No * No) * N) Ff.alloc((size_t)No * No * N);
-  if (acc.n != (size_t)N) acc.alloc(N);
   const MeshDev md = mesh_dev(mesh);
+  const unsigned S = (unsigned)mesh.Nkall;
   const R invN = (R)(1.0 / (double)p4->transformed_points());
-  for (int b = 0; b < No; ++b)
-    for (int a = 0; a < No; ++a) {
-      cpx<R>* g = grid(Ff, a, b);
-      AnomLoad<R> al{F, NkNw * (a + (long)No * b), NkNw * (b + (long)No * a), prt[a] * prt[b], sgn, dprt, md};
-      p4->exec_fused(al, GridStore<R>{g, (unsigned)mesh.Nkall}, g, tmp.p, -1, (R)1, s);
-    }
+  if (gap_prt.h != std::vector<double>(prt, prt + No)) gap_prt.set(std::vector<double>(prt, prt + No), s);
+  p4->exec_batch(AnomBatch<R>{F, NkNw, No, gap_prt.ptr(), sgn, dprt, md}, GridStore<R>{Ff.p, S, N}, Ff.p, No * No, tmp.p,
+                 -1, (R)1, s);
   GMOD_HIP(hipMemsetAsync(nd, 0, NkNw * No * No * sizeof(zd), s));
-  for (int m2 = 0; m2 < No; ++m2)
-    for (int l1 = 0; l1 < No; ++l1) {
-      bool first = true;
-      for (size_t q = 0; q < gap_pairs.size(); ++q) {
-        int l = gap_pairs[q][0], m = gap_pairs[q][1];
-        if (op.ol[l][0] != l1 || op.ol[m][1] != m2) continue;
-        const cpx<R>* fg = grid(Ff, op.ol[l][1], op.ol[m][0]);
-        if (vft_cached) {
-          mul_acc<R>(acc.p, Vft.p + q * N, fg, first, N, s);
-        } else {
-          zd stat(0.5 * (S_cache[m + Nchi * l] + sgn * C_cache[m + Nchi * l]), 0);
-          BosonLoad<R> bl{Vd_dev, NkNw * (m + (long)Nchi * l), NkNw * (l + (long)Nchi * m), stat, md};
-          p4->exec_fused(bl, MulAccStore<R>{acc.p, fg, first ? 1 : 0, (unsigned)mesh.Nkall}, work.p, tmp.p, -1, (R)1, s);
-        }
-        first = false;
-      }
-      if (first) continue;
-      p4->exec_fused(GridLoad<R>{acc.p, (unsigned)mesh.Nkall}, GatherStore<R>{nd + NkNw * (l1 + (long)No * m2), 1.0, nullptr, nullptr, 0, md},
-                     acc.p, tmp.p, +1, invN, s);
+  // the outputs (l1, m2) that have pairs, their products summed in pair order
+  const int nout = (int)gap_gat.h.size() / 4, step = p4->batch_items(nout);
+  if (acc.n < (size_t)step * N) acc.alloc((size_t)step * N);
+  const GatherBatch<R> gat{nd, NkNw, gap_gat.ptr(), GatherStore<R>{nd, weight, nullptr, nullptr, 0, md}};
+  for (int o0 = 0; o0 < nout; o0 += step) {
+    const int no = std::min(step, nout - o0);
+    if (vft_cached) {
+      contract<R>(acc.p, Vft.p, Ff.p, gap_off.d.p + o0, gap_ta.d.p, gap_tb.d.p, no, N, s);
+    } else {
+      for (int o = o0; o < o0 + no; ++o)
+        for (int c = gap_off.h[o]; c < gap_off.h[o + 1]; ++c)
+          p4->exec_fused(gap_boson(Vd_dev).from(gap_ta.h[c]),
+                         MulAccStore<R>{acc.p + (long)(o - o0) * N, Ff.p + (long)gap_tb.h[c] * N,
+                                        c == gap_off.h[o] ? 1 : 0, S},
+                         work.p, tmp.p, -1, (R)1, s);
     }
+    p4->exec_batch(GridLoad<R>{acc.p, S, N}, gat.from(o0), acc.p, no, tmp.p, +1, invN, s);
+  }
   hermitize_lower(nd, mesh.Nk, mesh.Nw, No, s);
 }
 
@@ -680,7 +741,7 @@ void ConvEngine<R>::gap_soc(zd* nd, const zd* F, hipStream_t s) {
   const int No = op.No;
   const long NW = mesh.Nkall * (long)mesh.Nw;
   if (Ff.n != (size_t)(No * No) * N) Ff.alloc((size_t)No * No * N);
-  if (acc.n != (size_t)N) acc.alloc(N);
+  if (acc.n < (size_t)N) acc.alloc(N);
   const MeshDev md = mesh_dev(mesh);
   const R invN = (R)(1.0 / (double)p4->transformed_points());
   std::vector<char> need((size_t)No * No, 0);
@@ -732,19 +793,11 @@ void ConvEngine<R>::set_reference(const zd* Gref, const zd* G0ref, bool tail, co
   const unsigned S = (unsigned)mesh.Nkall;
   auto ensure = [&](DBuf<cpx<R>>& b) { if (b.n != nb) b.alloc(nb); };
   ensure(Fr); ensure(Fd);
-  for (int b = 0; b < No; ++b)
-    for (int a = 0; a < No; ++a) {
-      cpx<R>* g = grid(Fr, a, b);
-      p4->exec_fused(GreenLoad<R>{Gref, a, b, No, md}, GridStore<R>{g, S}, g, tmp.p, -1, (R)1, s);
-    }
+  p4->exec_batch(GreenBatch<R>{Gref, No, md}, GridStore<R>{Fr.p, S, N}, Fr.p, No * No, tmp.p, -1, (R)1, s);
   if (!tail) return;
   ensure(F0r); ensure(F0d); ensure(TAr); ensure(TBr); ensure(TAd); ensure(TBd);
-  for (int b = 0; b < No; ++b)
-    for (int a = 0; a < No; ++a) {
-      cpx<R>* g = grid(F0r, a, b);
-      p4->exec_fused(GreenLoad<R>{G0ref, a, b, No, md}, GridStore<R>{g, S}, g, tmp.p, -1, (R)1, s);
-      tau_grids(grid(TAr, a, b), grid(TBr, a, b), a, b, eig_d, uni_d, mu_ref, mu_ref, false, temp, s);
-    }
+  p4->exec_batch(GreenBatch<R>{G0ref, No, md}, GridStore<R>{F0r.p, S, N}, F0r.p, No * No, tmp.p, -1, (R)1, s);
+  tau_grids(TAr.p, TBr.p, eig_d, uni_d, mu_ref, mu_ref, false, temp, s);
 }
 
 template <typename R>
@@ -785,12 +838,21 @@ void ConvEngine<R>::set_vertex_reference(const zd* Vref, const double* S_h, cons
     slot0_corr(dhF.p, Vref, dhF_offs.p, (int)heads.size(), s);
     GMOD_HIP(hipStreamSynchronize(s));  // hoffs is released here
   }
-  for (size_t h = 0; h < heads.size(); ++h) {
-    const int m = heads[h][0], l = heads[h][1];
-    zd stat(1.5 * S_h[m + Nchi * l] - 0.5 * C_h[m + Nchi * l], 0);
-    cpx<R>* g = FVr.p + h * N;
-    p4->exec_fused(BosonLoad<R>{Vref, NC * (m + (long)Nchi * l), NC * (l + (long)Nchi * m), stat, md},
-                   GridStore<R>{g, S}, g, tmp.p, -1, (R)1, s);
+  std::vector<int> sl;
+  std::vector<double> st;
+  for (auto& h : heads) {
+    const int m = h[0], l = h[1];
+    sl.push_back(m + Nchi * l);
+    sl.push_back(l + Nchi * m);
+    st.push_back(1.5 * S_h[m + Nchi * l] - 0.5 * C_h[m + Nchi * l]);
+  }
+  fv_heads.set(std::move(sl), s);
+  fv_stat.set(std::move(st), s);
+  const BosonBatch<R> bb{Vref, NC, fv_heads.ptr(), fv_stat.ptr(), md};
+  const int n = (int)heads.size(), step = p4->batch_items(n);
+  for (int i0 = 0; i0 < n; i0 += step) {
+    cpx<R>* g = FVr.p + (long)i0 * N;
+    p4->exec_batch(bb.from(i0), GridStore<R>{g, S, N}, g, std::min(step, n - i0), tmp.p, -1, (R)1, s);
   }
 }
 
@@ -814,85 +876,48 @@ void ConvEngine<R>::chi0_increment(zd* chi, const zd* chi_base, const zd* G, con
     if constexpr (sizeof(R) == 4) {
       if (dgbuf.n != (size_t)nG) dgbuf.alloc(nG);
       diff_to_f32(dgbuf.p, X, Xref, nG, s);
-      for (int b = 0; b < No; ++b)
-        for (int a = 0; a < No; ++a) {
-          cpx<R>* g = grid(F, a, b);
-          p4->exec_fused(GreenLoad<R, float>{dgbuf.p, a, b, No, md}, GridStore<R>{g, S}, g, tmp.p, -1, (R)1, s);
-        }
+      p4->exec_batch(GreenBatch<R, float>{dgbuf.p, No, md}, GridStore<R>{F.p, S, N}, F.p, No * No, tmp.p, -1, (R)1, s);
     } else {
-      for (int b = 0; b < No; ++b)
-        for (int a = 0; a < No; ++a) {
-          cpx<R>* g = grid(F, a, b);
-          GreenDiffLoad<R> dl{GreenLoad<double>{X, a, b, No, md}, GreenLoad<double>{Xref, a, b, No, md}};
-          p4->exec_fused(dl, GridStore<R>{g, S}, g, tmp.p, -1, (R)1, s);
-        }
+      throw Error("chi0_increment: FP32 transforms only");
     }
   };
   diff_pass(G, Gref, Fd);
-  DBuf<zd> slice;
   if (tail) {
     diff_pass(G0, G0ref, F0d);
-    for (int b = 0; b < No; ++b)
-      for (int a = 0; a < No; ++a)
-        tau_grids(grid(TAd, a, b), grid(TBd, a, b), a, b, eig_d, uni_d, mu, mu_ref, true, temp, s);
+    tau_grids(TAd.p, TBd.p, eig_d, uni_d, mu, mu_ref, true, temp, s);
   }
-  for (auto& lm : op.irr) {
-    auto pr = op.partner[lm[1] + Nchi * lm[0]];
-    if (pr[0] == lm[1] && pr[1] == lm[0] && slice.n != (size_t)NkNw) slice.alloc(NkNw);
+  // (mirrored copies as in chi0 measured no faster here: the 2 No^2 copies
+  // per iteration cost what the in-place reads save, and the spatial-first
+  // inverse reads the (-r,-t) operands as whole reversed planes)
+  const bool fuse = mesh.complete;
+  auto gather = [&](const PairTab& t, double wt, bool jumps, const zd* base, int acc_) {
+    GatherStore<R> g = gather_sf(chi, wt, jumps ? dJ : nullptr, jumps ? sawc_d : nullptr, acc_, s);
+    g.base = base;
+    return GatherBatch<R>{chi, NkNw, t.gat.ptr(), g};
+  };
+  const PairTab& t = fuse ? pairs_other : other_plain;
+  if (tail) {
+    const R mw = (R)(-w), pw = (R)w, mr = (R)(-wref);
+    product_batches(IncProductBatch<R, 3>{{Fr.p, F0r.p, TAr.p}, {Fd.p, F0d.p, TAd.p}, {Fr.p, F0r.p, TBr.p},
+                                          {Fd.p, F0d.p, TBd.p}, {mw, pw, mr}, {1, 1, 0}, N, t.prod.ptr(), md},
+                    gather(t, 1.0, true, chi_base, 0), t.n, s);
+    // a self-partner pair: the increment of conj(conv[G] + ref) - conv[G0]
+    product_batches(IncProductBatch<R, 2>{{Fr.p, TAr.p}, {Fd.p, TAd.p}, {Fr.p, TBr.p}, {Fd.p, TBd.p}, {mw, mr}, {1, 0},
+                                          N, pairs_self.prod.ptr(), md},
+                    gather(pairs_self, 1.0, true, chi_base, 0), pairs_self.n, s);
+    product_batches(IncProductBatch<R, 1>{{F0r.p}, {F0d.p}, {F0r.p}, {F0d.p}, {pw}, {1}, N, self_plain.prod.ptr(), md},
+                    gather(self_plain, 1.0, false, nullptr, 1), self_plain.n, s);
+  } else {
+    // (the reference conjugates a self-partner pair in place after the
+    // accumulation, fchi.f90:610: the stored value is conj(conv[G]), so the
+    // increment is conjugated before it is added)
+    auto inc = [&](const PairTab& q) {
+      return IncProductBatch<R, 1>{{Fr.p}, {Fd.p}, {Fr.p}, {Fd.p}, {(R)-1}, {1}, N, q.prod.ptr(), md};
+    };
+    product_batches(inc(t), gather(t, w, false, chi_base, 0), t.n, s);
+    product_batches(inc(pairs_self), gather(pairs_self, w, false, chi_base, 0), pairs_self.n, s);
   }
-
-  for (auto& lm : op.irr) {
-    const int l = lm[0], m = lm[1];
-    const int a13 = op.ol[l][0], b13 = op.ol[m][0], a42 = op.ol[m][1], b42 = op.ol[l][1];
-    auto pr = op.partner[m + Nchi * l];
-    const bool self = pr[0] == m && pr[1] == l;
-    const bool self_tail = tail && self;
-    IncProductLoad<R> pl{};
-    pl.m = md;
-    // (mirrored copies as in chi0 measured no faster here: the 2 No^2 copies
-    // per iteration cost what the in-place reads save, and the spatial-first
-    // inverse reads the (-r,-t) operands as whole reversed planes)
-    pl.add(grid(Fr, a13, b13), grid(Fd, a13, b13), grid(Fr, a42, b42), grid(Fd, a42, b42), (R)(tail ? -w : -1.0), 1);
-    if (tail) {
-      if (!self_tail)
-        pl.add(grid(F0r, a13, b13), grid(F0d, a13, b13), grid(F0r, a42, b42), grid(F0d, a42, b42), (R)w, 1);
-      pl.add(grid(TAr, a13, b13), grid(TAd, a13, b13), grid(TBr, a42, b42), grid(TBd, a42, b42), (R)(-wref), 0);
-    }
-    const zd* J = tail ? dJ + l + Nchi * m : nullptr;
-    zd* dst = chi + NkNw * (m + (long)Nchi * l);
-    const zd* base = chi_base + NkNw * (m + (long)Nchi * l);
-    if (self_tail) {
-      // increment of conj(conv[G] + ref) - conv[G0], formed apart and then added
-      if (!mesh.complete) GMOD_HIP(hipMemsetAsync(slice.p, 0, NkNw * sizeof(zd), s));
-      product_pass(pl, gather_sf(slice.p, 1.0, J, sawc_d, 0, s), s);
-      conj_copy(slice.p, slice.p, NkNw, s);
-      IncProductLoad<R> p0{};
-      p0.m = md;
-      p0.add(grid(F0r, a13, b13), grid(F0d, a13, b13), grid(F0r, a42, b42), grid(F0d, a42, b42), (R)w, 1);
-      p4->exec_fused(p0.template fixed<1>(), gather_sf(slice.p, 1.0, nullptr, nullptr, 1, s), work.p, tmp.p, +1, invN,
-                     s, true);
-      lincomb(dst, base, 1.0, slice.p, 1.0, NkNw, s);
-      continue;
-    }
-    if (self) {
-      // the reference conjugates a self-partner pair in place after the
-      // accumulation (fchi.f90:610): the stored value is conj(conv[G]), so the
-      // increment is conjugated before it is added
-      if (!mesh.complete) GMOD_HIP(hipMemsetAsync(slice.p, 0, NkNw * sizeof(zd), s));
-      product_pass(pl, gather_sf(slice.p, w, nullptr, nullptr, 0, s), s);
-      conj_copy(slice.p, slice.p, NkNw, s);
-      lincomb(dst, base, 1.0, slice.p, 1.0, NkNw, s);
-      continue;
-    }
-    GatherStore<R> gst = gather_sf(dst, tail ? 1.0 : w, J, tail ? sawc_d : nullptr, 0, s);
-    gst.base = base;
-    // the partner copy written by the gather (a complete mesh: every slot of
-    // the slice is written)
-    const bool fuse_pr = pr[0] >= 0 && mesh.complete;
-    if (fuse_pr) gst.pdst = chi + NkNw * (pr[0] + (long)Nchi * pr[1]);
-    product_pass(pl, gst, s);
-    if (pr[0] >= 0 && !fuse_pr) conj_copy(chi + NkNw * (pr[0] + (long)Nchi * pr[1]), dst, NkNw, s);
-  }
+  if (!fuse) partner_copies(chi, pairs_other.gat.d.p, pairs_other.n, NkNw, s);
 }
 
 template <typename R>
@@ -900,7 +925,7 @@ void ConvEngine<R>::sigma_increment(zd* sig, const zd* sig_base, const zd* V, co
                                     hipStream_t s, bool dv_ready) {
   const int No = op.No, Nchi = op.Nchi;
   const long NkNw = mesh.Nk * (long)mesh.Nw;
-  if (acc.n != (size_t)N) acc.alloc(N);
+  if (acc.n < (size_t)N) acc.alloc(N);
   const MeshDev md = mesh_dev(mesh);
   const unsigned S = (unsigned)mesh.Nkall;
   const R invN = (R)(1.0 / (double)p4->transformed_points());
@@ -914,13 +939,25 @@ void ConvEngine<R>::sigma_increment(zd* sig, const zd* sig_base, const zd* V, co
     diff_to_f32(dvbuf.p, V, Vref, nC, s);
   }
   // the inverse transform of output (m1, l1) from grid g, gathered onto sig_base + sig
-  auto gather_grid = [&](cpx<R>* g, int m1, int l1) {
-    const long o = NkNw * (m1 + (long)No * l1);
-    GatherStore<R> gst{sig + o, temp / (double)mesh.Nkall, nullptr, nullptr, 0, md};
-    gst.base = sig_base + o;
-    p4->exec_fused(GridLoad<R>{g, S}, gst, g, tmp.p, +1, invN, s);
+  auto gather_out = [&](int m1, int l1) {
+    GatherBatch<R> gat{sig, NkNw, orb_gat.ptr(),
+                       GatherStore<R>{sig, temp / (double)mesh.Nkall, nullptr, nullptr, 0, md}};
+    gat.proto.base = sig_base;
+    p4->exec_batch(GridLoad<R>{acc.p, S, N}, gat.from(m1 + No * l1), acc.p, 1, tmp.p, +1, invN, s);
   };
-  auto gather_out = [&](int m1, int l1) { gather_grid(acc.p, m1, l1); };
+  // every pair's slices, for the forms that transform pair by pair
+  if (all_heads.h.empty()) {
+    std::vector<int> sl;
+    for (int l = 0; l < Nchi; ++l)
+      for (int m = 0; m < Nchi; ++m) {
+        sl.push_back(m + Nchi * l);
+        sl.push_back(l + Nchi * m);
+      }
+    all_heads.set(std::move(sl), s);
+  }
+  auto pair_load = [&](int m, int l) {
+    return BosonBatch<R, float>{dvbuf.p, NC, all_heads.ptr(), DualPtr<double>{}, md}.from(m + (long)Nchi * l);
+  };
   std::vector<int> ytab;
   if (contract_form()) {
     // contraction form: the full transform of every vertex difference once
@@ -930,12 +967,19 @@ void ConvEngine<R>::sigma_increment(zd* sig, const zd* sig_base, const zd* V, co
     const std::vector<std::array<int, 2>> heads = share_heads(dent);
     const size_t nb = heads.size() * (size_t)N;
     if (DVt.n != nb) DVt.alloc(nb);
-    for (size_t h = 0; h < heads.size(); ++h) {
-      const int m = heads[h][0], l = heads[h][1];
-      const long oml = NC * (m + (long)Nchi * l), olm = NC * (l + (long)Nchi * m);
-      cpx<R>* g = DVt.p + h * N;
-      p4->exec_fused(BosonLoad<R, float>{dvbuf.p, oml, olm, zd(0, 0), md}, GridStore<R>{g, S}, g, tmp.p, -1, (R)1,
-                     s);
+    if (dv_heads.h.empty()) {
+      std::vector<int> sl;
+      for (auto& h : heads) {
+        sl.push_back(h[0] + Nchi * h[1]);
+        sl.push_back(h[1] + Nchi * h[0]);
+      }
+      dv_heads.set(std::move(sl), s);
+    }
+    const BosonBatch<R, float> bb{dvbuf.p, NC, dv_heads.ptr(), DualPtr<double>{}, md};
+    const int n = (int)heads.size(), step = p4->batch_items(n);
+    for (int i0 = 0; i0 < n; i0 += step) {
+      cpx<R>* g = DVt.p + (long)i0 * N;
+      p4->exec_batch(bb.from(i0), GridStore<R>{g, S, N}, g, std::min(step, n - i0), tmp.p, -1, (R)1, s);
     }
     {
       std::vector<long> hoffs;
@@ -964,7 +1008,10 @@ void ConvEngine<R>::sigma_increment(zd* sig, const zd* sig_base, const zd* V, co
                             mesh.rev.p, s);
     }
     GMOD_HIP(hipStreamSynchronize(s));  // ct is released at return
-    for (int o = 0; o < NAB; ++o) gather_grid(ysum.p + (size_t)o * N, o % No, o / No);
+    GatherBatch<R> gat{sig, NkNw, orb_gat.ptr(),
+                       GatherStore<R>{sig, temp / (double)mesh.Nkall, nullptr, nullptr, 0, md}};
+    gat.proto.base = sig_base;
+    p4->exec_batch(GridLoad<R>{ysum.p, S, N}, gat, ysum.p, NAB, tmp.p, +1, invN, s);
     return;
   }
   if (fv_shared) throw Error("sigma_increment: the reference vertex transforms are stored in the contraction form");
@@ -982,11 +1029,10 @@ void ConvEngine<R>::sigma_increment(zd* sig, const zd* sig_base, const zd* V, co
         for (int l = 0; l < Nchi; ++l)
           for (int m = 0; m < Nchi; ++m) {
             if (op.ol[m][0] != m1 || op.ol[l][0] != l1) continue;
-            const long oml = NC * (m + (long)Nchi * l), olm = NC * (l + (long)Nchi * m);
             const int a = op.ol[m][1], b = op.ol[l][1];
             SigmaIncStore<R> st{acc.p, grid(Fr, a, b), grid(Fd, a, b), FVr.p + (size_t)(m + Nchi * l) * N,
                                 first ? 1 : 0, S};
-            p4->exec_fused(BosonLoad<R, float>{dvbuf.p, oml, olm, zd(0, 0), md}, st, work.p, tmp.p, -1, (R)1, s);
+            p4->exec_fused(pair_load(m, l), st, work.p, tmp.p, -1, (R)1, s);
             first = false;
           }
         if (!first) gather_out(m1, l1);
@@ -996,32 +1042,35 @@ void ConvEngine<R>::sigma_increment(zd* sig, const zd* sig_base, const zd* V, co
   // transposed outputs share the head passes of their sources (the vertex
   // differences' static slot is zero, so the conjugate-reversal relation
   // holds, with the slot-0 correction)
-  const SigmaPlan P = plan_sigma(p4->accum_last_is_t(-1) && p4->reversal_ok());
+  const std::vector<SigmaGroup> P = plan_sigma(p4->accum_last_is_t(-1) && p4->reversal_ok(), 1, 1 << 20);
   accum_tab_h.clear();
   std::vector<int> smap;
-  for (size_t i = 0; i < P.outs.size(); ++i)
-    for (auto& e : P.src[i]) {
-      const int m = e[0], l = e[1], a = op.ol[m][1], b = op.ol[l][1];
-      if (grouped) {
-        accum_tab_h.push_back(ysum.p + (size_t)No * No * N + (size_t)(a + No * b) * N);  // Gn_ab
-      } else {
-        accum_tab_h.push_back(grid(Fr, a, b));
-        accum_tab_h.push_back(grid(Fd, a, b));
-        accum_tab_h.push_back(FVr.p + (size_t)(m + Nchi * l) * N);
+  std::vector<long> hoffs;
+  size_t nmax = 0;
+  for (auto& g : P) {
+    for (auto& sl : g.src)
+      for (auto& e : sl) {
+        const int m = e[0], l = e[1], a = op.ol[m][1], b = op.ol[l][1];
+        if (grouped) {
+          accum_tab_h.push_back(ysum.p + (size_t)No * No * N + (size_t)(a + No * b) * N);  // Gn_ab
+        } else {
+          accum_tab_h.push_back(grid(Fr, a, b));
+          accum_tab_h.push_back(grid(Fd, a, b));
+          accum_tab_h.push_back(FVr.p + (size_t)(m + Nchi * l) * N);
+        }
+        smap.push_back(e[2]);
       }
-      smap.push_back(e[2]);
-    }
-  if (srcs.n != (size_t)P.nmax * N) srcs.alloc((size_t)P.nmax * N);
+    for (auto& h : g.heads) head_offsets(hoffs, h[0], h[1]);
+    nmax = std::max(nmax, g.heads.size());
+  }
+  if (srcs.n < nmax * N) srcs.alloc(nmax * N);
   accum_tab.alloc(accum_tab_h.size());
   accum_tab.upload(accum_tab_h.data(), accum_tab_h.size(), s);
   srcmap_d.alloc(smap.size());
   srcmap_d.upload(smap.data(), smap.size(), s);
-  std::vector<long> hoffs;
-  for (auto& hs : P.heads)
-    for (auto& h : hs) head_offsets(hoffs, h[0], h[1]);
   if (dh_offs.n < hoffs.size()) dh_offs.alloc(hoffs.size());
   if (!hoffs.empty()) dh_offs.upload(hoffs.data(), hoffs.size(), s);
-  if (dhD.n < (size_t)P.nmax * mesh.Nkall) dhD.alloc((size_t)P.nmax * mesh.Nkall);
+  if (dhD.n < nmax * mesh.Nkall) dhD.alloc(nmax * mesh.Nkall);
   if (grouped) {
     if (ytab_d.n != ytab.size()) ytab_d.alloc(ytab.size());
     ytab_d.upload(ytab.data(), ytab.size(), s);
@@ -1033,30 +1082,24 @@ void ConvEngine<R>::sigma_increment(zd* sig, const zd* sig_base, const zd* V, co
     sigma_ref_contract<R>(ysum.p, ysum.p + (size_t)No * No * N, Fr.p, Fd.p, FVr.p, ytab_d.p, No * No, No, N, s);
   }
   long off = 0, hoff = 0;
-  for (size_t i = 0; i < P.outs.size(); ++i) {
-    for (auto& h : P.heads[i]) {
-      const int m = h[0], l = h[1];
-      const long oml = NC * (m + (long)Nchi * l), olm = NC * (l + (long)Nchi * m);
-      p4->exec_head(BosonLoad<R, float>{dvbuf.p, oml, olm, zd(0, 0), md}, srcs.p + (long)h[2] * N, tmp.p, -1, s);
+  for (auto& g : P) {
+    for (size_t h = 0; h < g.heads.size(); ++h)
+      p4->exec_head(pair_load(g.heads[h][0], g.heads[h][1]), srcs.p + (long)h * N, 1, tmp.p, -1, s);
+    slot0_corr(dhD.p, (const cpx<float>*)dvbuf.p, dh_offs.p + 2 * hoff, (int)g.heads.size(), s);
+    hoff += (long)g.heads.size();
+    for (size_t i = 0; i < g.outs.size(); ++i) {
+      const int nsrc = (int)g.src[i].size(), o = g.outs[i];
+      if (nsrc == 0) continue;
+      if (grouped) {
+        p4->exec_accum_last(srcs.p, N, nsrc, SigmaIncAccumG<R>{accum_tab.p + off, ysum.p + (size_t)o * N, acc.p, S}, -1,
+                            (R)1, s, srcmap_d.p + off, dhD.p);
+      } else {
+        p4->exec_accum_last(srcs.p, N, nsrc, SigmaIncAccum<R>{accum_tab.p + 3 * off, acc.p, S}, -1, (R)1, s,
+                            srcmap_d.p + off, dhD.p);
+      }
+      off += nsrc;
+      gather_out(o % No, o / No);
     }
-    // the heads of one output take consecutive slots
-    if (!P.heads[i].empty())
-      slot0_corr(dhD.p + (size_t)P.heads[i][0][2] * mesh.Nkall, (const cpx<float>*)dvbuf.p, dh_offs.p + 2 * hoff,
-                 (int)P.heads[i].size(), s);
-    hoff += (long)P.heads[i].size();
-    const int nsrc = (int)P.src[i].size();
-    const int m1 = P.outs[i] % No, l1 = P.outs[i] / No;
-    if (nsrc == 0) continue;
-    if (grouped) {
-      const cpx<R>* Y = ysum.p + (size_t)P.outs[i] * N;
-      p4->exec_accum_last(srcs.p, N, nsrc, SigmaIncAccumG<R>{accum_tab.p + off, Y, acc.p, S}, -1, (R)1, s,
-                          srcmap_d.p + off, dhD.p);
-    } else {
-      p4->exec_accum_last(srcs.p, N, nsrc, SigmaIncAccum<R>{accum_tab.p + 3 * off, acc.p, S}, -1, (R)1, s,
-                          srcmap_d.p + off, dhD.p);
-    }
-    off += nsrc;
-    gather_out(m1, l1);
   }
 }
 

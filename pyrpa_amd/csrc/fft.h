@@ -23,6 +23,8 @@
 // the last backward pass works on lines of one fixed t and skips the slots a
 // gather does not keep.
 #pragma once
+#include <algorithm>
+
 #include "fftbox.h"
 #include "gmod_common.h"
 
@@ -58,6 +60,9 @@ constexpr int FFT_MAX_LINES = 512;
 template <typename R> struct GridLoad {
   const cpx<R>* p;
   unsigned S;
+  long stride = 0;  // of a batch: item i is the grid p + i stride
+  using Item = GridLoad;
+  __host__ __device__ Item at(unsigned i) const { return GridLoad{p + (long)i * stride, S, 0}; }
   // S, t < 2^24 and S t < 2^31 (checked by the plan): a 24-bit multiply
   __device__ cpx<R> operator()(unsigned sp, unsigned t) const { return p[sp + __umul24(S, t)]; }
   __host__ double algo_bytes(double N) const { return N * sizeof(cpx<R>); }
@@ -65,6 +70,9 @@ template <typename R> struct GridLoad {
 template <typename R> struct GridStore {
   cpx<R>* p;
   unsigned S;
+  long stride = 0;
+  using Item = GridStore;
+  __host__ __device__ Item at(unsigned i) const { return GridStore{p + (long)i * stride, S, 0}; }
   struct Pre {};
   __device__ Pre prep(unsigned, unsigned) const { return Pre{}; }
   __device__ void commit(unsigned sp, unsigned t, const Pre&, cpx<R> v) const { p[sp + __umul24(S, t)] = v; }
@@ -217,6 +225,10 @@ class FFTPlan {
   void exec(cpx<R>* buf, cpx<R>* tmp, int sign, R scale, hipStream_t s) const {
     exec_fused(GridLoad<R>{buf, S_}, GridStore<R>{buf, S_}, buf, tmp, sign, scale, s);
   }
+  // n consecutive grids
+  void exec_many(cpx<R>* buf, int n, cpx<R>* tmp, int sign, R scale, hipStream_t s) const {
+    exec_batch(GridLoad<R>{buf, S_, size()}, GridStore<R>{buf, S_, size()}, buf, n, tmp, sign, scale, s);
+  }
   // First pass reads through `ld`, last pass writes through `st`; buf/tmp hold
   // the intermediate passes.
   // spatial_first (box plans): run the passes in the forward order
@@ -225,7 +237,20 @@ class FFTPlan {
   // segments that straddle cache lines.
   template <class LD, class ST>
   void exec_fused(LD ld, ST st, cpx<R>* buf, cpx<R>* tmp, int sign, R scale, hipStream_t s,
+                  bool spatial_first = false) const {
+    exec_batch(ld, st, buf, 1, tmp, sign, scale, s, spatial_first);
+  }
+  // n transforms, item i through ld.at(i) and st.at(i) with intermediates in
+  // buf + i size(); tmp (one grid) is used item by item where a plan needs a
+  // second buffer.  One launch per pass: a transform of a small or middling
+  // grid alone has too few boxes for the CUs.
+  template <class LD, class ST>
+  void exec_batch(LD ld, ST st, cpx<R>* buf, int n, cpx<R>* tmp, int sign, R scale, hipStream_t s,
                   bool spatial_first = false) const;
+  // Items to put in one batch of at most n: enough boxes for several rounds
+  // over the CUs, and more while the intermediates (one grid per item) stay
+  // within the last-level cache
+  int batch_items(int n) const;
   // Accumulating form (box_accum_kernel): exec_head runs every pass but the
   // last for one source (ld -> out; tmp as intermediate); exec_accum_last runs
   // the last pass of nsrc such sources (src + c stride) into the accumulator
@@ -241,14 +266,19 @@ class FFTPlan {
     const BoxArgs& a = bp.back();
     return a.nrad[0] == 0 && a.nrad[1] == 0 && a.nrad[2] == 0 && a.nrad[3] > 0;
   }
+  // (n sources, item i of ld into out + i size())
   template <class LD>
-  void exec_head(LD ld, cpx<R>* out, cpx<R>* tmp, int sign, hipStream_t s) const;
-  // srcmap (device, nsrc entries, optional): source c is buffer srcmap[c] >> 1,
+  void exec_head(LD ld, cpx<R>* out, int n, cpx<R>* tmp, int sign, hipStream_t s) const;
+  // srcmap (device, optional): source c is buffer srcmap[c] >> 1,
   // read conjugated at (-r, -t) when srcmap[c] & 1, plus at t = 0 the
-  // correction dhat[(srcmap[c] >> 1) S + sp] (S spatial points per buffer)
+  // correction dhat[(srcmap[c] >> 1) S + sp] (S spatial points per buffer).
+  // nout outputs: output o sums the sources off[o] .. off[o + 1] - 1 of the
+  // maps (off: device, nout + 1 entries; ntot sources in all); one output of
+  // nsrc sources without off
   template <class AC>
   void exec_accum_last(const cpx<R>* src, long stride, int nsrc, AC ac, int sign, R scale, hipStream_t s,
-                       const int* srcmap = nullptr, const cpx<R>* dhat = nullptr) const;
+                       const int* srcmap = nullptr, const cpx<R>* dhat = nullptr, const int* off = nullptr,
+                       int nout = 1) const;
   // the conjugated reversed reads of a source map are available (grid range)
   bool reversal_ok() const { return sprev_ok(dims_[0], dims_[1], dims_[2]); }
   // Boxes of the forward list's last pass (the last pass of a sign -1 or a
@@ -256,18 +286,24 @@ class FFTPlan {
   // kept_sp[sp] >= 0 needs: per box index (after box_remap) 1 if the box
   // holds such a point.  Empty unless that pass's boxes span the t axis and
   // hold few spatial points each; *frac receives the share of live boxes.
-  std::vector<unsigned char> fwd_last_live(const std::vector<int>& kept_sp, double* frac) const;
+  // (small: of the small boxes, which number differently)
+  std::vector<unsigned char> fwd_last_live(const std::vector<int>& kept_sp, double* frac, bool small) const;
   long size() const { return (long)dims_[0] * dims_[1] * dims_[2] * dims_[3]; }
   unsigned spatial() const { return S_; }
   long transformed_points() const;
   int num_passes() const { return box_.ok ? (int)box_.fwd.size() : (int)fwd_.size(); }
   bool uses_box() const { return box_.ok; }
+  // boxes of the first pass (the work-groups a single transform gives)
+  long boxes() const { return box_.ok && !box_.fwd.empty() ? box_.fwd[0].blocks() : 0; }
 
  private:
   template <class LD, class ST>
   void launch(const FFTPassDesc& p, LD ld, ST st, const cpx<R>* tw, R sc, hipStream_t s) const;
   template <class LD, class ST>
-  void launch_box(int sg, int i, LD ld, ST st, const cpx<R>* tw, R sc, hipStream_t s) const;
+  void launch_box(int sg, int i, LD ld, ST st, int n, int sign, R sc, hipStream_t s) const;
+  // pass i runs with the small boxes: the launch would leave CUs idle, or
+  // the pass is not tiled (two work-groups then share a CU)
+  bool small_pass(int sg, int i, long n) const;
   int dims_[4];
   int mask_;
   unsigned S_ = 1;
@@ -275,9 +311,15 @@ class FFTPlan {
   cpx<R>* tw_[2] = {nullptr, nullptr};  // [0]: sign -1 tables, [1]: sign +1 tables
   long tw_len_ = 0;
   BoxPlan<R> box_;                        // box passes (preferred when box_.ok)
-  cpx<R>* twb_[2] = {nullptr, nullptr};   // their twiddle pools
-  int* tabs_ = nullptr;                   // their tile tables
-  BoxArgs* argsd_[2] = {nullptr, nullptr};  // device copies of box_.fwd / box_.bwd
+  BoxPlan<R> box_s_;                      // the same passes with a quarter of the box
+  struct Tables {                         // device copies of a plan's tables
+    cpx<R>* tw[2] = {nullptr, nullptr};   // twiddle pools
+    int* tabs = nullptr;                  // tile tables
+    BoxArgs* args[2] = {nullptr, nullptr};
+  };
+  Tables dev_, dev_s_;
+  static void upload(const BoxPlan<R>& p, Tables& t);
+  static void free_tables(Tables& t);
   long persist_ = 256;                    // work-groups of a persistent tiled pass
 };
 
@@ -302,6 +344,15 @@ struct ReadFraction {
 template <class F>
 struct ReadFraction<F, std::void_t<decltype(std::declval<const F&>().read_fraction(true))>> {
   static double get(const F& f, bool t_box) { return f.read_fraction(t_box); }
+};
+// A store that holds per-box flags switches to those of the small boxes.
+template <class F, class = void>
+struct SmallBoxes {
+  static void use(F&) {}
+};
+template <class F>
+struct SmallBoxes<F, std::void_t<decltype(std::declval<F&>().use_small_boxes())>> {
+  static void use(F& f) { f.use_small_boxes(); }
 };
 template <typename R, class LD, class ST>
 double pass_bytes(const LD& ld, const ST& st, double N, bool t_box = false) {
@@ -341,46 +392,76 @@ void FFTPlan<R>::launch(const FFTPassDesc& p, LD ld, ST st, const cpx<R>* tw, R 
 
 template <typename R>
 template <class LD, class ST>
-void FFTPlan<R>::launch_box(int sg, int i, LD ld, ST st, const cpx<R>* tw, R sc, hipStream_t s) const {
-  const BoxArgs& a = (sg == 0 ? box_.fwd : box_.bwd)[i];
+void FFTPlan<R>::launch_box(int sg, int i, LD ld, ST st, int n, int sign, R sc, hipStream_t s) const {
+  const bool small = small_pass(sg, i, n);
+  if (small) SmallBoxes<ST>::use(st);
+  const BoxPlan<R>& bp = small ? box_s_ : box_;
+  const Tables& tb = small ? dev_s_ : dev_;
+  const BoxArgs& a = (sg == 0 ? bp.fwd : bp.bwd)[i];
   const size_t shm = (size_t)(a.lds_elems + a.ntwl) * sizeof(cpx<R>);
   static bool attr_done = false;  // one per kernel instantiation: allow the device's whole LDS
   if (!attr_done) {
-    GMOD_HIP(hipFuncSetAttribute((const void*)&box_fft_kernel<R, LD, ST>,
+    GMOD_HIP(hipFuncSetAttribute((const void*)&box_fft_kernel<R, LD, ST, true>,
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)box_.lds_limit));
+    GMOD_HIP(hipFuncSetAttribute((const void*)&box_fft_kernel<R, LD, ST, false>,
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)box_.lds_limit));
     attr_done = true;
   }
-  ProfScope ps(sizeof(R) == 4 ? PROF_FFT32 : PROF_FFT, pass_bytes<R>(ld, st, (double)size(), a.box[3] == dims_[3]),
-               s);
-  // tiled passes: persistent work-groups, one per CU, a multiple of 8
-  long grid = a.blocks();
-  if (a.tiled && grid > persist_) grid = persist_;
+  ProfScope ps(sizeof(R) == 4 ? PROF_FFT32 : PROF_FFT,
+               n * pass_bytes<R>(BatchOf<LD>::at(ld, 0), BatchOf<ST>::at(st, 0), (double)size(), a.box[3] == dims_[3]), s);
   // the pool a pass reads its tables from is the sign's; the power-of-two
   // sub-passes take the sign itself at compile time
-  const int sign = tw == twb_[0] ? -1 : 1;
-  hipLaunchKernelGGL((box_fft_kernel<R, LD, ST>), dim3((unsigned)grid), dim3(BOX_THREADS), shm, s, ld, st,
-                     (const BoxArgs*)(argsd_[sg] + i), tw, (const int*)tabs_, sc, sign);
+  const cpx<R>* tw = tb.tw[sign < 0 ? 0 : 1];
+  const long tot = a.blocks() * (long)n;
+  if (tot >= (1L << 31)) throw Error("FFT batch of 2^31 boxes or more");
+  if (a.tiled)  // persistent work-groups, one per CU, a multiple of 8
+    hipLaunchKernelGGL((box_fft_kernel<R, LD, ST, true>), dim3((unsigned)std::min(tot, persist_)), dim3(BOX_THREADS),
+                       shm, s, ld, st, (const BoxArgs*)(tb.args[sg] + i), tw, (const int*)tb.tabs, sc, sign,
+                       (unsigned)n);
+  else
+    hipLaunchKernelGGL((box_fft_kernel<R, LD, ST, false>), dim3((unsigned)tot), dim3(BOX_THREADS), shm, s, ld, st,
+                       (const BoxArgs*)(tb.args[sg] + i), tw, (const int*)tb.tabs, sc, sign, (unsigned)n);
   GMOD_CHECK_LAUNCH();
 }
 
 template <typename R>
 template <class LD, class ST>
-void FFTPlan<R>::exec_fused(LD ld, ST st, cpx<R>* buf, cpx<R>* tmp, int sign, R scale, hipStream_t s,
+void FFTPlan<R>::exec_batch(LD ld, ST st, cpx<R>* buf, int n, cpx<R>* tmp, int sign, R scale, hipStream_t s,
                             bool spatial_first) const {
+  if (n <= 0) return;
   if (box_.ok) {
-    const cpx<R>* twb = twb_[sign < 0 ? 0 : 1];  // the passes of either list run with the sign's twiddles
-    const int sg = (sign < 0 || spatial_first) ? 0 : 1;
+    const int sg = (sign < 0 || spatial_first) ? 0 : 1;  // the passes of either list run with the sign's twiddles
     const std::vector<BoxArgs>& bp = sg == 0 ? box_.fwd : box_.bwd;
     const int nb = (int)bp.size();
-    auto bo = [&](int which) { return which ? tmp : buf; };
-    for (int i = 0; i < nb; ++i) {
-      const BoxArgs& a = bp[i];
-      const R sc = (i == nb - 1) ? scale : (R)1;
-      const bool first = i == 0, last = i == nb - 1;
-      if (first && last) launch_box(sg, i, ld, st, twb, sc, s);
-      else if (first) launch_box(sg, i, ld, GridStore<R>{bo(a.dst), S_}, twb, sc, s);
-      else if (last) launch_box(sg, i, GridLoad<R>{bo(a.src), S_}, st, twb, sc, s);
-      else launch_box(sg, i, GridLoad<R>{bo(a.src), S_}, GridStore<R>{bo(a.dst), S_}, twb, sc, s);
+    bool in_place = true;
+    for (const BoxArgs& a : bp) in_place = in_place && a.src == 0 && a.dst == 0;
+    // a plan with a scratch buffer runs item by item
+    const int step = in_place ? n : 1;
+    for (int i0 = 0; i0 < n; i0 += step) {
+      cpx<R>* bb = buf + (long)i0 * size();
+      auto bo = [&](int which) { return which ? tmp : bb; };
+      auto run = [&](auto l, auto t, int i, R sc) { launch_box(sg, i, l, t, step, sign, sc, s); };
+      auto pass = [&](auto l, auto t) {
+        for (int i = 0; i < nb; ++i) {
+          const BoxArgs& a = bp[i];
+          const R sc = (i == nb - 1) ? scale : (R)1;
+          const GridLoad<R> gl{bo(a.src), S_, size()};
+          const GridStore<R> gs{bo(a.dst), S_, size()};
+          const bool first = i == 0, last = i == nb - 1;
+          if (first && last) run(l, t, i, sc);
+          else if (first) run(l, gs, i, sc);
+          else if (last) run(gl, t, i, sc);
+          else run(gl, gs, i, sc);
+        }
+      };
+      if (step == n) {
+        pass(ld, st);
+      } else if constexpr (std::is_same<LD, typename BatchOf<LD>::Item>::value &&
+                           std::is_same<ST, typename BatchOf<ST>::Item>::value) {
+        pass(BatchOf<LD>::at(ld, i0), BatchOf<ST>::at(st, i0));
+      } else {
+        throw Error("FFT: the split t axis (GMOD_FFT_TSPLIT) has no batched form");
+      }
     }
     return;
   }
@@ -388,15 +469,20 @@ void FFTPlan<R>::exec_fused(LD ld, ST st, cpx<R>* buf, cpx<R>* tmp, int sign, R 
   const std::vector<FFTPassDesc>& ps = sign < 0 ? fwd_ : bwd_;
   const int np = (int)ps.size();
   if (np == 0) throw Error("FFT with nothing to transform");
-  auto buf_of = [&](int which) { return which ? tmp : buf; };
-  for (int i = 0; i < np; ++i) {
-    const FFTPassDesc& p = ps[i];
-    const R sc = (i == np - 1) ? scale : (R)1;
-    const bool first = i == 0, last = i == np - 1;
-    if (first && last) launch(p, ld, st, tw, sc, s);
-    else if (first) launch(p, ld, GridStore<R>{buf_of(p.dst), S_}, tw, sc, s);
-    else if (last) launch(p, GridLoad<R>{buf_of(p.src), S_}, st, tw, sc, s);
-    else launch(p, GridLoad<R>{buf_of(p.src), S_}, GridStore<R>{buf_of(p.dst), S_}, tw, sc, s);
+  for (int it = 0; it < n; ++it) {
+    const typename BatchOf<LD>::Item li = BatchOf<LD>::at(ld, it);
+    const typename BatchOf<ST>::Item si = BatchOf<ST>::at(st, it);
+    cpx<R>* bb = buf + (long)it * size();
+    auto buf_of = [&](int which) { return which ? tmp : bb; };
+    for (int i = 0; i < np; ++i) {
+      const FFTPassDesc& p = ps[i];
+      const R sc = (i == np - 1) ? scale : (R)1;
+      const bool first = i == 0, last = i == np - 1;
+      if (first && last) launch(p, li, si, tw, sc, s);
+      else if (first) launch(p, li, GridStore<R>{buf_of(p.dst), S_}, tw, sc, s);
+      else if (last) launch(p, GridLoad<R>{buf_of(p.src), S_}, si, tw, sc, s);
+      else launch(p, GridLoad<R>{buf_of(p.src), S_}, GridStore<R>{buf_of(p.dst), S_}, tw, sc, s);
+    }
   }
 }
 
@@ -414,24 +500,23 @@ bool FFTPlan<R>::accum_ok(int sign) const {
 
 template <typename R>
 template <class LD>
-void FFTPlan<R>::exec_head(LD ld, cpx<R>* out, cpx<R>* tmp, int sign, hipStream_t s) const {
+void FFTPlan<R>::exec_head(LD ld, cpx<R>* out, int n, cpx<R>* tmp, int sign, hipStream_t s) const {
   const int sg = sign < 0 ? 0 : 1;
   const int nb = (int)(sg == 0 ? box_.fwd : box_.bwd).size();
-  const cpx<R>* twb = twb_[sg];
-  if (nb == 2) {
-    launch_box(sg, 0, ld, GridStore<R>{out, S_}, twb, (R)1, s);
-  } else {  // 3 passes: ld -> tmp -> out
-    launch_box(sg, 0, ld, GridStore<R>{tmp, S_}, twb, (R)1, s);
-    launch_box(sg, 1, GridLoad<R>{tmp, S_}, GridStore<R>{out, S_}, twb, (R)1, s);
-  }
+  (void)tmp;  // the passes before the last one are in place (accum_ok)
+  const GridStore<R> gs{out, S_, size()};
+  launch_box(sg, 0, ld, gs, n, sign, (R)1, s);
+  if (nb == 3) launch_box(sg, 1, GridLoad<R>{out, S_, size()}, gs, n, sign, (R)1, s);
 }
 
 template <typename R>
 template <class AC>
 void FFTPlan<R>::exec_accum_last(const cpx<R>* src, long stride, int nsrc, AC ac, int sign, R scale,
-                                 hipStream_t s, const int* srcmap, const cpx<R>* dhat) const {
+                                 hipStream_t s, const int* srcmap, const cpx<R>* dhat, const int* off,
+                                 int nout) const {
   if (srcmap && !reversal_ok()) throw Error("exec_accum_last: grid too large for the reversed reads");
   if (srcmap && !dhat) throw Error("exec_accum_last: a source map needs the slot-0 corrections");
+  if (nout > 1 && !off) throw Error("exec_accum_last: several outputs need their source ranges");
   const int sg = sign < 0 ? 0 : 1;
   const std::vector<BoxArgs>& bp = sg == 0 ? box_.fwd : box_.bwd;
   const int i = (int)bp.size() - 1;
@@ -445,12 +530,12 @@ void FFTPlan<R>::exec_accum_last(const cpx<R>* src, long stride, int nsrc, AC ac
   }
   const double N = (double)size();
   ProfScope ps(sizeof(R) == 4 ? PROF_FFT32 : PROF_FFT,
-               nsrc * (N * sizeof(cpx<R>) + ac.src_bytes(N)) + ac.sum_bytes(N), s);
-  long grid = a.blocks();
-  if (grid > persist_) grid = persist_;
-  hipLaunchKernelGGL((box_accum_kernel<R, 16, AC>), dim3((unsigned)grid), dim3(BOX_THREADS), shm, s, src, stride,
-                     nsrc, ac, (const BoxArgs*)(argsd_[sg] + i), twb_[sg], (const int*)tabs_, scale, sg == 0 ? -1 : 1,
-                     srcmap, make_sprev(dims_[0], dims_[1], dims_[2]), dhat);
+               nsrc * (N * sizeof(cpx<R>) + ac.src_bytes(N)) + nout * ac.sum_bytes(N), s);
+  const long tot = a.blocks() * (long)nout;
+  if (tot >= (1L << 31)) throw Error("FFT batch of 2^31 boxes or more");
+  hipLaunchKernelGGL((box_accum_kernel<R, 16, AC>), dim3((unsigned)std::min(tot, persist_)), dim3(BOX_THREADS), shm, s,
+                     src, stride, nsrc, ac, (const BoxArgs*)(dev_.args[sg] + i), dev_.tw[sg], (const int*)dev_.tabs,
+                     scale, sg == 0 ? -1 : 1, srcmap, make_sprev(dims_[0], dims_[1], dims_[2]), dhat, off, nout);
   GMOD_CHECK_LAUNCH();
 }
 

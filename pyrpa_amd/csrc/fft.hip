@@ -96,7 +96,7 @@ static void set_tiles(BoxArgs& a, std::vector<int>& tabs, int max_tiles) {
 }
 
 template <typename R>
-void BoxPlan<R>::build(int nx, int ny, int nz, int m, int mask, long budget, size_t lds_bytes) {
+void BoxPlan<R>::build(int nx, int ny, int nz, int m, int mask, long budget, size_t lds_bytes, long small) {
   ok = false;
   fwd.clear();
   bwd.clear();
@@ -260,11 +260,11 @@ void BoxPlan<R>::build(int nx, int ny, int nz, int m, int mask, long budget, siz
       }
     }
   }
-  // boxes are not capped below the LDS budget: halving them so that two
-  // work-groups share a CU measured no faster on the 4-orbital 32x32x16 x
-  // 2048 grid (FP64 unchanged, FP32 13 % slower with the 32 B rows of a
-  // 4-column t box)
-  const long small = budget;
+  // the boxes of a full launch are not capped below the LDS budget: halving
+  // them so that two work-groups share a CU measured no faster on the
+  // 4-orbital 32x32x16 x 2048 grid (FP64 unchanged, FP32 13 % slower with the
+  // 32 B rows of a 4-column t box)
+  if (small <= 0) small = budget;
   std::vector<BoxArgs> spatial;
   for (auto& gdims : groups) {
     int ext[4] = {1, 1, 1, 1};
@@ -274,6 +274,7 @@ void BoxPlan<R>::build(int nx, int ny, int nz, int m, int mask, long budget, siz
     const long cap = std::max(vol, small);
     if (ext[0] == 1) {  // keep rows contiguous: adjacent x columns in the box
       ext[0] = largest_divisor_le(nx, std::min<long>(256 / b, cap / vol));
+      if (ext[0] * b < 64) ext[0] = largest_divisor_le(nx, std::min<long>(256 / b, budget / vol));
       vol *= ext[0];
     }
     ext[3] = largest_divisor_le(m, cap / vol);
@@ -289,6 +290,8 @@ void BoxPlan<R>::build(int nx, int ny, int nz, int m, int mask, long budget, siz
     const long cap = std::max<long>(m, small);
     int ext[4] = {1, 1, 1, m};
     ext[0] = largest_divisor_le(nx, cap / m);
+    // rows under 64 B waste the cache lines they share: the whole budget then
+    if (ext[0] * b < 64) ext[0] = largest_divisor_le(nx, std::max<long>(m, budget) / m);
     if (ext[0] == nx) ext[1] = largest_divisor_le(ny, cap / ((long)m * nx));
     if (ext[0] == nx && ext[1] == ny) ext[2] = largest_divisor_le(nz, cap / ((long)m * nx * ny));
     if (!make_box(ext, {3}, tb)) return;
@@ -488,20 +491,10 @@ FFTPlan<R>::FFTPlan(int nx, int ny, int nz, int m, int axes_mask) {
       if (hipGetDevice(&dev) == hipSuccess &&
           hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && ncu >= 8)
         persist_ = (long)(ncu / 8) * 8;
-      for (int sg = 0; sg < 2; ++sg) {
-        const std::vector<BoxArgs>& v = sg == 0 ? box_.fwd : box_.bwd;
-        GMOD_HIP(hipMalloc(&argsd_[sg], std::max<size_t>(v.size(), 1) * sizeof(BoxArgs)));
-        if (!v.empty()) GMOD_HIP(hipMemcpy(argsd_[sg], v.data(), v.size() * sizeof(BoxArgs), hipMemcpyHostToDevice));
-      }
-      const size_t ntab = box_.tab_host.size();
-      GMOD_HIP(hipMalloc(&tabs_, std::max<size_t>(ntab, 1) * sizeof(int)));
-      if (ntab) GMOD_HIP(hipMemcpy(tabs_, box_.tab_host.data(), ntab * sizeof(int), hipMemcpyHostToDevice));
-      for (int sg = 0; sg < 2; ++sg) {
-        const size_t nt = box_.tw_host[sg].size();
-        GMOD_HIP(hipMalloc(&twb_[sg], std::max<size_t>(nt, 1) * sizeof(cpx<R>)));
-        if (nt)
-          GMOD_HIP(hipMemcpy(twb_[sg], box_.tw_host[sg].data(), nt * sizeof(cpx<R>), hipMemcpyHostToDevice));
-      }
+      upload(box_, dev_);
+      box_s_.build(nx, ny, nz, m, axes_mask, budget, lds, budget / 4);
+      if (box_s_.ok && box_s_.fwd.size() == box_.fwd.size()) upload(box_s_, dev_s_);
+      else box_s_.ok = false;
     }
   }
   // twiddle tables: tw[k] = exp(sign * 2 pi i k / len), computed in double
@@ -534,14 +527,57 @@ FFTPlan<R>::FFTPlan(int nx, int ny, int nz, int m, int axes_mask) {
 }
 
 template <typename R>
+void FFTPlan<R>::upload(const BoxPlan<R>& p, Tables& t) {
+  auto put = [](auto** dst, const auto* src, size_t n) {
+    GMOD_HIP(hipMalloc((void**)dst, std::max<size_t>(n, 1) * sizeof(*src)));
+    if (n) GMOD_HIP(hipMemcpy(*dst, src, n * sizeof(*src), hipMemcpyHostToDevice));
+  };
+  for (int sg = 0; sg < 2; ++sg) {
+    const std::vector<BoxArgs>& v = sg == 0 ? p.fwd : p.bwd;
+    put(&t.args[sg], v.data(), v.size());
+    put(&t.tw[sg], p.tw_host[sg].data(), p.tw_host[sg].size());
+  }
+  put(&t.tabs, p.tab_host.data(), p.tab_host.size());
+}
+
+template <typename R>
+void FFTPlan<R>::free_tables(Tables& t) {
+  for (auto p : t.args)
+    if (p) (void)hipFree(p);
+  for (auto p : t.tw)
+    if (p) (void)hipFree(p);
+  if (t.tabs) (void)hipFree(t.tabs);
+}
+
+template <typename R>
 FFTPlan<R>::~FFTPlan() {
   for (auto p : tw_)
     if (p) (void)hipFree(p);
-  for (auto p : twb_)
-    if (p) (void)hipFree(p);
-  if (tabs_) (void)hipFree(tabs_);
-  for (auto p : argsd_)
-    if (p) (void)hipFree(p);
+  free_tables(dev_);
+  free_tables(dev_s_);
+}
+
+// Quarter-size boxes where whole ones leave CUs idle (1 orbital, 32x32 x 512:
+// 64 boxes, now 256; a plain pass 16.9 -> 13.4 us) and for untiled passes,
+// which need two boxes in a CU's LDS to overlap (27x27x5 x 180: 28 us a grid
+// in a launch of its own, now 22 in a batch of 9); whole boxes elsewhere (see
+// BoxPlan::build: full launches measured slower with smaller boxes).
+template <typename R>
+bool FFTPlan<R>::small_pass(int sg, int i, long n) const {
+  if (!box_s_.ok) return false;
+  const BoxArgs& a = (sg == 0 ? box_.fwd : box_.bwd)[i];
+  const BoxArgs& as = (sg == 0 ? box_s_.fwd : box_s_.bwd)[i];
+  if (as.blocks() == a.blocks()) return false;
+  return !a.tiled || a.blocks() * n < persist_;
+}
+
+template <typename R>
+int FFTPlan<R>::batch_items(int n) const {
+  const long nb = std::max<long>(boxes(), 1), bytes = size() * (long)sizeof(cpx<R>);
+  // four rounds over the CUs (per-axis passes run item by item)
+  const long rounds = box_.ok ? (4 * persist_ + nb - 1) / nb : 1;
+  const long cached = (96L << 20) / bytes, room = std::max<long>(1, (2L << 30) / bytes);
+  return (int)std::max<long>(1, std::min<long>(n, std::min(room, std::max(rounds, cached))));
 }
 
 template <typename R>
@@ -566,11 +602,13 @@ const FFTPlan<R>& fft_plan(int nx, int ny, int nz, int m, int axes_mask) {
 }
 
 template <typename R>
-std::vector<unsigned char> FFTPlan<R>::fwd_last_live(const std::vector<int>& kept_sp, double* frac) const {
+std::vector<unsigned char> FFTPlan<R>::fwd_last_live(const std::vector<int>& kept_sp, double* frac,
+                                                     bool small) const {
   std::vector<unsigned char> live;
   if (frac) *frac = 1.0;
-  if (!box_.ok || box_.fwd.empty() || kept_sp.size() != (size_t)S_) return live;
-  const BoxArgs& a = box_.fwd.back();
+  const BoxPlan<R>& bp = small ? box_s_ : box_;
+  if (!bp.ok || bp.fwd.empty() || kept_sp.size() != (size_t)S_) return live;
+  const BoxArgs& a = bp.fwd.back();
   const long pts = (long)a.box[0] * a.box[1] * a.box[2];
   if (a.box[3] != dims_[3] || pts > 64) return live;
   const long nb = a.blocks();

@@ -296,13 +296,15 @@ __host__ __device__ __forceinline__ void box_load_tiled(cpx<R>* lds, const LD& l
 template <typename R, class LD>
 __host__ __device__ __forceinline__ void box_load(cpx<R>* lds, const LD& ld, const BoxArgs& a, const BoxOrigin& O,
                                                   int tid, int nthr, const int* __restrict__ tabs) {
-  if (a.tiled) {  // one pass on the device (nthr = BOX_THREADS); the host emulation loops over the threads
+#if !defined(__HIP_DEVICE_COMPILE__)
+  if (a.tiled) {  // the host emulation loops over the threads; the device runs tiled passes in box_persistent
     for (int t = tid; t < BOX_THREADS; t += nthr) box_load_tiled<R>(lds, ld, a, O, (unsigned)t, tabs);
     return;
   }
-  // U loads in flight per thread before the first LDS store: one work-group
-  // per CU has to keep ~64 KB of HBM reads outstanding
-  constexpr int U = sizeof(R) == 4 ? 16 : 8;
+#endif
+  // U loads in flight per thread before the first LDS store (two work-groups
+  // share the CU's registers)
+  constexpr int U = sizeof(R) == 4 ? 8 : 4;
   const int ex = a.box[0], ey = a.box[1], ez = a.box[2];
   for (int e0 = tid; e0 < a.elems; e0 += nthr * U) {
     cpx<R> v[U];
@@ -514,13 +516,15 @@ template <typename R, class ST>
 __host__ __device__ __forceinline__ void box_store(const cpx<R>* lds, const ST& st, const BoxArgs& a,
                                                    const BoxOrigin& O, R scale, const cpx<R>* __restrict__ tw,
                                                    int tid, int nthr, const int* __restrict__ tabs) {
+#if !defined(__HIP_DEVICE_COMPILE__)
   if (a.tiled) {
     for (int t = tid; t < BOX_THREADS; t += nthr) box_store_tiled<R>(lds, st, a, O, scale, (unsigned)t, tabs);
     return;
   }
+#endif
   // batches of U elements: every load a store functor needs (accumulators,
   // operands, gather indices) is issued before the batch's first store
-  constexpr int U = 8;
+  constexpr int U = 2;
   const int ex = a.box[0], ey = a.box[1], ez = a.box[2];
   for (int e0 = tid; e0 < a.elems; e0 += nthr * U) {
     unsigned spv[U], tv[U];
@@ -581,6 +585,21 @@ __host__ __device__ __forceinline__ void box_twiddles_to_lds(cpx<R>* lds, const 
   }
 }
 
+// A load or store functor of a batch of transforms names the functor of one
+// item (Item) and forms it with at(item); the grids and tables it needs are
+// found by the item's index, so the batch is one launch.  A functor without
+// Item is its own only item.
+template <class F, class = void>
+struct BatchOf {
+  using Item = F;
+  __host__ __device__ static const F& at(const F& f, unsigned) { return f; }
+};
+template <class F>
+struct BatchOf<F, std::void_t<typename F::Item>> {
+  using Item = typename F::Item;
+  __host__ __device__ static Item at(const F& f, unsigned i) { return f.at(i); }
+};
+
 // A store may also drop whole boxes by their index (skip_box(lb), lb the
 // box index after box_remap): the gather of a pass whose boxes span the
 // whole t axis keeps only the boxes that hold a kept spatial point.
@@ -609,11 +628,14 @@ __host__ __device__ __forceinline__ bool box_skipped(const ST& st, const BoxArgs
 // twiddles from global memory has run, so its HBM reads overlap the
 // remaining sub-passes and the store of the current box.  gridDim.x is a
 // multiple of 8, so a work-group keeps its XCD and box_remap's grouping holds.
+// A launch runs the boxes of nitem transforms: box b of the launch is box
+// b mod nb of item b / nb.
 template <class ST>
-__device__ __forceinline__ unsigned box_next_live(const ST& st, const BoxArgs& a, unsigned b, unsigned nb) {
-  while (b < nb) {
-    const unsigned lb = box_remap(b, nb, a.xcd_group);
-    if (!box_skipped(st, a, lb, box_origin(a, lb))) break;
+__device__ __forceinline__ unsigned box_next_live(const ST& st, const BoxArgs& a, unsigned b, unsigned nb,
+                                                  unsigned tot) {
+  while (b < tot) {
+    const unsigned it = b / nb, lb = box_remap(b - it * nb, nb, a.xcd_group);
+    if (!box_skipped(BatchOf<ST>::at(st, it), a, lb, box_origin(a, lb))) break;
     b += gridDim.x;
   }
   return b;
@@ -680,9 +702,10 @@ __device__ __forceinline__ void box_fetch(cpx<R> (&v)[TM], const LD& ld, const B
 template <typename R, class LD, class ST>
 __device__ __forceinline__ void box_persistent(cpx<R>* lds, const LD& ld, const ST& st, const BoxArgs& a,
                                                const cpx<R>* __restrict__ tw, const int* __restrict__ tabs, R scale,
-                                               int tid, int sign) {
+                                               int tid, int sign, unsigned nitem) {
   constexpr int TM = BOX_TILE_REGS<R>;
-  const unsigned nb = (unsigned)a.blocks();
+  using LI = typename BatchOf<LD>::Item;
+  const unsigned nb = (unsigned)a.blocks(), tot = nb * nitem;
   unsigned c[4];
   box_tile_coord(a, (unsigned)tid, c);
   const unsigned csp = c[0] + mul24(a.Nx, c[1]) + mul24(a.Nx * a.Ny, c[2]);
@@ -693,26 +716,32 @@ __device__ __forceinline__ void box_persistent(cpx<R>* lds, const LD& ld, const 
   const int* tt = tsp + a.ntiles;
   const int* tld = tt + a.ntiles;
   cpx<R> v[TM];
+  auto fetch = [&](unsigned n) {
+    const unsigned it = n / nb;
+    box_fetch<R, TM>(v, BatchOf<LD>::at(ld, it), a, n - it * nb, nb, csp, ct, tsp, tt);
+  };
   box_twiddles_to_lds<R>(lds, a, tw, tid, BOX_THREADS);  // ordered before use by the loop's first barrier
-  unsigned b = box_next_live(st, a, blockIdx.x, nb);
-  if (b < nb) box_fetch<R, TM>(v, ld, a, b, nb, csp, ct, tsp, tt);
-  while (b < nb) {
+  unsigned b = box_next_live(st, a, blockIdx.x, nb, tot);
+  if (b < tot) fetch(b);
+  while (b < tot) {
+    const unsigned it = b / nb;
+    const BoxOrigin O = box_origin(a, box_remap(b - it * nb, nb, a.xcd_group));
     {
-      const BoxOrigin O = box_origin(a, box_remap(b, nb, a.xcd_group));
+      const LI li = BatchOf<LD>::at(ld, it);
       const unsigned t0 = mul24((unsigned)O.bt, (unsigned)a.tl_mul) + ct;
 #pragma unroll
       for (int j = 0; j < TM; ++j)
-        if (j < a.ntiles) lds[l0 + (unsigned)tld[j]] = LoadRaw<R, LD>::finish(ld, v[j], t0 + (unsigned)tt[j]);
+        if (j < a.ntiles) lds[l0 + (unsigned)tld[j]] = LoadRaw<R, LI>::finish(li, v[j], t0 + (unsigned)tt[j]);
     }
     __syncthreads();
-    const unsigned nxt = box_next_live(st, a, b + gridDim.x, nb);
+    const unsigned nxt = box_next_live(st, a, b + gridDim.x, nb, tot);
     for (int i = 0; i < a.nsub; ++i) {
-      if (i == a.pf_at && nxt < nb) box_fetch<R, TM>(v, ld, a, nxt, nb, csp, ct, tsp, tt);
+      if (i == a.pf_at && nxt < tot) fetch(nxt);
       box_dispatch<R>(lds, a, box_sub_at(a, i), tw, tid, BOX_THREADS, sign);
       __syncthreads();
     }
-    if (a.pf_at >= a.nsub && nxt < nb) box_fetch<R, TM>(v, ld, a, nxt, nb, csp, ct, tsp, tt);
-    box_store_tiled<R>(lds, st, a, box_origin(a, box_remap(b, nb, a.xcd_group)), scale, (unsigned)tid, tabs);
+    if (a.pf_at >= a.nsub && nxt < tot) fetch(nxt);
+    box_store_tiled<R>(lds, BatchOf<ST>::at(st, it), a, O, scale, (unsigned)tid, tabs);
     __syncthreads();  // the LDS box is rewritten by the next iteration
     b = nxt;
   }
@@ -779,18 +808,22 @@ struct AccumSrcLoad {
 // srcmap (optional): source c is buffer srcmap[c] >> 1 of src, conjugated at
 // (-r, -t) when srcmap[c] & 1 (rv: the spatial reversal), with the slot-0
 // correction dhat + (srcmap[c] >> 1) S; else buffer c.
+// nout sums in one launch: output o sums the sources off[o] .. off[o + 1] - 1
+// of srcmap and of ac's operand table into ac's sum grid o (ac.at(o, off[o]));
+// off null: one output of nsrc sources.
 template <typename R, int MAXR, class AC>
 __global__ void __launch_bounds__(BOX_THREADS)
-box_accum_kernel(const cpx<R>* __restrict__ src, long src_stride, int nsrc, AC ac, const BoxArgs* __restrict__ ap,
+box_accum_kernel(const cpx<R>* __restrict__ src, long src_stride, int nsrc1, AC acs, const BoxArgs* __restrict__ ap,
                  const cpx<R>* __restrict__ tw, const int* __restrict__ tabs, R scale, int sign,
-                 const int* __restrict__ srcmap, SpRev rv, const cpx<R>* __restrict__ dhat) {
+                 const int* __restrict__ srcmap1, SpRev rv, const cpx<R>* __restrict__ dhat,
+                 const int* __restrict__ off, int nout) {
   extern __shared__ unsigned char smem_raw[];
   cpx<R>* lds = reinterpret_cast<cpx<R>*>(smem_raw);
   const BoxArgs& a = *ap;
   constexpr int TM = BOX_TILE_REGS<R>;
   constexpr int U = 8;
   const int tid = threadIdx.x;
-  const unsigned nb = (unsigned)a.blocks();
+  const unsigned nb = (unsigned)a.blocks(), tot = nb * (unsigned)nout;
   unsigned c4[4];
   box_tile_coord(a, (unsigned)tid, c4);
   const unsigned csp = c4[0] + mul24(a.Nx, c4[1]) + mul24(a.Nx * a.Ny, c4[2]);
@@ -812,8 +845,11 @@ box_accum_kernel(const cpx<R>* __restrict__ src, long src_stride, int nsrc, AC a
   constexpr bool PF = sizeof(R) == 4;
   constexpr int TV = PF ? TM : 1;
   cpx<R> v[TV], sum[TM];
-  auto srcld = [&](int cc) {
-    const int e = srcmap ? srcmap[cc] : 2 * cc;
+  // of output o: its first source, its number of sources
+  auto first = [&](unsigned o) { return off ? off[o] : 0; };
+  auto count = [&](unsigned o) { return off ? off[o + 1] - off[o] : nsrc1; };
+  auto srcld = [&](unsigned o, int cc) {
+    const int e = srcmap1 ? srcmap1[first(o) + cc] : 2 * cc;
     return AccumSrcLoad<R>{src + (long)(e >> 1) * src_stride, dhat ? dhat + (long)(e >> 1) * a.S : nullptr, rv,
                            a.S, a.M, e & 1};
   };
@@ -821,18 +857,21 @@ box_accum_kernel(const cpx<R>* __restrict__ src, long src_stride, int nsrc, AC a
   unsigned b = blockIdx.x;
   int c = 0;
   if constexpr (PF) {
-    if (b < nb) box_fetch<R, TM>(v, srcld(0), a, b, nb, csp, ct, tsp, tt);
+    if (b < tot) box_fetch<R, TM>(v, srcld(b / nb, 0), a, b % nb, nb, csp, ct, tsp, tt);
   }
-  while (b < nb) {
+  while (b < tot) {
+    const unsigned o = b / nb, bl = b - o * nb;
+    const int nsrc = count(o);
+    const AC ac = acs.at(o, first(o));
     if constexpr (PF) {
 #pragma unroll
       for (int j = 0; j < TM; ++j)
         if (j < a.ntiles) lds[l0 + (unsigned)tld[j]] = v[j];
     } else {
-      const BoxOrigin O = box_origin(a, box_remap(b, nb, a.xcd_group));
+      const BoxOrigin O = box_origin(a, box_remap(bl, nb, a.xcd_group));
       const unsigned sp0 = box_sp(a, O, 0, 0, 0) + csp;
       const unsigned t0 = mul24((unsigned)O.bt, (unsigned)a.tl_mul) + ct;
-      const AccumSrcLoad<R> sc = srcld(c);
+      const AccumSrcLoad<R> sc = srcld(o, c);
 #pragma unroll
       for (int j0 = 0; j0 < TM; j0 += 8) {
         cpx<R> w[8];
@@ -846,19 +885,19 @@ box_accum_kernel(const cpx<R>* __restrict__ src, long src_stride, int nsrc, AC a
     const bool more = c + 1 < nsrc;
     const unsigned b2 = more ? b : b + gridDim.x;
     const int c2 = more ? c + 1 : 0;
-    const AccumSrcLoad<R> ld2 = srcld(c2);
     for (int i = 0; i < a.nsub; ++i) {
       if constexpr (PF) {
-        if (i == a.pf_at && b2 < nb) box_fetch<R, TM>(v, ld2, a, b2, nb, csp, ct, tsp, tt);
+        if (i == a.pf_at && b2 < tot) box_fetch<R, TM>(v, srcld(b2 / nb, c2), a, b2 % nb, nb, csp, ct, tsp, tt);
       }
       box_dispatch<R, MAXR>(lds, a, box_sub_at(a, i), tw, tid, BOX_THREADS, sign);
       __syncthreads();
     }
     if constexpr (PF) {
-      if (a.pf_at >= a.nsub && b2 < nb) box_fetch<R, TM>(v, ld2, a, b2, nb, csp, ct, tsp, tt);
+      if (a.pf_at >= a.nsub && b2 < tot)
+        box_fetch<R, TM>(v, srcld(b2 / nb, c2), a, b2 % nb, nb, csp, ct, tsp, tt);
     }
     // contributions of source c
-    const BoxOrigin O = box_origin(a, box_remap(b, nb, a.xcd_group));
+    const BoxOrigin O = box_origin(a, box_remap(bl, nb, a.xcd_group));
     const unsigned sp0 = box_sp(a, O, 0, 0, 0) + csp;
     const unsigned t0 = mul24((unsigned)O.bt, (unsigned)a.ts_mul) + mul24(c4[3], (unsigned)a.ts_str);
 #pragma unroll
@@ -887,29 +926,39 @@ box_accum_kernel(const cpx<R>* __restrict__ src, long src_stride, int nsrc, AC a
 // The pass descriptor is read from device memory (the plan's copy) rather
 // than passed by value: run-time indices into a by-value kernel argument
 // make the compiler copy the whole argument to scratch memory.
-template <typename R, class LD, class ST>
-__global__ void __launch_bounds__(BOX_THREADS)
+// Bound by the overlap of a box's load, sub-passes and store, not by bytes.
+// TILED: persistent work-groups, one per CU (the prefetch takes the registers
+// of a second one); else a work-group per box, two per CU (4 waves per SIMD),
+// so that one loads or stores while the other transforms.
+// nitem transforms in one launch: alone, a grid of 16x16x8 x 512 gives 128
+// boxes to 256 CUs (136 bubble products of 4 orbitals: 32 us each, now 21 in
+// batches of 8; their gathers 25 -> 11 us), and 16x16 x 256 eight boxes
+// (spin-orbit bubbles 13.6 -> 1.1 us each).
+template <typename R, class LD, class ST, bool TILED>
+__global__ void __launch_bounds__(BOX_THREADS, TILED ? 2 : 4)
 box_fft_kernel(LD ld, ST st, const BoxArgs* __restrict__ ap, const cpx<R>* __restrict__ tw,
-               const int* __restrict__ tabs, R scale, int sign) {
+               const int* __restrict__ tabs, R scale, int sign, unsigned nitem) {
   extern __shared__ unsigned char smem_raw[];
   cpx<R>* lds = reinterpret_cast<cpx<R>*>(smem_raw);
   const BoxArgs& a = *ap;
-  if (a.tiled) {
-    box_persistent<R>(lds, ld, st, a, tw, tabs, scale, threadIdx.x, sign);
-    return;
-  }
-  const unsigned lb = box_remap(blockIdx.x, gridDim.x, a.xcd_group);
-  const BoxOrigin O = box_origin(a, lb);
-  if (box_skipped(st, a, lb, O)) return;
-  const int tid = threadIdx.x;
-  box_twiddles_to_lds<R>(lds, a, tw, tid, BOX_THREADS);
-  box_load<R>(lds, ld, a, O, tid, BOX_THREADS, tabs);
-  __syncthreads();
-  for (int i = 0; i < a.nsub; ++i) {
-    box_dispatch<R>(lds, a, box_sub_at(a, i), tw, tid, BOX_THREADS, sign);
+  if constexpr (TILED) {
+    box_persistent<R>(lds, ld, st, a, tw, tabs, scale, threadIdx.x, sign, nitem);
+  } else {
+    const unsigned nb = (unsigned)a.blocks(), it = blockIdx.x / nb;
+    const unsigned lb = box_remap(blockIdx.x - it * nb, nb, a.xcd_group);
+    const BoxOrigin O = box_origin(a, lb);
+    const typename BatchOf<ST>::Item si = BatchOf<ST>::at(st, it);
+    if (box_skipped(si, a, lb, O)) return;
+    const int tid = threadIdx.x;
+    box_twiddles_to_lds<R>(lds, a, tw, tid, BOX_THREADS);
+    box_load<R>(lds, BatchOf<LD>::at(ld, it), a, O, tid, BOX_THREADS, tabs);
     __syncthreads();
+    for (int i = 0; i < a.nsub; ++i) {
+      box_dispatch<R>(lds, a, box_sub_at(a, i), tw, tid, BOX_THREADS, sign);
+      __syncthreads();
+    }
+    box_store<R>(lds, si, a, O, scale, tw, tid, BOX_THREADS, tabs);
   }
-  box_store<R>(lds, st, a, O, scale, tw, tid, BOX_THREADS, tabs);
 }
 
 // Host-side plan of box passes (built without a device).
@@ -923,7 +972,10 @@ struct BoxPlan {
   size_t lds_limit = 0;      // the device's per-work-group LDS limit the plan was built for
   // plan the transform of the axes in `mask` of an (nx,ny,nz,m) grid with
   // boxes of at most `budget` elements and `lds_bytes` of LDS
-  void build(int nx, int ny, int nz, int m, int mask, long budget, size_t lds_bytes);
+  // (small: fill a box with untransformed points up to this many elements;
+  // 0: the budget).  The passes' dimensions, radices and order, and so the
+  // results, do not depend on it.
+  void build(int nx, int ny, int nz, int m, int mask, long budget, size_t lds_bytes, long small = 0);
 };
 
 }  // namespace gmod

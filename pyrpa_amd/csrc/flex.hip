@@ -755,8 +755,7 @@ static double eliash_driver(const EliashIn& A, zd* delta_out) {
   const long rest = Nw * No * No;
   auto apply = [&](zd* w_out, const zd* v_in) {
     anomalous_f(Fk.p, G.p, v_in, Nk, (int)Nw, No, s);
-    eng.gap(w_out, Fk.p, A.prt, singlet, s);
-    scale(w_out, nS, weight, s);
+    eng.gap(w_out, Fk.p, A.prt, singlet, weight, s);
   };
   auto norm = [&](const zd* f) { return std::sqrt(2.0 * dot_w(f, f, mesh.kw.p, Nk, rest, s).re); };
   auto inner = [&](const zd* u, const zd* v) { return dot_w(u, v, mesh.kw.p, Nk, rest, s) * 2.0; };
@@ -1026,8 +1025,7 @@ static void nonlin_eliash_driver(const NonlinIn& A, zd* delta_io, zd* sigma_out,
   for (long it = 1; it <= A.itemax; ++it) {
     it_done = it;
     if (verbose) printf("iter=%5ld\n", it);
-    eng.gap(nd.p, F.p, A.prt, singlet, s);
-    scale(nd.p, nS, weight, s);
+    eng.gap(nd.p, F.p, A.prt, singlet, weight, s);
     const double diff = max_abs_diff(nd.p, D.p, (long)nS, s);
     const double dnorm = max_abs_diff(D.p, nullptr, (long)nS, s) + 1.0e-30;
     const double new_max = max_abs_diff(nd.p, nullptr, (long)nS, s);

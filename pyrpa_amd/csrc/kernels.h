@@ -52,6 +52,35 @@ struct MeshDev {
 // counts N b; a read of irreducible slices counts their Nk Nw elements.
 MeshDev mesh_dev(const Mesh& m);
 
+// A table that kernels read in device memory and launch code on the host
+template <typename T>
+struct DualPtr {
+  const T* d = nullptr;
+  const T* h = nullptr;
+  __host__ __device__ T operator[](long i) const {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return d[i];
+#else
+    return h[i];
+#endif
+  }
+  __host__ __device__ explicit operator bool() const { return d != nullptr; }
+  DualPtr operator+(long i) const { return d ? DualPtr{d + i, h + i} : DualPtr{}; }
+};
+template <typename T>
+struct DualTab {
+  std::vector<T> h;
+  DBuf<T> d;
+  // h stays as the copy's source; waits only when it replaces an earlier one
+  void set(std::vector<T> v, hipStream_t s) {
+    if (!h.empty()) GMOD_HIP(hipStreamSynchronize(s));
+    h = std::move(v);
+    d.alloc(h.size());
+    if (!h.empty()) d.upload(h.data(), h.size(), s);
+  }
+  DualPtr<T> ptr() const { return DualPtr<T>{d.p, h.data()}; }
+};
+
 // G_ab on the full grid (fchi.f90:563-583, fself.f90:226-236):
 //   slot t <  Nw : w_t ;  k direct -> G(k)_ab, k = -k_irr -> G(k_irr)_ba
 //   slot t >= Nw : -w_j with j = M-1-t ; direct -> conj G_ba, reversed -> conj G_ab
@@ -79,6 +108,16 @@ struct GreenLoad {
   __device__ cpx<R> value(Key kf, unsigned sp, unsigned t) const { return finish(raw(kf, sp, t), t); }
   __device__ cpx<R> operator()(unsigned sp, unsigned t) const { return value(key(sp), sp, t); }
   __host__ double algo_bytes(double) const { return 2.0 * m.irr_elems() * sizeof(cpx<S>); }
+};
+
+// every G_ab: item a + No b
+template <typename R, typename S = double>
+struct GreenBatch {
+  const cpx<S>* G;
+  int No;
+  MeshDev m;
+  using Item = GreenLoad<R, S>;
+  __host__ __device__ Item at(unsigned i) const { return Item{G, (int)i % No, (int)i / No, No, m}; }
 };
 
 // G_ab of a spinful basis on the full grid (fchi0withsoc.f90:57-75,
@@ -112,6 +151,20 @@ struct SocGreenLoad {
   __host__ double algo_bytes(double) const { return 2.0 * m.irr_elems() * sizeof(zd); }
 };
 
+template <typename R>
+struct SocGreenBatch {
+  const zd* G;
+  int No;
+  DualPtr<int> inv;
+  DualPtr<double> spin;
+  MeshDev m;
+  using Item = SocGreenLoad<R>;
+  __host__ __device__ Item at(unsigned i) const {
+    const int a = (int)i % No, b = (int)i / No;
+    return Item{G, a, b, inv[a], inv[b], No, spin[a] * spin[b], m};
+  }
+};
+
 // bosonic V_(m,l) (fself.f90:203-224, feliash.f90:543-564): slot 0 = nu_0,
 // slot Nw = the nu -> infinity value `stat`, slots t and M-t = +-nu_t
 template <typename R, typename S = double>
@@ -141,6 +194,21 @@ struct BosonLoad {
   __device__ cpx<R> value(Key kf, unsigned sp, unsigned t) const { return finish(raw(kf, sp, t), t); }
   __device__ cpx<R> operator()(unsigned sp, unsigned t) const { return value(key(sp), sp, t); }
   __host__ double algo_bytes(double) const { return 2.0 * m.irr_elems() * sizeof(cpx<S>); }  // V_ml, V_lm slices
+};
+
+// pairs (m, l) by their slices m + Nchi l and l + Nchi m (tab[2 i], tab[2 i + 1]) and static values
+template <typename R, typename S = double>
+struct BosonBatch {
+  const cpx<S>* V;
+  long NC;
+  DualPtr<int> tab;
+  DualPtr<double> stat;  // none: zero
+  MeshDev m;
+  using Item = BosonLoad<R, S>;
+  __host__ __device__ Item at(unsigned i) const {
+    return Item{V, NC * tab[2 * (long)i], NC * tab[2 * (long)i + 1], zd(stat ? stat[i] : 0.0, 0), m};
+  }
+  BosonBatch from(long i) const { return BosonBatch{V, NC, tab + 2 * i, stat + i, m}; }
 };
 
 // The nu_0 mismatch of a transposed pair of bosonic grids: for the stored
@@ -238,17 +306,31 @@ struct AnomLoad {
   long oab, oba;
   double pp, sgn, dprt;
   MeshDev m;
-  __device__ cpx<R> operator()(unsigned sp, unsigned tu) const {
+  using Key = int;  // packed 2 k + flag (Mesh::kf_s)
+  __device__ Key key(unsigned sp) const { return m.kf_s[sp]; }
+  __device__ cpx<R> value(Key kf, unsigned, unsigned tu) const {
     const int t = (int)tu;
-    const long k = m.irr_s[sp];
-    const int f = m.flag_s[sp];
-    if (t < m.Nw) {
-      zd v = F[k + m.Nk * (long)t + oab];
-      return cpx<R>(f == 0 ? v : v * (pp * dprt));
-    }
-    const int j = m.M - 1 - t;
-    if (f == 0) return cpx<R>(conj(F[k + m.Nk * (long)j + oab]) * (sgn * dprt * pp));
-    return cpx<R>(F[k + m.Nk * (long)j + oba] * sgn);
+    const bool hi = t >= m.Nw, rev = (kf & 1) != 0;
+    const int j = hi ? m.M - 1 - t : t;
+    const zd v = F[(kf >> 1) + m.Nk * (long)j + (hi && rev ? oba : oab)];
+    const double f = hi ? (rev ? sgn : sgn * dprt * pp) : (rev ? pp * dprt : 1.0);
+    return cpx<R>((hi && !rev ? conj(v) : v) * f);
+  }
+  __device__ cpx<R> operator()(unsigned sp, unsigned t) const { return value(key(sp), sp, t); }
+};
+// every F_ab: item a + No b
+template <typename R>
+struct AnomBatch {
+  const zd* F;
+  long NkNw;
+  int No;
+  DualPtr<double> prt;
+  double sgn, dprt;
+  MeshDev m;
+  using Item = AnomLoad<R>;
+  __host__ __device__ Item at(unsigned i) const {
+    const int a = (int)i % No, b = (int)i / No;
+    return Item{F, NkNw * (a + (long)No * b), NkNw * (b + (long)No * a), prt[a] * prt[b], sgn, dprt, m};
   }
 };
 
@@ -356,6 +438,41 @@ struct ProductLoad {
   __host__ double algo_bytes(double N) const { return 2.0 * nterm * N * sizeof(cpx<R>); }  // A and B per term
 };
 
+// products of orbital pairs: term u of item i multiplies grid tab[2 i] of A[u]
+// by grid tab[2 i + 1] of B[u] (consecutive grids of N elements)
+template <typename R, int NT>
+struct ProductBatch {
+  const cpx<R>* A[NT];
+  const cpx<R>* B[NT];
+  R coef[NT];
+  int revt[NT];
+  long N;
+  DualPtr<int> tab;
+  MeshDev m;
+  int bmir = 0;
+  using Item = ProductLoad<R, NT>;
+  __host__ __device__ Item at(unsigned i) const {
+    Item p{};
+    const long x = N * tab[2 * (long)i], y = N * tab[2 * (long)i + 1];
+#pragma unroll
+    for (int u = 0; u < NT; ++u) {
+      p.A[u] = A[u] + x;
+      p.B[u] = B[u] + y;
+      p.coef[u] = coef[u];
+      p.revt[u] = revt[u];
+    }
+    p.nterm = NT;
+    p.m = m;
+    p.bmir = bmir;
+    return p;
+  }
+  ProductBatch from(long i) const {
+    ProductBatch p = *this;
+    p.tab = tab + 2 * i;
+    return p;
+  }
+};
+
 // G_ab(current) - G_ab(reference) on the full grid, formed in FP64 before
 // the conversion to the grid precision (increments of the bilinear bubble)
 template <typename R>
@@ -438,6 +555,42 @@ struct IncProductLoad {
   __host__ double algo_bytes(double N) const { return 4.0 * nterm * N * sizeof(cpx<R>); }  // Ar, Ad, Br, Bd per term
 };
 
+// the same for a batch, items as for ProductBatch
+template <typename R, int NT>
+struct IncProductBatch {
+  const cpx<R>* Ar[NT];
+  const cpx<R>* Ad[NT];
+  const cpx<R>* Br[NT];
+  const cpx<R>* Bd[NT];
+  R coef[NT];
+  int revt[NT];
+  long N;
+  DualPtr<int> tab;
+  MeshDev m;
+  using Item = IncProductLoad<R, NT>;
+  __host__ __device__ Item at(unsigned i) const {
+    Item p{};
+    const long x = N * tab[2 * (long)i], y = N * tab[2 * (long)i + 1];
+#pragma unroll
+    for (int u = 0; u < NT; ++u) {
+      p.Ar[u] = Ar[u] + x;
+      p.Ad[u] = Ad[u] + x;
+      p.Br[u] = Br[u] + y;
+      p.Bd[u] = Bd[u] + y;
+      p.coef[u] = coef[u];
+      p.revt[u] = revt[u];
+    }
+    p.nterm = NT;
+    p.m = m;
+    return p;
+  }
+  IncProductBatch from(long i) const {
+    IncProductBatch p = *this;
+    p.tab = tab + 2 * i;
+    return p;
+  }
+};
+
 // Sigma increment per vertex pair: acc (+)= dV~ (Fr + Fd) + FVr Fd, where dV~
 // is the transformed vertex increment, Fr / Fd the transformed reference /
 // increment of G_ab and FVr the transformed reference vertex of the pair
@@ -515,6 +668,7 @@ struct SigmaIncAccum {
   cpx<R>* const* tab;  // [c][0..2] = Fr_c, Fd_c, FVr_c
   cpx<R>* out;
   unsigned S;
+  __device__ SigmaIncAccum at(unsigned, int) const { return *this; }
   struct Pre { cpx<R> fr, fd, fv; };
   __device__ Pre prep(int c, unsigned sp, unsigned t) const {
     const size_t ad = sp + __umul24(S, t);
@@ -535,6 +689,7 @@ struct SigmaIncAccumG {
   const cpx<R>* Y;
   cpx<R>* out;
   unsigned S;
+  __device__ SigmaIncAccumG at(unsigned, int) const { return *this; }
   struct Pre { cpx<R> g; };
   __device__ Pre prep(int c, unsigned sp, unsigned t) const { return Pre{tab[c][sp + __umul24(S, t)]}; }
   __device__ cpx<R> contrib(int, const Pre& q, cpx<R> v) const { return v * q.g; }
@@ -572,6 +727,8 @@ struct MulAccAccum {
   cpx<R>* const* tab;  // [c] = F_c
   cpx<R>* out;
   unsigned S;
+  long N;
+  __device__ MulAccAccum at(unsigned o, int first) const { return MulAccAccum{tab + first, out + (long)o * N, S, N}; }
   struct Pre { cpx<R> f; };
   __device__ Pre prep(int c, unsigned sp, unsigned t) const { return Pre{tab[c][sp + __umul24(S, t)]}; }
   __device__ cpx<R> contrib(int, const Pre& q, cpx<R> v) const { return v * q.f; }
@@ -599,8 +756,16 @@ struct GatherStore {
   // optional, for a last pass whose boxes span the t axis: per box (index
   // after box_remap), nonzero if it holds a kept spatial point; live_frac is
   // the fraction of boxes that do
+  // (live_s, live_s_frac: of the plan's small boxes)
   const unsigned char* live = nullptr;
   double live_frac = 1.0;
+  const unsigned char* live_s = nullptr;
+  double live_s_frac = 1.0;
+  int cj = 0;  // the value is conjugated before base is added
+  void use_small_boxes() {
+    live = live_s;
+    live_frac = live_s_frac;
+  }
   struct Pre { long o; zd old, bv, js; };  // o < 0: slot or point not kept
   // branch-free: a dropped slot or point is not stored, and an operand the
   // store does not use is read at element 0 (one cached line) and dropped
@@ -623,6 +788,7 @@ struct GatherStore {
     if (q.o < 0) return;
     zd x = zd(v) * w;
     if (sawc) x += q.js;
+    if (cj) x = conj(x);
     if (base) x += q.bv;
     const zd f = acc ? q.old + x : x;
     dst[q.o] = f;
@@ -639,19 +805,55 @@ struct GatherStore {
   __host__ double read_fraction(bool t_box) const { return t_box ? (live ? live_frac : 1.0) : (double)m.Nw / m.M; }
 };
 
+// slices of a (Nk, Nw, ...) array: item i stores slice tab[4 i] of dst (base:
+// of base), its partner tab[4 i + 1] (none if negative), reads J[tab[4 i + 2]];
+// tab[4 i + 3]: 1 conjugated (cj), 2 the partner's sign is -1
+template <typename R>
+struct GatherBatch {
+  zd* dst;
+  long NkNw;
+  DualPtr<int> tab;
+  GatherStore<R> proto;
+  using Item = GatherStore<R>;
+  __host__ __device__ Item at(unsigned i) const {
+    const long t = 4 * (long)i;
+    Item g = proto;
+    g.dst = dst + NkNw * tab[t];
+    if (proto.base) g.base = proto.base + NkNw * tab[t];
+    const int p = tab[t + 1], f = tab[t + 3];
+    if (p >= 0) g.pdst = dst + NkNw * p;
+    if (proto.J) g.J = proto.J + tab[t + 2];
+    g.cj = f & 1;
+    g.psign = (f & 2) ? -1.0 : 1.0;
+    return g;
+  }
+  GatherBatch from(long i) const { return GatherBatch{dst, NkNw, tab + 4 * i, proto}; }
+  void use_small_boxes() { proto.use_small_boxes(); }
+};
+
+// Products summed over sources: out + o N (o < nout) = sum of A_{ta[c]} B_{tb[c]}
+// over c = off[o] .. off[o + 1] - 1 in turn (grids of N elements)
+template <typename R>
+void contract(cpx<R>* out, const cpx<R>* A, const cpx<R>* B, const int* off, const int* ta, const int* tb, int nout,
+              long N, hipStream_t s);
+// partner slices of a (Nk, Nw, ...) array: slice tab[4 i + 1] = +-conj slice
+// tab[4 i] (GatherBatch's table; negative: none)
+void partner_copies(zd* a, const int* tab, int n, long NkNw, hipStream_t s);
+
 // acc (+)= A * B
 template <typename R>
 void mul_acc(cpx<R>* acc, const cpx<R>* A, const cpx<R>* B, bool first, long n, hipStream_t s);
 
-// The analytic tau reference kernels of one orbital pair (a, b) written out on
+// The analytic tau reference kernels of the orbital pairs (a, b) written out on
 // the full grid (the functions of TauRefLoad, fchi.f90:703-729, 791-812):
 // ta(sp, s) = sum_n c_n g0_n(tau_s), tb(sp, s) = sum_n c_n g1_n(tau_s), with
 // c_n = U_an conj(U_bn) (conjugated at -k).  diff: the differences between
 // chemical potentials mu and mu2.  The exponentials advance by one factor per
 // slot (No <= 8; FP64 arithmetic, stored at the grid precision).
+// Every pair: grids a + No b of ta and tb.
 template <typename R>
-void tau_ref_grids(cpx<R>* ta, cpx<R>* tb, const double* eig, const zd* uni, int a, int b, int No, double mu,
-                   double mu2, bool diff, double beta, double dtau, const MeshDev& m, hipStream_t s);
+void tau_ref_grids(cpx<R>* ta, cpx<R>* tb, const double* eig, const zd* uni, int No, double mu, double mu2, bool diff,
+                   double beta, double dtau, const MeshDev& m, hipStream_t s);
 
 // Tail constants of chi0 (fchi.f90:731-772), on the device: rb[m + No l] =
 // the full-zone average of sum_n U_mn conj(U_ln) f_n(mu) (transposed at -k);
@@ -666,10 +868,10 @@ void sawtooth(zd* sawc, int Nw, double temp, hipStream_t s);
 void conj_copy(zd* dst, const zd* src, long n, hipStream_t s);
 void conj_copy(zd* dst, const zd* src, long n, double sign, hipStream_t s);  // dst = sign conj(src), sign = +-1
 void threshold(zd* a, long n, double eps, hipStream_t s);
-// dst(r, t) = src(-r, -t) on an (Nx, Ny, Nz, M) grid (the operand a
+// dst(r, t) = src(-r, -t) on n (Nx, Ny, Nz, M) grids (the operand a
 // (-r, -tau) product reads, laid out to be read in place)
 template <typename R>
-void mirror_grid(cpx<R>* dst, const cpx<R>* src, int Nx, int Ny, int Nz, int M, hipStream_t s);
+void mirror_grid(cpx<R>* dst, const cpx<R>* src, int Nx, int Ny, int Nz, int M, int n, hipStream_t s);
 // dst(k, e) = src(k, w = 0, e) with threshold eps, e < nmat (the first
 // frequency slice of a (Nk, Nw, nmat) array, as a (Nk, nmat) array)
 void threshold_slice(zd* dst, const zd* src, long Nk, long NkNw, long nmat, double eps, hipStream_t s);
