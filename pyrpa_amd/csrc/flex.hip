@@ -521,7 +521,7 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
       // the new residual's row of the Gram matrix (n entries 0 .. n-1 are in
       // use); the others stand from the iterations before
       std::vector<zd> row(n);
-      dots(row.data(), res.p + cur * nS, res.p, (long)nS, n, nullptr, (long)nS, 1, s);
+      dots(row.data(), res.p + cur * nS, res.p, (long)nS, n, (long)nS, s);
       for (int i = 0; i < n; ++i) gram[cur + m * i] = gram[i + m * cur] = row[i].re;
       std::vector<double> B((n + 1) * (n + 1), 0.0), c(n + 1, 0.0);
       for (int a = 0; a < n; ++a) {

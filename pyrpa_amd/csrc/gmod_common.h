@@ -122,18 +122,17 @@ struct DBuf {
 };
 
 // ----------------------------------------------------------------- context
-// Results that the host waits for (reductions, error flags) are written by
-// the kernel that finishes them straight into `pin` (pinned, mapped), so a
-// wait is one stream synchronisation without a copy; `red` holds partial sums
-// and the ticket counter of the reductions (zero between launches).  One call
-// uses them at a time: every entry point holds `lock`.
-constexpr int PIN_DOUBLES = 4096;
-constexpr int RED_MAX_BLOCKS = 1024, RED_MAX_WIDTH = 4;
+// Results that the host waits for (partial results of reductions, error flags)
+// are written by their kernel straight into `pin` (pinned, mapped), so a wait
+// is one stream synchronisation without a copy; `red` holds the partial sums
+// that a following launch combines.  One call uses them at a time: every entry
+// point holds `lock`.
+constexpr int PIN_DOUBLES = 8192;
+constexpr int RED_MAX_BLOCKS = 512;
 struct Context {
   hipStream_t stream = nullptr;
   double* pin = nullptr;
   double* red = nullptr;
-  unsigned* ticket = nullptr;
   int device = 0;
   int precision = 0;  // 0: FP64 everywhere; 1: FP32 convolutions (FP64 LU/Dyson/mu/lambda)
   int verbose = 0;

@@ -894,9 +894,8 @@ void sum_diff(zd* a, zd* b, long n, hipStream_t s);
 // ---- deterministic reductions (fixed order), each waiting for its result
 // sum over k-space arrays laid out (Nk, rest): weights kw[k] (or 1)
 zd dot_w(const zd* u, const zd* v, const double* kw, long Nk, long rest, hipStream_t s);  // sum kw conj(u) v
-// the same with nv vectors v + i stride
-void dots(zd* out, const zd* u, const zd* v, long stride, int nv, const double* kw, long Nk, long rest,
-          hipStream_t s);
+// sum conj(u) v for the nv vectors v + i stride of n elements
+void dots(zd* out, const zd* u, const zd* v, long stride, int nv, long n, hipStream_t s);
 // sum kw |nd|^2, Re sum kw conj(D) nd, sum kw |D|^2
 void power_dots(double out[3], const zd* nd, const zd* D, const double* kw, long Nk, long rest, hipStream_t s);
 // modified Gram-Schmidt: for each v in turn h_i = f sum kw conj(v) x, x -= h_i v;

@@ -658,39 +658,45 @@ double gram_schmidt(zd* x, const std::vector<const zd*>& vs, zd* h, double f, co
   return std::sqrt(f * t);
 }
 
-// sum kw conj(u) v_y of the nv vectors v + y stride (blockIdx.y = y)
+// sum conj(u) v_y of the nv vectors v + y stride (blockIdx.y = y)
 __global__ void __launch_bounds__(RED_TPB)
-k_dots(const zd* __restrict__ u, const zd* __restrict__ v, long stride, const double* __restrict__ kw, long Nk,
-       long n, double* part, unsigned* ticket, double* out) {
+k_dots(const zd* __restrict__ u, const zd* __restrict__ v, long stride, long n, double* part) {
   const zd* __restrict__ vy = v + (long)blockIdx.y * stride;
   double r[2] = {0, 0};
   for (long e = blockIdx.x * (long)RED_TPB + threadIdx.x; e < n; e += (long)gridDim.x * RED_TPB) {
     const zd p = conj(u[e]) * vy[e];
-    const double w = kw ? kw[e % Nk] : 1.0;
-    r[0] += w * p.re;
-    r[1] += w * p.im;
+    r[0] += p.re;
+    r[1] += p.im;
   }
-  finish_reduce<RedSum, 2>(r, blockIdx.x, gridDim.x, part + (long)blockIdx.y * 2 * RED_MAX_BLOCKS,
-                           ticket + blockIdx.y, out + 2 * blockIdx.y);
+  put_partial<RedSum, 2>(r, blockIdx.x, part + (long)blockIdx.y * 2 * gridDim.x);
 }
 
-void dots(zd* out, const zd* u, const zd* v, long stride, int nv, const double* kw, long Nk, long rest,
-          hipStream_t s) {
-  const long n = Nk * rest;
-  Context& c = ctx();
-  for (int v0 = 0; v0 < nv; v0 += 64) {  // as many as there are ticket counters
-    const int m = std::min(64, nv - v0);
-    hipLaunchKernelGGL(k_dots, dim3(red_blocks(n), m), dim3(RED_TPB), 0, s, u, v + v0 * stride, stride, kw, Nk, n,
-                       c.red, c.ticket, c.pin);
+void dots(zd* out, const zd* u, const zd* v, long stride, int nv, long n, hipStream_t s) {
+  const double* p = ctx().pin;
+  const int nb = red_blocks(n), room = PIN_DOUBLES / (2 * nb);
+  for (int v0 = 0; v0 < nv; v0 += room) {
+    const int m = std::min(room, nv - v0);
+    hipLaunchKernelGGL(k_dots, dim3(nb, m), dim3(RED_TPB), 0, s, u, v + v0 * stride, stride, n, ctx().pin);
     GMOD_CHECK_LAUNCH();
     wait(s);
-    for (int i = 0; i < m; ++i) out[v0 + i] = zd(c.pin[2 * i], c.pin[2 * i + 1]);
+    for (int i = 0; i < m; ++i)
+      out[v0 + i] = zd(sum_partials(p + 2 * nb * i, nb, 2, 0), sum_partials(p + 2 * nb * i, nb, 2, 1));
   }
+}
+
+// extremes: the partial results combined on the host; the error flag, when
+// asked for, behind them
+template <class Op>
+static double host_extreme(int nb, const int* err, int* err_out) {
+  const double* p = ctx().pin;
+  double r = Op::id();
+  for (int b = 0; b < nb; ++b) r = Op::op(r, p[b]);
+  if (err) *err_out = (int)p[nb];
+  return r;
 }
 
 __global__ void __launch_bounds__(RED_TPB)
-k_max_rel(const zd* __restrict__ s0, const zd* __restrict__ sd, long n, double floor, double* part, unsigned* ticket,
-          double* out, const int* err) {
+k_max_rel(const zd* __restrict__ s0, const zd* __restrict__ sd, long n, double floor, double* part, const int* err) {
   double best[1] = {0.0};
   for (long e = blockIdx.x * (long)RED_TPB + threadIdx.x; e < n; e += (long)gridDim.x * RED_TPB) {
     const zd d = sd[e];
@@ -701,71 +707,61 @@ k_max_rel(const zd* __restrict__ s0, const zd* __restrict__ sd, long n, double f
       if (r > best[0]) best[0] = r;
     }
   }
-  finish_reduce<RedMax, 1>(best, blockIdx.x, gridDim.x, part, ticket, out, err);
+  put_partial<RedMax, 1>(best, blockIdx.x, part);
+  if (err && blockIdx.x == 0 && threadIdx.x == 0) part[gridDim.x] = (double)*err;
 }
 double max_rel_err(const zd* s0, const zd* sd, long n, double floor, hipStream_t s, const int* err, int* err_out) {
-  Context& c = ctx();
-  hipLaunchKernelGGL(k_max_rel, dim3(red_blocks(n)), dim3(RED_TPB), 0, s, s0, sd, n, floor, c.red, c.ticket, c.pin,
-                     err);
+  const int nb = red_blocks(n);
+  hipLaunchKernelGGL(k_max_rel, dim3(nb), dim3(RED_TPB), 0, s, s0, sd, n, floor, ctx().pin, err);
   GMOD_CHECK_LAUNCH();
   wait(s);
-  if (err) *err_out = (int)c.pin[1];
-  return c.pin[0];
+  return host_extreme<RedMax>(nb, err, err_out);
 }
 
 template <class Op>
 __global__ void __launch_bounds__(RED_TPB)
-k_extreme(const double* __restrict__ a, long stride, long n, double* part, unsigned* ticket, double* out,
-          const int* err) {
+k_extreme(const double* __restrict__ a, long stride, long n, double* part, const int* err) {
   double best[1] = {Op::id()};
   for (long e = blockIdx.x * (long)RED_TPB + threadIdx.x; e < n; e += (long)gridDim.x * RED_TPB)
     best[0] = Op::op(best[0], a[e * stride]);
-  finish_reduce<Op, 1>(best, blockIdx.x, gridDim.x, part, ticket, out, err);
+  put_partial<Op, 1>(best, blockIdx.x, part);
+  if (err && blockIdx.x == 0 && threadIdx.x == 0) part[gridDim.x] = (double)*err;
+}
+template <class Op>
+static double extreme(const double* a, long stride, long n, hipStream_t s, const int* err, int* err_out) {
+  const int nb = red_blocks(n);
+  hipLaunchKernelGGL(k_extreme<Op>, dim3(nb), dim3(RED_TPB), 0, s, a, stride, n, ctx().pin, err);
+  GMOD_CHECK_LAUNCH();
+  wait(s);
+  return host_extreme<Op>(nb, err, err_out);
 }
 double max_value(const double* a, long n, hipStream_t s, const int* err, int* err_out) {
-  Context& c = ctx();
-  hipLaunchKernelGGL(k_extreme<RedMax>, dim3(red_blocks(n)), dim3(RED_TPB), 0, s, a, 1L, n, c.red, c.ticket, c.pin,
-                     err);
-  GMOD_CHECK_LAUNCH();
-  wait(s);
-  if (err) *err_out = (int)c.pin[1];
-  return c.pin[0];
+  return extreme<RedMax>(a, 1, n, s, err, err_out);
 }
 double max_real(const zd* a, long n, hipStream_t s) {
-  Context& c = ctx();
-  hipLaunchKernelGGL(k_extreme<RedMax>, dim3(red_blocks(n)), dim3(RED_TPB), 0, s, (const double*)a, 2L, n, c.red,
-                     c.ticket, c.pin, (const int*)nullptr);
-  GMOD_CHECK_LAUNCH();
-  wait(s);
-  return c.pin[0];
+  return extreme<RedMax>((const double*)a, 2, n, s, nullptr, nullptr);
 }
 double min_real(const zd* a, long n, hipStream_t s) {
-  Context& c = ctx();
-  hipLaunchKernelGGL(k_extreme<RedMin>, dim3(red_blocks(n)), dim3(RED_TPB), 0, s, (const double*)a, 2L, n, c.red,
-                     c.ticket, c.pin, (const int*)nullptr);
-  GMOD_CHECK_LAUNCH();
-  wait(s);
-  return c.pin[0];
+  return extreme<RedMin>((const double*)a, 2, n, s, nullptr, nullptr);
 }
 
 // max |a - b| (b null: max |a|)
 __global__ void __launch_bounds__(RED_TPB)
-k_max_absdiff(const zd* __restrict__ a, const zd* __restrict__ b, long n, double* part, unsigned* ticket,
-              double* out) {
+k_max_absdiff(const zd* __restrict__ a, const zd* __restrict__ b, long n, double* part) {
   double best[1] = {0.0};
   for (long e = blockIdx.x * (long)RED_TPB + threadIdx.x; e < n; e += (long)gridDim.x * RED_TPB) {
     const zd d = b ? a[e] - b[e] : a[e];
     const double r = hypot(d.re, d.im);
     if (r > best[0]) best[0] = r;
   }
-  finish_reduce<RedMax, 1>(best, blockIdx.x, gridDim.x, part, ticket, out);
+  put_partial<RedMax, 1>(best, blockIdx.x, part);
 }
 double max_abs_diff(const zd* a, const zd* b, long n, hipStream_t s) {
-  Context& c = ctx();
-  hipLaunchKernelGGL(k_max_absdiff, dim3(red_blocks(n)), dim3(RED_TPB), 0, s, a, b, n, c.red, c.ticket, c.pin);
+  const int nb = red_blocks(n);
+  hipLaunchKernelGGL(k_max_absdiff, dim3(nb), dim3(RED_TPB), 0, s, a, b, n, ctx().pin);
   GMOD_CHECK_LAUNCH();
   wait(s);
-  return c.pin[0];
+  return host_extreme<RedMax>(nb, nullptr, nullptr);
 }
 
 // y = sum_i c_i x_i over up to COMBINE vectors x + idx_i stride (add: onto y)

@@ -1572,11 +1572,11 @@ __global__ void __launch_bounds__(128) k_charpoly(zd* coef, const zd* sig, const
 }
 
 // n(mu) pieces from the characteristic polynomials (see k_charpoly), summed
-// in the same launch (latency-bound: with a copy of the partial sums to the
-// host a trial mu took 24 us at 1 orbital, 32x32 x 256)
+// by the host from pinned memory (latency-bound: with a copy of the partial
+// sums a trial mu took 24 us at 1 orbital, 32x32 x 256)
 template <int NO>
 __global__ void __launch_bounds__(RED_TPB) k_filling_cp(const zd* coef, const double* eig, double rmu, double temp,
-                                                        long Nk, int Nw, double* part, unsigned* ticket, double* out) {
+                                                        long Nk, int Nw, double* part) {
   const long tot = Nk * (long)Nw;
   double r[2] = {0.0, 0.0};
   for (long e = blockIdx.x * (long)RED_TPB + threadIdx.x; e < tot; e += (long)gridDim.x * RED_TPB) {
@@ -1598,7 +1598,7 @@ __global__ void __launch_bounds__(RED_TPB) k_filling_cp(const zd* coef, const do
       for (int n = 0; n < NO; ++n) r[0] += 0.5 * (1.0 - tanh(0.5 * (eig[n + NO * k] - rmu) / temp));
     }
   }
-  finish_reduce<RedSum, 2>(r, blockIdx.x, gridDim.x, part, ticket, out);
+  put_partial<RedSum, 2>(r, blockIdx.x, part);
 }
 
 template <int NO>
@@ -1798,13 +1798,11 @@ void filling_charpoly(zd* coef, const zd* sigma, const zd* hamk, long Nk, int Nw
 
 void filling_parts_cp(double out[2], const zd* coef, const double* eig, double rmu, double temp, long Nk, int Nw,
                       int No, hipStream_t s) {
-  Context& c = ctx();
-  LAUNCH_NO(No, k_filling_cp, dim3(red_blocks(Nk * (long)Nw)), dim3(RED_TPB), coef, eig, rmu, temp, Nk, Nw, c.red,
-            c.ticket, c.pin);
+  const int nb = red_blocks(Nk * (long)Nw);
+  LAUNCH_NO(No, k_filling_cp, dim3(nb), dim3(RED_TPB), coef, eig, rmu, temp, Nk, Nw, ctx().pin);
   GMOD_CHECK_LAUNCH();
   GMOD_HIP(hipStreamSynchronize(s));
-  out[0] = c.pin[0];
-  out[1] = c.pin[1];
+  for (int c = 0; c < 2; ++c) out[c] = sum_partials(ctx().pin, nb, 2, c);
 }
 
 void green0(zd* G, const double* eig, const zd* uni, double mu, double temp, long Nk, int Nw, int No,

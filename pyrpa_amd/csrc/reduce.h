@@ -1,6 +1,8 @@
-// Deterministic reductions to the host in one launch: every work-group
-// reduces its share, the last one to finish (a ticket counter) combines the
-// partial results in their fixed order and writes the result to pinned memory.
+// Deterministic reductions to the host in one launch: every work-group writes
+// its partial result to pinned memory, the host combines the few hundred of
+// them in order after the wait it needs anyway (about 1 us).  Combining them on
+// the device by the last work-group to finish needs a fence per work-group,
+// which writes the L2 back: 33 us against 17 for n(mu) at 2.1 M points.
 #pragma once
 #include "gmod_common.h"
 
@@ -8,23 +10,23 @@ namespace gmod {
 
 constexpr int RED_TPB = 256;
 
-// work-groups for n elements: one per 1024, at most RED_MAX_BLOCKS
+// work-groups for n elements: one per 512, at most RED_MAX_BLOCKS
 inline int red_blocks(long n) {
-  const long b = (n + 1023) / 1024;
+  const long b = (n + 511) / 512;
   return (int)(b < 1 ? 1 : b > RED_MAX_BLOCKS ? RED_MAX_BLOCKS : b);
 }
 
 struct RedSum {
-  static __device__ double id() { return 0.0; }
-  static __device__ double op(double a, double b) { return a + b; }
+  static __host__ __device__ double id() { return 0.0; }
+  static __host__ __device__ double op(double a, double b) { return a + b; }
 };
 struct RedMax {
-  static __device__ double id() { return -HUGE_VAL; }
-  static __device__ double op(double a, double b) { return fmax(a, b); }
+  static __host__ __device__ double id() { return -HUGE_VAL; }
+  static __host__ __device__ double op(double a, double b) { return fmax(a, b); }
 };
 struct RedMin {
-  static __device__ double id() { return HUGE_VAL; }
-  static __device__ double op(double a, double b) { return fmin(a, b); }
+  static __host__ __device__ double id() { return HUGE_VAL; }
+  static __host__ __device__ double op(double a, double b) { return fmin(a, b); }
 };
 
 // v: this thread's values -> on thread 0 the work-group's (RED_TPB threads)
@@ -49,39 +51,22 @@ __device__ __forceinline__ void block_reduce(double (&v)[W], double* sh) {
   __syncthreads();
 }
 
-// The launch's result for the nb work-groups b = 0 .. nb - 1: out[0 .. W) and,
-// when err is given, out[W] = its value (an error flag read along).  part has
-// room for nb W values, *ticket is zero before and after.
+// the work-group's partial result at part[W b]
 template <class Op, int W>
-__device__ __forceinline__ void finish_reduce(double (&v)[W], int b, int nb, double* part, unsigned* ticket,
-                                              double* out, const int* err = nullptr) {
+__device__ __forceinline__ void put_partial(double (&v)[W], int b, double* part) {
   __shared__ double sh[W * (RED_TPB / 64)];
-  __shared__ unsigned last;
   block_reduce<Op, W>(v, sh);
   if (threadIdx.x == 0) {
 #pragma unroll
     for (int c = 0; c < W; ++c) part[W * b + c] = v[c];
-    __threadfence();
-    last = atomicAdd(ticket, 1u) == (unsigned)nb - 1u;
   }
-  __syncthreads();
-  if (!last) return;
-  __threadfence();
-  double r[W];
-#pragma unroll
-  for (int c = 0; c < W; ++c) r[c] = Op::id();
-  for (int i = threadIdx.x; i < nb; i += RED_TPB) {
-#pragma unroll
-    for (int c = 0; c < W; ++c)
-      r[c] = Op::op(r[c], __hip_atomic_load(part + W * i + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-  }
-  block_reduce<Op, W>(r, sh);
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int c = 0; c < W; ++c) out[c] = r[c];
-    if (err) out[W] = (double)*err;
-    *ticket = 0u;
-  }
+}
+
+// host: the partial results of component c combined in order
+inline double sum_partials(const double* part, int nb, int W, int c) {
+  double r = 0.0;
+  for (int b = 0; b < nb; ++b) r += part[W * b + c];
+  return r;
 }
 
 }  // namespace gmod

@@ -21,10 +21,7 @@ Context& ctx() {
     GMOD_HIP(hipSetDevice(0));
     GMOD_HIP(hipStreamCreateWithFlags(&cc->stream, hipStreamNonBlocking));
     GMOD_HIP(hipHostMalloc((void**)&cc->pin, PIN_DOUBLES * sizeof(double), hipHostMallocMapped));
-    GMOD_HIP(hipMalloc((void**)&cc->red, (size_t)RED_MAX_BLOCKS * RED_MAX_WIDTH * 64 * sizeof(double)));
-    GMOD_HIP(hipMalloc((void**)&cc->ticket, 64 * sizeof(unsigned)));
-    GMOD_HIP(hipMemset(cc->ticket, 0, 64 * sizeof(unsigned)));
-    GMOD_HIP(hipDeviceSynchronize());
+    GMOD_HIP(hipMalloc((void**)&cc->red, PIN_DOUBLES * sizeof(double)));
     if (const char* p = getenv("GMOD_PRECISION")) cc->precision = atoi(p);
     if (const char* v = getenv("GMOD_VERBOSE")) cc->verbose = atoi(v);
     return cc;
