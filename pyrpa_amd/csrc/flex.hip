@@ -8,6 +8,7 @@
 
 #include "../../include/gmod.h"
 #include "engine.h"
+#include "transfer.h"
 
 namespace gmod {
 
@@ -64,9 +65,15 @@ struct Upload {
   template <typename T>
   void operator()(DBuf<T>& d, const T* h, size_t n) {
     d.alloc(n);
-    d.upload(h, n, s);
+    copy_to_device(d.p, h, n * sizeof(T), s);
   }
 };
+
+// a result into the caller's array, complete on return
+template <typename T>
+static void fetch(T* h, const DBuf<T>& d, size_t n, hipStream_t s) {
+  copy_to_host(h, d.p, n * sizeof(T), s);
+}
 
 // Stoner factor: max_q max Re eig(chi0(q,0) S) (fchi.f90:352-399); thr > 0:
 // of the thresholded chi0 (the first frequency slice is copied with it)
@@ -119,7 +126,7 @@ static void chi0_driver(zd* chi_h, const zd* Gk, const int64_t* kmap, const int6
     up(S_d, S, (size_t)Nchi * Nchi);
     *stoner = stoner_factor(chi.p, Nk, Nw, Nchi, S_d.p, s, 0.0, alpha);
   }
-  chi.download(chi_h, NkNw * Nchi * Nchi, s);
+  fetch(chi_h, chi, NkNw * Nchi * Nchi, s);
   GMOD_HIP(hipStreamSynchronize(s));
 }
 
@@ -567,16 +574,13 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
   check_err(err, s, "mkself");
   const double t_solve = secs(t_dev);
   if (stoner >= 1.0 && verbose) printf("[FLEX] WARNING: Stoner factor >= 1 at the final iteration\n");
-  std::vector<zd> h(nS);
-  sig.download(h.data(), nS, s);
-  GMOD_HIP(hipStreamSynchronize(s));
-  memcpy(sig_out, h.data(), nS * sizeof(zd));
+  fetch(sig_out, sig, nS, s);
   *mu_out = mu;
   if (A.sw_out) {
     std::ofstream f("sigma.bin", std::ios::binary);
     write_record(f, &mu_file, 8);
     write_record(f, &mu_old_file, 8);
-    write_record(f, h.data(), nS * sizeof(zd));
+    write_record(f, sig_out, nS * sizeof(zd));
     double meta[4] = {T, (double)Nw, (double)No, (double)Nk};
     write_record(f, meta, 32);
     if (!f) throw Error("io_sigma: cannot write sigma.bin");
@@ -749,7 +753,8 @@ static double eliash_driver(const EliashIn& A, zd* delta_out) {
   up(C_d, A.Cmat, (size_t)Nchi * Nchi);
   rpa_vertex(chi.p, NkNw, BatchLayout{1, NkNw}, Nchi, S_d.p, C_d.p, singlet ? 1 : 2, err.p, s);
   check_err(err, s, "get_V_delta_nsoc_flex");
-  chi.download(A.chi, nC, s);  // chi is inout: it leaves holding V_Delta (feliash.f90:42,61)
+  HostCopy v_out;  // chi is inout: it leaves holding V_Delta (feliash.f90:42,61), copied while the solver runs
+  v_out.start(A.chi, chi.p, nC * sizeof(zd), s);
   ConvEngine<R> eng(mesh, op);
   eng.prepare_gap(chi.p, A.Smat, A.Cmat, singlet, s);
   const long rest = Nw * No * No;
@@ -815,7 +820,8 @@ static double eliash_driver(const EliashIn& A, zd* delta_out) {
     copy(D.p, nd.p, nS, s);
     scale(D.p, nS, 1.0 / nrm, s);
   }
-  D.download(delta_out, nS, s);
+  v_out.wait();
+  fetch(delta_out, D, nS, s);
   GMOD_HIP(hipStreamSynchronize(s));
   return lam_out;
 }
@@ -865,7 +871,8 @@ static double eliash_soc_driver(const EliashSocIn& A, zd* delta_out) {
   up(inv_d, invh.data(), (size_t)No);
   soc_vertex(chi.p, chi.p, NkNw, BatchLayout{1, NkNw}, Nchi, V_d.p, 0.0, err.p, s);
   check_err(err, s, "get_V_soc_flex");
-  chi.download(A.chi, nC, s);  // chi is inout: it leaves holding V_Delta (feliashwithsoc.f90:55)
+  HostCopy v_out;  // chi is inout: it leaves holding V_Delta (feliashwithsoc.f90:55), copied while the solver runs
+  v_out.start(A.chi, chi.p, nC * sizeof(zd), s);
   if (verbose)
     printf("V_delta max is %16.8E\nV_delta min is %16.8E\n", max_real(chi.p, nC, s), min_real(chi.p, nC, s));
   ConvEngine<R> eng(mesh, op);
@@ -930,7 +937,8 @@ static double eliash_soc_driver(const EliashSocIn& A, zd* delta_out) {
     copy(D.p, nd.p, nF, s);
     scale(D.p, nF, 1.0 / nrm, s);
   }
-  D.download(delta_out, nF, s);
+  v_out.wait();
+  fetch(delta_out, D, nF, s);
   GMOD_HIP(hipStreamSynchronize(s));
   return lam;
 }
@@ -1126,9 +1134,9 @@ static void nonlin_eliash_driver(const NonlinIn& A, zd* delta_io, zd* sigma_out,
       vertices();
     }
   }
-  D.download(delta_io, nS, s);
-  sig.download(sigma_out, nS, s);
-  G.download(Gk_io, nS, s);
+  fetch(delta_io, D, nS, s);
+  fetch(sigma_out, sig, nS, s);
+  fetch(Gk_io, G, nS, s);
   GMOD_HIP(hipStreamSynchronize(s));
   g_nonlin_stats[0] = (double)it_done;
   g_nonlin_stats[1] = (double)status;
@@ -1223,7 +1231,7 @@ extern "C" void get_vsigma_flex_nosoc_(gmod_z* chi, const double* Smat, const do
   up(C, Cmat, (size_t)n * n);
   rpa_vertex(c.p, NkNw, BatchLayout{1, NkNw}, n, S.p, C.p, 0, err.p, s);
   check_err(err, s, "get_vsigma_flex_nosoc");
-  c.download((zd*)chi, (size_t)NkNw * n * n, s);
+  fetch((zd*)chi, c, (size_t)NkNw * n * n, s);
   GMOD_HIP(hipStreamSynchronize(s));
   GMOD_CATCH
 }
@@ -1246,7 +1254,7 @@ extern "C" void gmod_v_soc_flex(gmod_z* chi, const double* Vmat, const int64_t* 
   up(V, Vmat, (size_t)n * n);
   soc_vertex(c.p, c.p, NkNw, BatchLayout{1, NkNw}, n, V.p, 0.0, err.p, s);
   check_err(err, s, "get_V_soc_flex");
-  c.download((zd*)chi, (size_t)NkNw * n * n, s);
+  fetch((zd*)chi, c, (size_t)NkNw * n * n, s);
   GMOD_HIP(hipStreamSynchronize(s));
   GMOD_CATCH
 }
@@ -1267,9 +1275,17 @@ extern "C" void get_chis(gmod_z* chis, const gmod_z* chi0, const double* Smat, c
   up(S, Smat, (size_t)n * n);
   rpa_solve(o.p, BatchLayout{(long)n * n, 1}, a.p, BatchLayout{(long)n * n, 1}, nw, n, S.p, -1.0, err.p, s);
   check_err(err, s, "get_chis");
-  o.download((zd*)chis, (size_t)n * n * nw, s);
+  fetch((zd*)chis, o, (size_t)n * n * nw, s);
   GMOD_HIP(hipStreamSynchronize(s));
   GMOD_CATCH
+}
+
+// the rows chi(:, 1, :, :) of the caller's array, all that a static
+// susceptibility reads
+static std::vector<zd> static_slice(const zd* chi, long nk, long NkNw, int n) {
+  std::vector<zd> out((size_t)nk * n * n);
+  for (int e = 0; e < n * n; ++e) memcpy(&out[(size_t)nk * e], chi + NkNw * e, nk * sizeof(zd));
+  return out;
 }
 
 extern "C" void get_chis_chic(gmod_z* chis, gmod_z* chic, const gmod_z* chi, const double* Smat, const double* Cmat,
@@ -1284,15 +1300,15 @@ extern "C" void get_chis_chic(gmod_z* chis, gmod_z* chic, const gmod_z* chi, con
   DBuf<double> S, C;
   DBuf<int> err(1);
   err.zero(s);
-  // only the static slice chi(:,1,:,:) is read: copy it with the full layout
-  up(a, (const zd*)chi, (size_t)NkNw * n * n);
+  const std::vector<zd> slice = static_slice((const zd*)chi, nk, NkNw, n);
+  up(a, slice.data(), slice.size());
   up(S, Smat, (size_t)n * n);
   up(C, Cmat, (size_t)n * n);
-  rpa_solve(os.p, BatchLayout{1, nk}, a.p, BatchLayout{1, NkNw}, nk, n, S.p, -1.0, err.p, s);
-  rpa_solve(oc.p, BatchLayout{1, nk}, a.p, BatchLayout{1, NkNw}, nk, n, C.p, 1.0, err.p, s);
+  rpa_solve(os.p, BatchLayout{1, nk}, a.p, BatchLayout{1, nk}, nk, n, S.p, -1.0, err.p, s);
+  rpa_solve(oc.p, BatchLayout{1, nk}, a.p, BatchLayout{1, nk}, nk, n, C.p, 1.0, err.p, s);
   check_err(err, s, "get_chis_chic");
-  os.download((zd*)chis, (size_t)nk * n * n, s);
-  oc.download((zd*)chic, (size_t)nk * n * n, s);
+  fetch((zd*)chis, os, (size_t)nk * n * n, s);
+  fetch((zd*)chic, oc, (size_t)nk * n * n, s);
   GMOD_HIP(hipStreamSynchronize(s));
   GMOD_CATCH
 }
@@ -1319,14 +1335,14 @@ extern "C" void gmod_get_chis_chic_all(gmod_z* chis, gmod_z* chic, const gmod_z*
     up(S, Smat, (size_t)n * n);
     rpa_solve(o.p, BatchLayout{1, NkNw}, a.p, BatchLayout{1, NkNw}, NkNw, n, S.p, -1.0, err.p, s);
     check_err(err, s, "gmod_get_chis_chic_all (chi_s)");
-    o.download((zd*)chis, tot, s);
+    fetch((zd*)chis, o, tot, s);
     GMOD_HIP(hipStreamSynchronize(s));
   }
   if (chic) {
     up(C, Cmat, (size_t)n * n);
     rpa_solve(o.p, BatchLayout{1, NkNw}, a.p, BatchLayout{1, NkNw}, NkNw, n, C.p, 1.0, err.p, s);
     check_err(err, s, "gmod_get_chis_chic_all (chi_c)");
-    o.download((zd*)chic, tot, s);
+    fetch((zd*)chic, o, tot, s);
     GMOD_HIP(hipStreamSynchronize(s));
   }
   GMOD_CATCH
@@ -1368,7 +1384,7 @@ extern "C" void get_eig_or_tr_chi(gmod_z* chiqout, const gmod_z* chi, const int6
     hipLaunchKernelGGL(k_trace_map, dim3(256), dim3(256), 0, s, o.p, a.p, iv.p, nka, nk, n);
   }
   GMOD_CHECK_LAUNCH();
-  o.download((zd*)chiqout, nka, s);
+  fetch((zd*)chiqout, o, nka, s);
   GMOD_HIP(hipStreamSynchronize(s));
   GMOD_CATCH
 }
@@ -1459,7 +1475,7 @@ extern "C" void gen_green0_(gmod_z* Gk, const double* eig, const gmod_z* uni, co
   up(e, eig, (size_t)No * *Nk);
   up(u, (const zd*)uni, (size_t)No * No * *Nk);
   green0(G.p, e.p, u.p, *mu, *temp, *Nk, (int)*Nw, No, s);
-  G.download((zd*)Gk, n, s);
+  fetch((zd*)Gk, G, n, s);
   GMOD_HIP(hipStreamSynchronize(s));
   GMOD_CATCH
 }
@@ -1476,7 +1492,7 @@ extern "C" void gen_green_inv_(gmod_z* Gk, const gmod_z* self, const gmod_z* ham
   up(sg, (const zd*)self, n);
   up(h, (const zd*)hamk, (size_t)No * No * *Nk);
   green_inv(G.p, sg.p, h.p, *mu, *temp, *Nk, (int)*Nw, No, s);
-  G.download((zd*)Gk, n, s);
+  fetch((zd*)Gk, G, n, s);
   GMOD_HIP(hipStreamSynchronize(s));
   GMOD_CATCH
 }
@@ -1495,7 +1511,7 @@ extern "C" void getinv_(gmod_z* Gk, const int64_t* Nk, const int64_t* Nw, const 
   up(G, (const zd*)Gk, n);
   batched_inv(G.p, tot, No, err.p, s);
   check_err(err, s, "getinv");
-  G.download((zd*)Gk, n, s);
+  fetch((zd*)Gk, G, n, s);
   GMOD_HIP(hipStreamSynchronize(s));
   GMOD_CATCH
 }
@@ -1587,12 +1603,13 @@ extern "C" void get_chis_chic_soc(gmod_z* chic, gmod_z* chiszz, gmod_z* chispm, 
   DBuf<double> V;
   DBuf<int> err(1);
   err.zero(s);
-  up(a, (const zd*)chi, (size_t)NkNw * n * n);
+  const std::vector<zd> slice = static_slice((const zd*)chi, nk, NkNw, n);
+  up(a, slice.data(), slice.size());
   up(V, Vmat, (size_t)n * n);
-  rpa_solve(o.p, BatchLayout{1, nk}, a.p, BatchLayout{1, NkNw}, nk, n, V.p, 1.0, err.p, s);
+  rpa_solve(o.p, BatchLayout{1, nk}, a.p, BatchLayout{1, nk}, nk, n, V.p, 1.0, err.p, s);
   check_err(err, s, "get_chis_chic_soc");
   std::vector<zd> X(tot);
-  o.download(X.data(), tot, s);
+  fetch(X.data(), o, tot, s);
   GMOD_HIP(hipStreamSynchronize(s));
   auto sp = [&](int orb) { return slist[orb - 1]; };
   zd* cc = (zd*)chic;
@@ -1708,7 +1725,7 @@ extern "C" void mkfk_trs_soc_(gmod_z* fk, const gmod_z* Gk, const gmod_z* delta,
   up(sl, slh.data(), (size_t)No);
   up(inv, invh.data(), (size_t)No);
   anomalous_f_soc(F.p, G.p, D.p, iv.p, sg.p, sl.p, inv.p, nkall, nk, (int)nw, No, *gap_sym, s);
-  F.download((zd*)fk, nF, s);
+  fetch((zd*)fk, F, nF, s);
   GMOD_HIP(hipStreamSynchronize(s));
   GMOD_CATCH
 }
@@ -1861,8 +1878,8 @@ extern "C" void get_chi0sc_(gmod_z* Vsigma, gmod_z* Vdelta, const gmod_z* Gk, co
   if (ctx().precision >= 1) run(std::make_unique<ConvEngine<float>>(mesh, op));
   else run(std::make_unique<ConvEngine<double>>(mesh, op));
   sum_diff(cs.p, cc.p, (long)nC, s);
-  cs.download((zd*)Vsigma, nC, s);
-  cc.download((zd*)Vdelta, nC, s);
+  fetch((zd*)Vsigma, cs, nC, s);
+  fetch((zd*)Vdelta, cc, nC, s);
   GMOD_HIP(hipStreamSynchronize(s));
   GMOD_CATCH
 }
@@ -1888,8 +1905,8 @@ extern "C" void mkv_flex_nosoc_(gmod_z* Vdelta, gmod_z* Vsigma, const double* Sm
   up(C, Cmat, (size_t)n * n);
   sc_vertex(vs.p, vd.p, NkNw, BatchLayout{1, NkNw}, n, S.p, C.p, *sw_pair, err.p, s);
   check_err(err, s, "mkV_flex_nosoc");
-  vs.download((zd*)Vsigma, nC, s);
-  vd.download((zd*)Vdelta, nC, s);
+  fetch((zd*)Vsigma, vs, nC, s);
+  fetch((zd*)Vdelta, vd, nC, s);
   GMOD_HIP(hipStreamSynchronize(s));
   GMOD_CATCH
 }
@@ -1906,7 +1923,7 @@ extern "C" void mkfk_trs_nsoc_(gmod_z* fk, const gmod_z* Gk, const gmod_z* delta
   up(G, (const zd*)Gk, n);
   up(D, (const zd*)delta, n);
   anomalous_f(F.p, G.p, D.p, *Nk, (int)*Nw, No, s);
-  F.download((zd*)fk, n, s);
+  fetch((zd*)fk, F, n, s);
   GMOD_HIP(hipStreamSynchronize(s));
   GMOD_CATCH
 }
@@ -1929,7 +1946,7 @@ extern "C" void get_initial_delta_(gmod_z* delta, const double* init_delta, cons
   const size_t n = (size_t)*Nk * *Nw * No * No;
   DBuf<zd> D(n);
   initial_delta(D.p, init_delta, (const zd*)uni, mesh, No, *gap_sym, s);
-  D.download((zd*)delta, n, s);
+  fetch((zd*)delta, D, n, s);
   GMOD_HIP(hipStreamSynchronize(s));
   GMOD_CATCH
 }

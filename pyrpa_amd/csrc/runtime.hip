@@ -8,6 +8,7 @@
 
 #include "../../include/gmod.h"
 #include "gmod_common.h"
+#include "transfer.h"
 
 namespace gmod {
 
@@ -196,7 +197,11 @@ extern "C" int gmod_profile_read(double* out, int n) {
 }
 extern "C" double gmod_pool_bytes(void) { return pool_bytes(); }
 extern "C" void gmod_release_memory(void) {
-  try { pool().trim(); } catch (std::exception& e) { set_error(e.what()); }
+  try {
+    std::lock_guard<std::mutex> g(ctx().lock);
+    release_transfer_buffers();
+    pool().trim();
+  } catch (std::exception& e) { set_error(e.what()); }
 }
 
 // Device buffers for callers of the device-pointer entry points that hold no
