@@ -14,7 +14,8 @@
 // output scale, and stores.  Axes longer than 256 are split n = n1*n2 into two
 // passes (four-step): pass A = length-n1 transforms with the w_n^(k1*t2)
 // twiddle, pass B = length-n2 transforms with a transposing store.
-// Non-power-of-two lengths use a direct DFT from LDS.
+// Non-power-of-two lengths use a direct DFT from LDS, several outputs and
+// lines per thread.
 //
 // The first pass reads through a Load functor and the last pass writes through
 // a Store functor, so the irreducible -> full-grid scatter, the pointwise
@@ -81,9 +82,27 @@ template <typename R> struct GridStore {
   __device__ bool skip(unsigned) const { return false; }
 };
 
-template <typename R, bool POW2, class LD, class ST>
+// Direct DFT of the lines in LDS for a length that is no power of two: a
+// thread forms DFT_K outputs of DFT_L lines at once, so an element or a
+// twiddle read from LDS serves several products.  One output at a time read a
+// line element from LDS and a twiddle from global memory for each product and
+// waited for both in turn; a 29x29x1x92 transform took 267 us in FP64, now 49,
+// 44x44x1x162 377 -> 77, 12x12x1x1632 356 -> 75.  What remains is the chain of
+// n products per thread.  Every output is the sum over e = 0 .. n - 1 in turn.
+constexpr int DFT_K = 4, DFT_L = 2;
+// x w with the roundings written out (which product of a sum is rounded by
+// itself is the compiler's choice otherwise, instance by instance; an Arnoldi
+// iteration near its breakdown shows the difference)
+template <typename R> __device__ inline cpx<R> dft_mul(cpx<R> x, cpx<R> w) {
+  return {__builtin_elementwise_fma(x.re, w.re, -(x.im * w.im)), __builtin_elementwise_fma(x.im, w.re, x.re * w.im)};
+}
+
+// blockIdx.y: the item of a batch
+template <typename R, bool POW2, class LDB, class STB>
 __global__ void __launch_bounds__(FFT_THREADS)
-fft_pass_kernel(LD ld, ST st, PassArgs a, const cpx<R>* __restrict__ tw, const cpx<R>* __restrict__ tw4, R scale) {
+fft_pass_kernel(LDB ldb, STB stb, PassArgs a, const cpx<R>* __restrict__ tw, const cpx<R>* __restrict__ tw4, R scale) {
+  const typename BatchOf<LDB>::Item ld = BatchOf<LDB>::at(ldb, blockIdx.y);
+  const typename BatchOf<STB>::Item st = BatchOf<STB>::at(stb, blockIdx.y);
   extern __shared__ unsigned char smem_raw[];
   __shared__ unsigned l_spi[FFT_MAX_LINES], l_ti[FFT_MAX_LINES], l_spo[FFT_MAX_LINES], l_to[FFT_MAX_LINES],
       l_mid[FFT_MAX_LINES];
@@ -133,8 +152,59 @@ fft_pass_kernel(LD ld, ST st, PassArgs a, const cpx<R>* __restrict__ tw, const c
       }
     }
   }
+  if (!POW2) {
+    cpx<R>* ltw = lds + lines * a.pitch;
+    for (int i = tid; i < n; i += FFT_THREADS) ltw[i] = tw[i];
+    __syncthreads();
+    const int KG = (n + DFT_K - 1) / DFT_K, LG = (nl + DFT_L - 1) / DFT_L;
+    const bool along = a.out_elem == 1;  // lanes along the output's contiguous direction
+    for (int u = tid; u < KG * LG; u += FFT_THREADS) {
+      const int kg = along ? u % KG : u / LG, lg = along ? u / KG : u % LG;
+      int k[DFT_K], idx[DFT_K];
+      const cpx<R>* row[DFT_L];
+#pragma unroll
+      for (int i = 0; i < DFT_K; ++i) {
+        k[i] = kg + i * KG < n ? kg + i * KG : 0;
+        idx[i] = 0;
+      }
+#pragma unroll
+      for (int j = 0; j < DFT_L; ++j) row[j] = lds + (lg + j * LG < nl ? lg + j * LG : 0) * a.pitch;
+      cpx<R> acc[DFT_K][DFT_L];
+#pragma unroll
+      for (int i = 0; i < DFT_K; ++i)
+#pragma unroll
+        for (int j = 0; j < DFT_L; ++j) acc[i][j] = cpx<R>(0, 0);
+      for (int e = 0; e < n; ++e) {
+        cpx<R> x[DFT_L];
+#pragma unroll
+        for (int j = 0; j < DFT_L; ++j) x[j] = row[j][e];
+#pragma unroll
+        for (int i = 0; i < DFT_K; ++i) {
+          const cpx<R> w = ltw[idx[i]];
+#pragma unroll
+          for (int j = 0; j < DFT_L; ++j) acc[i][j] += dft_mul(x[j], w);
+          idx[i] += k[i];
+          if (idx[i] >= n) idx[i] -= n;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < DFT_K; ++i)
+#pragma unroll
+        for (int j = 0; j < DFT_L; ++j) {
+          const int ko = kg + i * KG, L = lg + j * LG;
+          if (ko >= n || L >= nl) continue;
+          cpx<R> v = acc[i][j];
+          if (a.twn) {
+            const unsigned ti = (unsigned)ko * l_mid[L];
+            v = dft_mul(v, tw4[(a.twn & (a.twn - 1)) == 0 ? (ti & (unsigned)(a.twn - 1)) : ti % (unsigned)a.twn]);
+          }
+          st(l_spo[L] + ko * dso, l_to[L] + ko * dto, v * scale);
+        }
+    }
+    return;
+  }
   __syncthreads();
-  if (POW2) {
+  {
     int lh = 0;
     if (a.logn & 1) {  // one radix-2 stage (h = 1, twiddle 1)
       const int half = n >> 1;
@@ -171,18 +241,7 @@ fft_pass_kernel(LD ld, ST st, PassArgs a, const cpx<R>* __restrict__ tw, const c
       __syncthreads();
     }
   }
-  auto value = [&](int L, int k) -> cpx<R> {
-    if (POW2) return lds[L * a.pitch + k];
-    cpx<R> acc(0, 0);
-    const cpx<R>* row = lds + L * a.pitch;
-    int idx = 0;
-    for (int e = 0; e < n; ++e) {
-      acc += row[e] * tw[idx];
-      idx += k;
-      if (idx >= n) idx -= n;
-    }
-    return acc;
-  };
+  auto value = [&](int L, int k) -> cpx<R> { return lds[L * a.pitch + k]; };
   // ---- store
   if (a.out_elem == 1) {
     for (int idx = tid; idx < total; idx += FFT_THREADS) {
@@ -298,7 +357,7 @@ class FFTPlan {
 
  private:
   template <class LD, class ST>
-  void launch(const FFTPassDesc& p, LD ld, ST st, const cpx<R>* tw, R sc, hipStream_t s) const;
+  void launch(const FFTPassDesc& p, LD ld, ST st, int n, const cpx<R>* tw, R sc, hipStream_t s) const;
   template <class LD, class ST>
   void launch_box(int sg, int i, LD ld, ST st, int n, int sign, R sc, hipStream_t s) const;
   // pass i runs with the small boxes: the launch would leave CUs idle, or
@@ -364,11 +423,11 @@ inline int fft_ilog2(long n) { int l = 0; while ((1L << l) < n) ++l; return l; }
 
 template <typename R>
 template <class LD, class ST>
-void FFTPlan<R>::launch(const FFTPassDesc& p, LD ld, ST st, const cpx<R>* tw, R sc, hipStream_t s) const {
+void FFTPlan<R>::launch(const FFTPassDesc& p, LD ld, ST st, int n, const cpx<R>* tw, R sc, hipStream_t s) const {
+  const bool pow2 = fft_is_pow2(p.n);
   PassArgs a;
   a.n = p.n;
-  a.logn = fft_is_pow2(p.n) ? fft_ilog2(p.n) : 0;
-  a.lines = p.lines;
+  a.logn = pow2 ? fft_ilog2(p.n) : 0;
   a.pitch = p.n + 1;
   a.n_inner = (unsigned)p.n_inner;
   a.n_mid = (unsigned)p.n_mid;
@@ -377,16 +436,26 @@ void FFTPlan<R>::launch(const FFTPassDesc& p, LD ld, ST st, const cpx<R>* tw, R 
   a.out_mid = (unsigned)p.out_mid; a.out_outer = (unsigned)p.out_outer; a.out_elem = (unsigned)p.out_elem;
   a.S = S_;
   a.twn = p.twn;
-  a.loglines = fft_is_pow2(p.lines) ? fft_ilog2(p.lines) : -1;
-  const long blocks = (a.total_lines + p.lines - 1) / p.lines;
-  const size_t shm = (size_t)p.lines * a.pitch * sizeof(cpx<R>);
-  ProfScope ps(sizeof(R) == 4 ? PROF_FFT32 : PROF_FFT, pass_bytes<R>(ld, st, (double)size()), s);
-  if (fft_is_pow2(p.n))
-    hipLaunchKernelGGL((fft_pass_kernel<R, true, LD, ST>), dim3((unsigned)blocks), dim3(FFT_THREADS), shm, s, ld, st,
-                       a, tw + p.tw_off, tw + p.tw4_off, sc);
+  // lines of a work-group: what the LDS budget takes (the direct DFT's
+  // twiddles beside them), fewer (at least 8: a cache line of a strided
+  // axis) while that leaves fewer than four work-groups per CU
+  a.lines = pow2 ? p.lines : std::max(1, std::min<int>(p.lines, (p.lines * p.n - p.n) / a.pitch));
+  int want = 8;
+  while ((long)want * 4 * persist_ < (long)a.total_lines * n) want *= 2;
+  a.lines = std::min(a.lines, want);
+  a.loglines = fft_is_pow2(a.lines) ? fft_ilog2(a.lines) : -1;
+  const long blocks = (a.total_lines + a.lines - 1) / a.lines;
+  const size_t shm = ((size_t)a.lines * a.pitch + (pow2 ? 0 : p.n)) * sizeof(cpx<R>);
+  ProfScope ps(sizeof(R) == 4 ? PROF_FFT32 : PROF_FFT,
+               n * pass_bytes<R>(BatchOf<LD>::at(ld, 0), BatchOf<ST>::at(st, 0), (double)size()), s);
+  if (n > 65535) throw Error("FFT batch of more than 65535 transforms");
+  const dim3 g((unsigned)blocks, (unsigned)n);
+  if (pow2)
+    hipLaunchKernelGGL((fft_pass_kernel<R, true, LD, ST>), g, dim3(FFT_THREADS), shm, s, ld, st, a, tw + p.tw_off,
+                       tw + p.tw4_off, sc);
   else
-    hipLaunchKernelGGL((fft_pass_kernel<R, false, LD, ST>), dim3((unsigned)blocks), dim3(FFT_THREADS), shm, s, ld,
-                       st, a, tw + p.tw_off, tw + p.tw4_off, sc);
+    hipLaunchKernelGGL((fft_pass_kernel<R, false, LD, ST>), g, dim3(FFT_THREADS), shm, s, ld, st, a, tw + p.tw_off,
+                       tw + p.tw4_off, sc);
   GMOD_CHECK_LAUNCH();
 }
 
@@ -469,20 +538,26 @@ void FFTPlan<R>::exec_batch(LD ld, ST st, cpx<R>* buf, int n, cpx<R>* tmp, int s
   const std::vector<FFTPassDesc>& ps = sign < 0 ? fwd_ : bwd_;
   const int np = (int)ps.size();
   if (np == 0) throw Error("FFT with nothing to transform");
-  for (int it = 0; it < n; ++it) {
-    const typename BatchOf<LD>::Item li = BatchOf<LD>::at(ld, it);
-    const typename BatchOf<ST>::Item si = BatchOf<ST>::at(st, it);
-    cpx<R>* bb = buf + (long)it * size();
-    auto buf_of = [&](int which) { return which ? tmp : bb; };
-    for (int i = 0; i < np; ++i) {
-      const FFTPassDesc& p = ps[i];
-      const R sc = (i == np - 1) ? scale : (R)1;
-      const bool first = i == 0, last = i == np - 1;
-      if (first && last) launch(p, li, si, tw, sc, s);
-      else if (first) launch(p, li, GridStore<R>{buf_of(p.dst), S_}, tw, sc, s);
-      else if (last) launch(p, GridLoad<R>{buf_of(p.src), S_}, si, tw, sc, s);
-      else launch(p, GridLoad<R>{buf_of(p.src), S_}, GridStore<R>{buf_of(p.dst), S_}, tw, sc, s);
-    }
+  bool scratch = false;
+  for (const FFTPassDesc& p : ps) scratch = scratch || p.src != 0 || p.dst != 0;
+  // a second buffer for every item of a batch (its block returns to the pool
+  // in stream order)
+  DBuf<cpx<R>> many;
+  if (scratch && n > 1) {
+    many.alloc((size_t)n * size());
+    tmp = many.p;
+  }
+  auto buf_of = [&](int which) { return which ? tmp : buf; };
+  for (int i = 0; i < np; ++i) {
+    const FFTPassDesc& p = ps[i];
+    const R sc = (i == np - 1) ? scale : (R)1;
+    const GridLoad<R> gl{buf_of(p.src), S_, size()};
+    const GridStore<R> gs{buf_of(p.dst), S_, size()};
+    const bool first = i == 0, last = i == np - 1;
+    if (first && last) launch(p, ld, st, n, tw, sc, s);
+    else if (first) launch(p, ld, gs, n, tw, sc, s);
+    else if (last) launch(p, gl, st, n, tw, sc, s);
+    else launch(p, gl, gs, n, tw, sc, s);
   }
 }
 

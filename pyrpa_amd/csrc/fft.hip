@@ -574,8 +574,8 @@ bool FFTPlan<R>::small_pass(int sg, int i, long n) const {
 template <typename R>
 int FFTPlan<R>::batch_items(int n) const {
   const long nb = std::max<long>(boxes(), 1), bytes = size() * (long)sizeof(cpx<R>);
-  // four rounds over the CUs (per-axis passes run item by item)
-  const long rounds = box_.ok ? (4 * persist_ + nb - 1) / nb : 1;
+  // four rounds over the CUs (per-axis passes: by their elements)
+  const long rounds = box_.ok ? (4 * persist_ + nb - 1) / nb : 1 + (4 * persist_ * 2048) / size();
   const long cached = (96L << 20) / bytes, room = std::max<long>(1, (2L << 30) / bytes);
   return (int)std::max<long>(1, std::min<long>(n, std::min(room, std::max(rounds, cached))));
 }

@@ -1,7 +1,7 @@
 """Batched transform passes against the oracle where their launches differ:
 grids of a single box, few boxes (quarter-size boxes, tiled and not), boxes
 whose element count is no multiple of the work-group (the untiled kernel),
-lengths the box passes do not cover (a prime above 7: item by item through
+lengths the box passes do not cover (a prime above 7: the direct DFT of
 the per-axis passes), one item and many, a mesh with odd lengths, and the
 spinful functors.  FP64: 1e-11 of the largest element (the transforms' rounding
 is a few log2 N ulp); FP32 transforms: 2^-24 log2 N times a small factor."""
