@@ -487,20 +487,21 @@ __device__ __forceinline__ long long gj_row_max(long long k) {
 // formed right after column k + 1 of its row is updated.  At the end the lane
 // that was pivot of column k holds row k of M^-1 (xrow = k), entry j in
 // column piv[j] (the pivot row of column j).  Returns true if a pivot was
-// zero or not finite.
-template <int N>
+// zero or (unless ZERO_ONLY) not finite.  Lanes r >= N of a smaller matrix are
+// never a pivot.
+template <int N, bool ZERO_ONLY = false>
 __device__ __forceinline__ bool gj_invert(zd (&mrow)[N], int r, zd* prow, int* piv, int& xrow) {
-  bool used = false;
+  bool used = N < 16 && r >= N;
   bool singular = false;
   zd dpiv(1.0, 0);
-  long long key = gj_key(abs1(mrow[0]), r);  // my candidate for the next column
+  long long key = gj_key(used ? -1.0 : abs1(mrow[0]), r);  // my candidate for the next column
 #pragma unroll
   for (int k = 0; k < N; ++k) {
     wave_sync();
     const long long kb = gj_row_max(key);
     const int pr = 15 - (int)(kb & 0xF);
     const double best = __longlong_as_double(kb & ~0xFLL);
-    singular = singular || !(best > 0.0 && best < 1e300);  // zero, or a clamped inf / NaN
+    singular = singular || !(best > 0.0 && (ZERO_ONLY || best < 1e300));  // zero, or a clamped inf / NaN
     if (r == pr) {
 #pragma unroll
       for (int j = 0; j < N; ++j) prow[j] = mrow[j];
@@ -736,6 +737,174 @@ k_vertex_gj(const zd* chi_in, zd* chi_out, long batch, long es, const VSparse* _
   }
 }
 
+// The row-per-lane Gauss-Jordan inversion where k_vertex_gj does not apply:
+// KIND 0, the FLEX vertex (mode 0) of Nchi = N < 16, both systems of a matrix
+// in two 16-lane groups; KIND 1, the spinful vertex of Nchi = 16,
+//   -V + V (I + chi0 V)^-1 chi0 V = -V (I + chi0 V)^-1,
+// one system (V in place of S), four matrices per wavefront.  Both bound by
+// the chain of N pivot steps.  At N = 9 seven of sixteen lanes idle, and it is
+// faster than a column per lane all the same: a step exchanges one row within
+// a wavefront, the LU waits for the whole work-group twice.  3 orbitals,
+// 27x27x5 x 90: 1295 us by columns, 719 by rows (registers for three or four
+// waves per SIMD spill: 1173, 1413); spinful 2 orbitals, 16x16 x 128: 740 us
+// with a wavefront per matrix in LDS, 87 by rows.
+template <int N, int KIND>
+__global__ void __launch_bounds__(64 * GJ_WAVES) __attribute__((amdgpu_waves_per_eu(2)))
+k_vertex_rows(const zd* chi_in, zd* chi_out, long batch, long es, const VSparse* __restrict__ spg,
+              const double* __restrict__ Sd, const double* __restrict__ Cd, double thr, int* err) {
+  static_assert(N <= 16, "a 16-lane group per system");
+  constexpr int NT = 64 * GJ_WAVES;
+  constexpr int NN = N * N, MS = NN + 1;            // padded as in k_vertex_gj
+  constexpr int MAT = GJ_WAVES * (KIND == 0 ? 2 : 4);  // matrices per block
+  constexpr int PER = (MAT * NN + NT - 1) / NT;
+  __shared__ VSparse sp;
+  __shared__ double2 Abuf_[MAT * MS];                 // chi0, later X or the inverse
+  __shared__ double2 Vbuf_[KIND == 0 ? MAT * MS : 1];  // A W, then the vertex
+  constexpr int PROW = 2 * N + 1;
+  __shared__ double2 Prow_[GJ_WAVES * 4 * PROW];
+  __shared__ int Piv_[GJ_WAVES * 4 * N];
+  zd* Abuf = reinterpret_cast<zd*>(Abuf_);
+  zd* Vbuf = reinterpret_cast<zd*>(Vbuf_);
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  {
+    const int* src = reinterpret_cast<const int*>(spg);
+    int* dst = reinterpret_cast<int*>(&sp);
+    for (int i = tid; i < (int)(sizeof(VSparse) / sizeof(int)); i += NT) dst[i] = src[i];
+  }
+  const int g = lane >> 4, r = lane & 15;
+  const int mloc = KIND == 0 ? wave * 2 + (g >> 1) : wave * 4 + g;  // matrix of my group within the block
+  const int sys = KIND == 0 ? g & 1 : 0;                            // 0: S (or V) system, 1: C system
+  zd* A = Abuf + mloc * MS;
+  zd* prow = reinterpret_cast<zd*>(Prow_) + (wave * 4 + g) * PROW;
+  int* piv = Piv_ + (wave * 4 + g) * N;
+  const int ra = r < N ? r : 0;
+  zd nxt[PER];
+  auto fetch = [&](long b0) {  // element i: matrix i % MAT, entry i / MAT
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int i = tid + u * NT;
+      const int m = i % MAT, e = i / MAT;
+      nxt[u] = chi_in[b0 + m < batch && e < NN ? b0 + m + (long)e * es : 0];
+    }
+  };
+  __syncthreads();
+  const long bstep = (long)gridDim.x * MAT;
+  if ((long)blockIdx.x * MAT < batch) fetch((long)blockIdx.x * MAT);
+  for (long b0 = (long)blockIdx.x * MAT; b0 < batch; b0 += bstep) {
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int i = tid + u * NT;
+      const int m = i % MAT, e = i / MAT;
+      zd v = b0 + m < batch ? nxt[u] : zd(0, 0);
+      if (thr > 0.0) {
+        if (fabs(v.re) < thr) v.re = 0.0;
+        if (fabs(v.im) < thr) v.im = 0.0;
+      }
+      if (e < NN) Abuf[m * MS + e] = v;
+    }
+    __syncthreads();
+    if (b0 + bstep < batch) fetch(b0 + bstep);
+    zd vinit[KIND == 0 ? PER : 1];
+    if (KIND == 0) {  // V = st - 0.25 W A W, block-wide
+      for (int i = tid; i < MAT * NN; i += NT) {
+        const int m = i / NN, e = i % NN, p = e % N, q = e / N;
+        zd acc(0, 0);
+#pragma unroll
+        for (int t = 0; t < VW_NZ; ++t) acc += Abuf[m * MS + p + N * sp.idx[2][q][t]] * sp.val[2][q][t];
+        Vbuf[m * MS + e] = acc;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < PER; ++u) {
+        const int i = tid + u * NT;
+        if (i >= MAT * NN) continue;
+        const int m = i / NN, e = i % NN, p = e % N, q = e / N;
+        zd acc(0, 0);
+#pragma unroll
+        for (int t = 0; t < VW_NZ; ++t) acc += Vbuf[m * MS + sp.idx[2][p][t] + N * q] * sp.val[2][p][t];
+        vinit[u] = zd(1.5 * Sd[e] - 0.5 * Cd[e], 0) - acc * 0.25;
+      }
+    }
+    // ---- my row of M = I -+ A K
+    zd mrow[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      zd acc(0, 0);
+#pragma unroll
+      for (int t = 0; t < VW_NZ; ++t) acc += A[ra + N * sp.idx[sys][j][t]] * sp.val[sys][j][t];
+      mrow[j] = KIND == 0 && sys == 0 ? zd(0, 0) - acc : acc;
+      if (j == r) mrow[j] += zd(1.0, 0);
+    }
+    __syncthreads();  // all reads of A and of A W are complete
+    if (KIND == 0) {
+#pragma unroll
+      for (int u = 0; u < PER; ++u) {
+        const int i = tid + u * NT;
+        if (i < MAT * NN) Vbuf[(i / NN) * MS + i % NN] = vinit[u];
+      }
+    }
+    int xrow = 0;
+    const bool singular = gj_invert<N, true>(mrow, r, prow, piv, xrow);
+    if (singular && r == 0 && b0 + mloc < batch) atomicOr(err, 1);
+    // ---- KIND 0: V += 1.5 S X_s, then V += 0.5 C X_c; KIND 1: -V M^-1
+#pragma unroll
+    for (int pass = 0; pass < (KIND == 0 ? 2 : 1); ++pass) {
+      if (sys == pass && r < N) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          const int q = piv[j];
+          zd x = mrow[j];
+          if (KIND == 0) {  // X = M^-1 - I for the S system, I - M^-1 for the C system
+            if (q == xrow) x -= zd(1.0, 0);
+            if (pass == 1) x = zd(0, 0) - x;
+          }
+          A[xrow + N * q] = x;
+        }
+      }
+      __syncthreads();
+      if (KIND == 0) {
+        for (int i = tid; i < MAT * NN; i += NT) {
+          const int m = i / NN, e = i % NN, p = e % N, q = e / N;
+          zd acc(0, 0);
+#pragma unroll
+          for (int t = 0; t < VW_NZ; ++t)
+            acc += Abuf[m * MS + sp.idx[pass][p][t] + N * q] * sp.val[pass][p][t];
+          Vbuf[m * MS + e] += acc * (pass == 0 ? 1.5 : 0.5);
+        }
+        __syncthreads();
+      }
+    }
+    for (int i = tid; i < MAT * NN; i += NT) {
+      const int m = i % MAT, e = i / MAT;
+      if (b0 + m >= batch) continue;
+      zd v;
+      if (KIND == 0) {
+        v = Vbuf[m * MS + e];
+      } else {
+        const int p = e % N, q = e / N;
+        v = zd(0, 0);
+#pragma unroll
+        for (int t = 0; t < VW_NZ; ++t) v -= Abuf[m * MS + sp.idx[0][p][t] + N * q] * sp.val[0][p][t];
+      }
+      chi_out[b0 + m + (long)e * es] = v;
+    }
+    __syncthreads();
+  }
+}
+
+template <int N, int KIND>
+static void launch_vertex_rows(const zd* in, zd* out, long batch, long es, const VSparse& sp, const double* S,
+                               const double* C, double thr, int* err, hipStream_t s) {
+  DBuf<VSparse> spd(1);
+  spd.upload(&sp, 1, s);
+  const long mat = GJ_WAVES * (KIND == 0 ? 2 : 4);
+  const unsigned grid = (unsigned)std::min<long>((batch + mat - 1) / mat, 256L * 32);
+  hipLaunchKernelGGL((k_vertex_rows<N, KIND>), dim3(grid), dim3(64 * GJ_WAVES), 0, s, in, out, batch, es, spd.p, S,
+                     C, thr, err);
+  GMOD_CHECK_LAUNCH();
+  GMOD_HIP(hipStreamSynchronize(s));  // sp is the caller's
+}
+
 // The vertices of the superconducting loop (ffeliash.f90:386-457) for
 // Nchi = 16 with sparse S, C: the Gauss-Jordan scheme of k_vertex_gj with the
 // S system solved on chi0_S and the C system on chi0_C (read from vs and vd),
@@ -962,6 +1131,13 @@ void rpa_vertex(zd* chi, long batch, BatchLayout L, int n, const double* S, cons
                 hipStream_t s) {
   if (batch <= 0) return;
   if (vertex_gj(chi, chi, batch, L, n, S, C, mode, 0.0, nullptr, nullptr, err, s)) return;
+  // 3 orbitals, sparse S and C: the FLEX vertex by rows (719 us, by columns
+  // 1295).  The pairing vertices stay with the LU: they are formed once per
+  // solve, and the Arnoldi solver of the gap equation shows a change of rounding
+  if (VSparse sp; L.bs == 1 && n == 9 && mode == 0 && vertex_sparse(S, C, n, sp, s)) {
+    launch_vertex_rows<9, 0>(chi, chi, batch, L.es, sp, S, C, 0.0, err, s);
+    return;
+  }
   if (L.bs == 1) {
     switch (n) {
       case 1: launch_vertex_reg<1>(chi, batch, L.es, S, C, mode, err, s); return;
@@ -1052,6 +1228,10 @@ k_soc_vertex(const zd* chi_in, zd* out, BatchLayout L, long batch, int n, const 
 void soc_vertex(const zd* chi_in, zd* out, long batch, BatchLayout L, int n, const double* V, double thr, int* err,
                 hipStream_t s) {
   if (batch <= 0) return;
+  if (VSparse sp; L.bs == 1 && n == 16 && vertex_sparse(V, V, n, sp, s)) {
+    launch_vertex_rows<16, 1>(chi_in, out, batch, L.es, sp, V, V, thr, err, s);
+    return;
+  }
   const size_t shm = 3 * (size_t)n * n * sizeof(zd);
   if (shm <= 160 * 1024) {
     const unsigned grid = (unsigned)std::min<long>(batch, 256L * 64);
