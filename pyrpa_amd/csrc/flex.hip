@@ -310,6 +310,12 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
     filling_parts_cp(parts, cpoly.p, eig_d.p, rmu, T, Nk, (int)Nw, No, s);
     return (parts[0] + 2.0 * T * parts[1]) / (double)Nk;
   };
+  auto get_rn2 = [&](double mu0, double mu1, double& rn0, double& rn1) {
+    double parts[4];
+    filling_parts_cp2(parts, cpoly.p, eig_d.p, mu0, mu1, T, Nk, (int)Nw, No, s);
+    rn0 = (parts[0] + 2.0 * T * parts[1]) / (double)Nk;
+    rn1 = (parts[2] + 2.0 * T * parts[3]) / (double)Nk;
+  };
   const double rfill = A.rfill;
   auto renew_mu = [&]() {
     if (cpoly.n != (size_t)(NkNw * No)) cpoly.alloc((size_t)NkNw * No);
@@ -321,16 +327,16 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
     double rnS = 0, rnL = 0, muS = 0, muL = 0;
     bool found = false;
     if (bracket_valid) {
-      rnS = get_rn(muS_cache);
-      rnL = get_rn(muL_cache);
+      get_rn2(muS_cache, muL_cache, rnS, rnL);
       if (rnS < rfill && rnL > rfill) { muS = muS_cache; muL = muL_cache; found = true; }
     }
     if (!found) {
       muL = mu + dmu;
       muS = mu - dmu;
+      get_rn2(muS, muL, rnS, rnL);
       for (int it = 1; it <= 100; ++it) {
         mu = muL;
-        rnL = get_rn(mu);
+        if (it > 1) rnL = get_rn(mu);
         if (rnL < rfill) {
           if (std::fabs(rfill - rnL) > 0.5) muL += 1.0;
           else if (std::fabs(rfill - rnL) > dmu) muL += 0.5;
@@ -340,7 +346,7 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
       }
       for (int it = 1; it <= 100; ++it) {
         mu = muS;
-        rnS = get_rn(mu);
+        if (it > 1) rnS = get_rn(mu);
         if (rnS > rfill) {
           if (std::fabs(rnS - rfill) > 0.5) muS -= 1.0;
           else if (std::fabs(rnS - rfill) > dmu) muS -= 0.5;
@@ -387,9 +393,8 @@ static void mkself_driver(const FlexIn& A, zd* sig_out, double* mu_out, bool mix
     }
     if (rnL == rnS) mu = (muS + muL) * 0.5;
     else mu = (muS * rnL - muL * rnS) / (rnL - rnS);
-    double fill = get_rn(mu);
     mu_old = mu;
-    if (verbose) printf("mu  =%8.4f filling =%8.4f\n", mu, fill);
+    if (verbose) printf("mu  =%8.4f filling =%8.4f\n", mu, get_rn(mu));
   };
 
   // the reference of the increment iterations: the current iterate, whose

@@ -52,6 +52,9 @@ void dyson(zd* G, const zd* sigma, const zd* hamk, double mu, double temp, long 
 void filling_charpoly(zd* coef, const zd* sigma, const zd* hamk, long Nk, int Nw, int No, hipStream_t s);
 void filling_parts_cp(double out[2], const zd* coef, const double* eig, double rmu, double temp, long Nk, int Nw,
                       int No, hipStream_t s);
+// the same at two chemical potentials: out[0..1] at mu0, out[2..3] at mu1
+void filling_parts_cp2(double out[4], const zd* coef, const double* eig, double mu0, double mu1, double temp, long Nk,
+                       int Nw, int No, hipStream_t s);
 // G0 (fself.f90:1-41)
 void green0(zd* G, const double* eig, const zd* uni, double mu, double temp, long Nk, int Nw, int No,
             hipStream_t s);

@@ -1751,34 +1751,55 @@ __global__ void __launch_bounds__(128) k_charpoly(zd* coef, const zd* sig, const
   }
 }
 
-// n(mu) pieces from the characteristic polynomials (see k_charpoly), summed
-// by the host from pinned memory (latency-bound: with a copy of the partial
-// sums a trial mu took 24 us at 1 orbital, 32x32 x 256)
+// n(mu) pieces of element (k, j) from the characteristic polynomials (see
+// k_charpoly): r[1] += Re Tr (G - G0), r[0] += the Fermi functions (once per k)
+template <int NO>
+__device__ __forceinline__ void filling_add(double* r, const zd* coef, const double* eig, double rmu, double temp,
+                                            long e, long Nk, long tot) {
+  const long k = e % Nk;
+  const long j = e / Nk;
+  const zd z(rmu, (double)(2 * j + 1) * PI_D * temp);
+  zd p(1.0, 0), dp(0, 0);  // Horner for p and p'
+#pragma unroll
+  for (int i = 0; i < NO; ++i) {
+    dp = dp * z + p;
+    p = p * z + coef[e + tot * i];
+  }
+  double d = (dp / p).re;
+#pragma unroll
+  for (int n = 0; n < NO; ++n) d -= (zd(1.0, 0) / (z - zd(eig[n + NO * k], 0))).re;
+  r[1] += d;
+  if (j == 0) {
+#pragma unroll
+    for (int n = 0; n < NO; ++n) r[0] += 0.5 * (1.0 - tanh(0.5 * (eig[n + NO * k] - rmu) / temp));
+  }
+}
+
+// n(mu), summed by the host from pinned memory (latency-bound: with a copy of
+// the partial sums a trial mu took 24 us at 1 orbital, 32x32 x 256)
 template <int NO>
 __global__ void __launch_bounds__(RED_TPB) k_filling_cp(const zd* coef, const double* eig, double rmu, double temp,
                                                         long Nk, int Nw, double* part) {
   const long tot = Nk * (long)Nw;
   double r[2] = {0.0, 0.0};
-  for (long e = blockIdx.x * (long)RED_TPB + threadIdx.x; e < tot; e += (long)gridDim.x * RED_TPB) {
-    const long k = e % Nk;
-    const long j = e / Nk;
-    const zd z(rmu, (double)(2 * j + 1) * PI_D * temp);
-    zd p(1.0, 0), dp(0, 0);  // Horner for p and p'
-#pragma unroll
-    for (int i = 0; i < NO; ++i) {
-      dp = dp * z + p;
-      p = p * z + coef[e + tot * i];
-    }
-    double d = (dp / p).re;
-#pragma unroll
-    for (int n = 0; n < NO; ++n) d -= (zd(1.0, 0) / (z - zd(eig[n + NO * k], 0))).re;
-    r[1] += d;
-    if (j == 0) {
-#pragma unroll
-      for (int n = 0; n < NO; ++n) r[0] += 0.5 * (1.0 - tanh(0.5 * (eig[n + NO * k] - rmu) / temp));
-    }
-  }
+  for (long e = blockIdx.x * (long)RED_TPB + threadIdx.x; e < tot; e += (long)gridDim.x * RED_TPB)
+    filling_add<NO>(r, coef, eig, rmu, temp, e, Nk, tot);
   put_partial<RedSum, 2>(r, blockIdx.x, part);
+}
+
+// the two ends of a bracket in one launch: a trial mu of a small mesh is
+// mostly launch and wait (12 us, the kernel 5): one launch instead of two here
+// and no evaluation only to print it, 1 orbital 32x32 x 256 21.1 -> 20.3 ms
+template <int NO>
+__global__ void __launch_bounds__(RED_TPB) k_filling_cp2(const zd* coef, const double* eig, double mu0, double mu1,
+                                                         double temp, long Nk, int Nw, double* part) {
+  const long tot = Nk * (long)Nw;
+  double r[4] = {0.0, 0.0, 0.0, 0.0};
+  for (long e = blockIdx.x * (long)RED_TPB + threadIdx.x; e < tot; e += (long)gridDim.x * RED_TPB) {
+    filling_add<NO>(r, coef, eig, mu0, temp, e, Nk, tot);
+    filling_add<NO>(r + 2, coef, eig, mu1, temp, e, Nk, tot);
+  }
+  put_partial<RedSum, 4>(r, blockIdx.x, part);
 }
 
 template <int NO>
@@ -1983,6 +2004,15 @@ void filling_parts_cp(double out[2], const zd* coef, const double* eig, double r
   GMOD_CHECK_LAUNCH();
   GMOD_HIP(hipStreamSynchronize(s));
   for (int c = 0; c < 2; ++c) out[c] = sum_partials(ctx().pin, nb, 2, c);
+}
+
+void filling_parts_cp2(double out[4], const zd* coef, const double* eig, double mu0, double mu1, double temp, long Nk,
+                       int Nw, int No, hipStream_t s) {
+  const int nb = red_blocks(Nk * (long)Nw);
+  LAUNCH_NO(No, k_filling_cp2, dim3(nb), dim3(RED_TPB), coef, eig, mu0, mu1, temp, Nk, Nw, ctx().pin);
+  GMOD_CHECK_LAUNCH();
+  GMOD_HIP(hipStreamSynchronize(s));
+  for (int c = 0; c < 4; ++c) out[c] = sum_partials(ctx().pin, nb, 4, c);
 }
 
 void green0(zd* G, const double* eig, const zd* uni, double mu, double temp, long Nk, int Nw, int No,
