@@ -473,33 +473,6 @@ struct ProductBatch {
   }
 };
 
-// G_ab(current) - G_ab(reference) on the full grid, formed in FP64 before
-// the conversion to the grid precision (increments of the bilinear bubble)
-template <typename R>
-struct GreenDiffLoad {
-  GreenLoad<double> cur, ref;  // on one mesh: one key serves both
-  using Key = typename GreenLoad<double>::Key;
-  __device__ Key key(unsigned sp) const { return cur.key(sp); }
-  __device__ cpx<R> value(Key q, unsigned sp, unsigned t) const {
-    return cpx<R>(cur.value(q, sp, t) - ref.value(q, sp, t));
-  }
-  __device__ cpx<R> operator()(unsigned sp, unsigned t) const { return value(key(sp), sp, t); }
-  __host__ double algo_bytes(double N) const { return cur.algo_bytes(N) + ref.algo_bytes(N); }
-};
-
-// V(current) - V(reference): the static nu->inf slot cancels
-template <typename R>
-struct BosonDiffLoad {
-  BosonLoad<double> cur, ref;
-  using Key = typename BosonLoad<double>::Key;
-  __device__ Key key(unsigned sp) const { return cur.key(sp); }
-  __device__ cpx<R> value(Key q, unsigned sp, unsigned t) const {
-    return cpx<R>(cur.value(q, sp, t) - ref.value(q, sp, t));
-  }
-  __device__ cpx<R> operator()(unsigned sp, unsigned t) const { return value(key(sp), sp, t); }
-  __host__ double algo_bytes(double N) const { return cur.algo_bytes(N) + ref.algo_bytes(N); }
-};
-
 template <typename R>
 struct TauRefDiffLoad {
   TauRefLoad<double> cur, ref;
@@ -522,21 +495,6 @@ struct IncProductLoad {
   int nterm;
   MeshDev m;
   int bmir = 0;  // 1: every Br, Bd is a mirrored grid (all revt = 1) read at (r, t)
-  template <int N>
-  __host__ IncProductLoad<R, N> fixed() const {
-    IncProductLoad<R, N> p{};
-    for (int i = 0; i < INC_MAXT; ++i) {
-      p.Ar[i] = Ar[i]; p.Ad[i] = Ad[i]; p.Br[i] = Br[i]; p.Bd[i] = Bd[i]; p.coef[i] = coef[i]; p.revt[i] = revt[i];
-    }
-    p.nterm = nterm;
-    p.m = m;
-    p.bmir = bmir;
-    return p;
-  }
-  __host__ void add(const cpx<R>* ar, const cpx<R>* ad, const cpx<R>* br, const cpx<R>* bd, R c, int rt) {
-    if (nterm >= INC_MAXT) throw Error("too many increment terms");
-    Ar[nterm] = ar; Ad[nterm] = ad; Br[nterm] = br; Bd[nterm] = bd; coef[nterm] = c; revt[nterm] = rt; ++nterm;
-  }
   using Key = unsigned;  // spatial index of -r (no load with mirrored B)
   __device__ Key key(unsigned sp) const { return bmir ? sp : (unsigned)m.rev[sp]; }
   __device__ cpx<R> operator()(unsigned sp, unsigned t) const { return value(key(sp), sp, t); }
@@ -881,8 +839,6 @@ void copy(zd* dst, const zd* src, long n, hipStream_t s);
 void lincomb(zd* y, const zd* a, double ca, const zd* b, double cb, long n, hipStream_t s);  // y = ca a + cb b
 void threshold_copy(zd* dst, const zd* src, long n, double eps, hipStream_t s);              // dst = thr(src)
 void diff_to_f32(cpx<float>* dst, const zd* a, const zd* b, long n, hipStream_t s);          // dst = (float)(a - b)
-template <typename R>
-void add_inplace(cpx<R>* y, const cpx<R>* x, long n, hipStream_t s);  // y += x
 
 // y = x f;  y = sum_i c_i (x + idx_i stride)
 void scale_copy(zd* y, const zd* x, double f, long n, hipStream_t s);

@@ -438,17 +438,6 @@ void diff_to_f32(cpx<float>* dst, const zd* a, const zd* b, long n, hipStream_t 
   GMOD_CHECK_LAUNCH();
 }
 
-template <typename R>
-__global__ void k_add_inplace(cpx<R>* y, const cpx<R>* x, long n) {
-  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x)
-    y[e] = y[e] + x[e];
-}
-template <typename R>
-void add_inplace(cpx<R>* y, const cpx<R>* x, long n, hipStream_t s) {
-  hipLaunchKernelGGL(k_add_inplace<R>, dim3(nblocks(n)), dim3(TPB), 0, s, y, x, n);
-  GMOD_CHECK_LAUNCH();
-}
-
 __global__ void k_lincomb(zd* y, const zd* a, double ca, const zd* b, double cb, long n) {
   for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += (long)gridDim.x * blockDim.x)
     y[e] = a[e] * ca + b[e] * cb;
@@ -903,7 +892,6 @@ void sigma_inc_contract(cpx<R>* out, const cpx<R>* Fr, const cpx<R>* Fd, const c
   template void mul_acc<R>(cpx<R>*, const cpx<R>*, const cpx<R>*, bool, long, hipStream_t); \
   template void contract<R>(cpx<R>*, const cpx<R>*, const cpx<R>*, const int*, const int*, const int*, int, long, \
                             hipStream_t); \
-  template void add_inplace<R>(cpx<R>*, const cpx<R>*, long, hipStream_t); \
   template void sigma_ref_contract<R>(cpx<R>*, cpx<R>*, const cpx<R>*, const cpx<R>*, const cpx<R>*, const int*, int, \
                                       int, long, hipStream_t); \
   template void sigma_inc_contract<R>(cpx<R>*, const cpx<R>*, const cpx<R>*, const cpx<R>*, const cpx<R>*, \
