@@ -64,6 +64,7 @@ template <typename R> struct GridLoad {
   long stride = 0;  // of a batch: item i is the grid p + i stride
   using Item = GridLoad;
   __host__ __device__ Item at(unsigned i) const { return GridLoad{p + (long)i * stride, S, 0}; }
+  GridLoad from(long i) const { return GridLoad{p + i * stride, S, stride}; }
   // S, t < 2^24 and S t < 2^31 (checked by the plan): a 24-bit multiply
   __device__ cpx<R> operator()(unsigned sp, unsigned t) const { return p[sp + __umul24(S, t)]; }
   __host__ double algo_bytes(double N) const { return N * sizeof(cpx<R>); }
@@ -74,6 +75,7 @@ template <typename R> struct GridStore {
   long stride = 0;
   using Item = GridStore;
   __host__ __device__ Item at(unsigned i) const { return GridStore{p + (long)i * stride, S, 0}; }
+  GridStore from(long i) const { return GridStore{p + i * stride, S, stride}; }
   struct Pre {};
   __device__ Pre prep(unsigned, unsigned) const { return Pre{}; }
   __device__ void commit(unsigned sp, unsigned t, const Pre&, cpx<R> v) const { p[sp + __umul24(S, t)] = v; }
@@ -510,26 +512,18 @@ void FFTPlan<R>::exec_batch(LD ld, ST st, cpx<R>* buf, int n, cpx<R>* tmp, int s
       cpx<R>* bb = buf + (long)i0 * size();
       auto bo = [&](int which) { return which ? tmp : bb; };
       auto run = [&](auto l, auto t, int i, R sc) { launch_box(sg, i, l, t, step, sign, sc, s); };
-      auto pass = [&](auto l, auto t) {
-        for (int i = 0; i < nb; ++i) {
-          const BoxArgs& a = bp[i];
-          const R sc = (i == nb - 1) ? scale : (R)1;
-          const GridLoad<R> gl{bo(a.src), S_, size()};
-          const GridStore<R> gs{bo(a.dst), S_, size()};
-          const bool first = i == 0, last = i == nb - 1;
-          if (first && last) run(l, t, i, sc);
-          else if (first) run(l, gs, i, sc);
-          else if (last) run(gl, t, i, sc);
-          else run(gl, gs, i, sc);
-        }
-      };
-      if (step == n) {
-        pass(ld, st);
-      } else if constexpr (std::is_same<LD, typename BatchOf<LD>::Item>::value &&
-                           std::is_same<ST, typename BatchOf<ST>::Item>::value) {
-        pass(BatchOf<LD>::at(ld, i0), BatchOf<ST>::at(st, i0));
-      } else {
-        throw Error("FFT: the split t axis (GMOD_FFT_TSPLIT) has no batched form");
+      const LD l = BatchOf<LD>::from(ld, i0);
+      const ST t = BatchOf<ST>::from(st, i0);
+      for (int i = 0; i < nb; ++i) {
+        const BoxArgs& a = bp[i];
+        const R sc = (i == nb - 1) ? scale : (R)1;
+        const GridLoad<R> gl{bo(a.src), S_, size()};
+        const GridStore<R> gs{bo(a.dst), S_, size()};
+        const bool first = i == 0, last = i == nb - 1;
+        if (first && last) run(l, t, i, sc);
+        else if (first) run(l, gs, i, sc);
+        else if (last) run(gl, t, i, sc);
+        else run(gl, gs, i, sc);
       }
     }
     return;

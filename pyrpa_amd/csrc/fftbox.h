@@ -587,17 +587,22 @@ __host__ __device__ __forceinline__ void box_twiddles_to_lds(cpx<R>* lds, const 
 
 // A load or store functor of a batch of transforms names the functor of one
 // item (Item) and forms it with at(item); the grids and tables it needs are
-// found by the item's index, so the batch is one launch.  A functor without
-// Item is its own only item.
+// found by the item's index, so the batch is one launch.  from(i) is the batch
+// that begins at item i.  A functor without Item is its own only item.
 template <class F, class = void>
 struct BatchOf {
   using Item = F;
   __host__ __device__ static const F& at(const F& f, unsigned) { return f; }
+  static F from(const F& f, long i) {
+    if (i != 0) throw Error("FFT: a single transform run as a batch");
+    return f;
+  }
 };
 template <class F>
 struct BatchOf<F, std::void_t<typename F::Item>> {
   using Item = typename F::Item;
   __host__ __device__ static Item at(const F& f, unsigned i) { return f.at(i); }
+  static F from(const F& f, long i) { return f.from(i); }
 };
 
 // A store may also drop whole boxes by their index (skip_box(lb), lb the

@@ -116,8 +116,13 @@ struct GreenBatch {
   const cpx<S>* G;
   int No;
   MeshDev m;
+  unsigned i0 = 0;  // item 0's index
   using Item = GreenLoad<R, S>;
-  __host__ __device__ Item at(unsigned i) const { return Item{G, (int)i % No, (int)i / No, No, m}; }
+  __host__ __device__ Item at(unsigned j) const {
+    const int i = (int)(i0 + j);
+    return Item{G, i % No, i / No, No, m};
+  }
+  GreenBatch from(long i) const { return GreenBatch{G, No, m, i0 + (unsigned)i}; }
 };
 
 // G_ab of a spinful basis on the full grid (fchi0withsoc.f90:57-75,
@@ -158,11 +163,13 @@ struct SocGreenBatch {
   DualPtr<int> inv;
   DualPtr<double> spin;
   MeshDev m;
+  unsigned i0 = 0;
   using Item = SocGreenLoad<R>;
-  __host__ __device__ Item at(unsigned i) const {
-    const int a = (int)i % No, b = (int)i / No;
+  __host__ __device__ Item at(unsigned j) const {
+    const int i = (int)(i0 + j), a = i % No, b = i / No;
     return Item{G, a, b, inv[a], inv[b], No, spin[a] * spin[b], m};
   }
+  SocGreenBatch from(long i) const { return SocGreenBatch{G, No, inv, spin, m, i0 + (unsigned)i}; }
 };
 
 // bosonic V_(m,l) (fself.f90:203-224, feliash.f90:543-564): slot 0 = nu_0,
@@ -327,11 +334,13 @@ struct AnomBatch {
   DualPtr<double> prt;
   double sgn, dprt;
   MeshDev m;
+  unsigned i0 = 0;
   using Item = AnomLoad<R>;
-  __host__ __device__ Item at(unsigned i) const {
-    const int a = (int)i % No, b = (int)i / No;
+  __host__ __device__ Item at(unsigned j) const {
+    const int i = (int)(i0 + j), a = i % No, b = i / No;
     return Item{F, NkNw * (a + (long)No * b), NkNw * (b + (long)No * a), prt[a] * prt[b], sgn, dprt, m};
   }
+  AnomBatch from(long i) const { return AnomBatch{F, NkNw, No, prt, sgn, dprt, m, i0 + (unsigned)i}; }
 };
 
 // one leg of the anomalous bubble chi^FF (ffeliash.f90:556-580): slot t < Nw
