@@ -302,9 +302,10 @@ class FFTPlan {
     exec_batch(ld, st, buf, 1, tmp, sign, scale, s, spatial_first);
   }
   // n transforms, item i through ld.at(i) and st.at(i) with intermediates in
-  // buf + i size(); tmp (one grid) is used item by item where a plan needs a
-  // second buffer.  One launch per pass: a transform of a small or middling
-  // grid alone has too few boxes for the CUs.
+  // buf + i size().  One launch per pass: a transform of a small or middling
+  // grid alone has too few boxes for the CUs.  Where a plan needs a second
+  // buffer, tmp (one grid) serves item by item, or batch_items grids of its
+  // own serve the items of a launch.
   template <class LD, class ST>
   void exec_batch(LD ld, ST st, cpx<R>* buf, int n, cpx<R>* tmp, int sign, R scale, hipStream_t s,
                   bool spatial_first = false) const;
@@ -534,24 +535,31 @@ void FFTPlan<R>::exec_batch(LD ld, ST st, cpx<R>* buf, int n, cpx<R>* tmp, int s
   if (np == 0) throw Error("FFT with nothing to transform");
   bool scratch = false;
   for (const FFTPassDesc& p : ps) scratch = scratch || p.src != 0 || p.dst != 0;
-  // a second buffer for every item of a batch (its block returns to the pool
-  // in stream order)
+  // where the passes need a second buffer, one per item of a launch, a batch
+  // is cut to batch_items (its block returns to the pool in stream order)
+  const int step = scratch ? batch_items(n) : n;
   DBuf<cpx<R>> many;
-  if (scratch && n > 1) {
-    many.alloc((size_t)n * size());
+  if (scratch && step > 1) {
+    many.alloc((size_t)step * size());
     tmp = many.p;
   }
-  auto buf_of = [&](int which) { return which ? tmp : buf; };
-  for (int i = 0; i < np; ++i) {
-    const FFTPassDesc& p = ps[i];
-    const R sc = (i == np - 1) ? scale : (R)1;
-    const GridLoad<R> gl{buf_of(p.src), S_, size()};
-    const GridStore<R> gs{buf_of(p.dst), S_, size()};
-    const bool first = i == 0, last = i == np - 1;
-    if (first && last) launch(p, ld, st, n, tw, sc, s);
-    else if (first) launch(p, ld, gs, n, tw, sc, s);
-    else if (last) launch(p, gl, st, n, tw, sc, s);
-    else launch(p, gl, gs, n, tw, sc, s);
+  for (int i0 = 0; i0 < n; i0 += step) {
+    const int m = std::min(step, n - i0);
+    cpx<R>* bb = buf + (long)i0 * size();
+    const LD l = BatchOf<LD>::from(ld, i0);
+    const ST t = BatchOf<ST>::from(st, i0);
+    auto buf_of = [&](int which) { return which ? tmp : bb; };
+    for (int i = 0; i < np; ++i) {
+      const FFTPassDesc& p = ps[i];
+      const R sc = (i == np - 1) ? scale : (R)1;
+      const GridLoad<R> gl{buf_of(p.src), S_, size()};
+      const GridStore<R> gs{buf_of(p.dst), S_, size()};
+      const bool first = i == 0, last = i == np - 1;
+      if (first && last) launch(p, l, t, m, tw, sc, s);
+      else if (first) launch(p, l, gs, m, tw, sc, s);
+      else if (last) launch(p, gl, t, m, tw, sc, s);
+      else launch(p, gl, gs, m, tw, sc, s);
+    }
   }
 }
 
