@@ -181,7 +181,7 @@ class ConvEngine {
   std::vector<double> sig_stat;
   const cpx<R>* sig_fg = nullptr;
   bool sig_fused = false, sig_unfused = false;
-  int sig_slots = 0, sig_outs = 0;
+  int sig_slots = 0, sig_outs = 0, sig_cap = 1;
   DualTab<int> sig_off, sig_map, sig_heads, sig_ta, sig_tb, sig_gat;
   DualTab<double> sig_hstat;
   DualTab<long> sig_hoffs;

@@ -516,9 +516,10 @@ void ConvEngine<R>::sigma_tables(const double* stat_h, hipStream_t s) {
     for (int m = 0; m < Nchi; ++m)
       if (stat_h[m + Nchi * l] != stat_h[l + Nchi * m]) { share = false; break; }
   // as many outputs at once as give the CUs several rounds of boxes, their
-  // sources within 4 GB
-  const long slots = std::max<long>(1, (4L << 30) / (N * (long)sizeof(cpx<R>)));
-  sig_groups = plan_sigma(share, p4->batch_items(No * No), (int)std::min<long>(slots, 1 << 20));
+  // sources within 4 GB; a single output of the unfused form whose sources
+  // exceed that is summed in parts
+  sig_cap = (int)std::min<long>(std::max<long>(1, (4L << 30) / (N * (long)sizeof(cpx<R>))), 1 << 20);
+  sig_groups = plan_sigma(share, p4->batch_items(No * No), sig_cap);
   std::vector<int> smap, off, heads, ta, tb, gat;
   std::vector<double> hstat;
   std::vector<long> hoffs;
@@ -530,14 +531,17 @@ void ConvEngine<R>::sigma_tables(const double* stat_h, hipStream_t s) {
     g.first_src = (int)smap.size();
     g.first_head = (int)heads.size() / 2;
     g.first_out = (int)gat.size() / 4;
+    const int nh = (int)g.heads.size();
+    const bool parts = !sig_fused && nh > sig_cap;  // one output, a head per source
     off.push_back(0);
     int c = 0;
     for (size_t i = 0; i < g.outs.size(); ++i) {
       for (auto& e : g.src[i]) {
+        if (parts && c > 0 && c % sig_cap == 0) off.push_back(c);
         const int ab = op.ol[e[0]][1] + No * op.ol[e[1]][1];
         accum_tab_h.push_back(Fg.p + (long)ab * N);
         smap.push_back(e[2]);
-        ta.push_back(e[2] >> 1);
+        ta.push_back((e[2] >> 1) % (parts ? sig_cap : nh));
         tb.push_back(ab);
         ++c;
       }
@@ -552,7 +556,7 @@ void ConvEngine<R>::sigma_tables(const double* stat_h, hipStream_t s) {
       hstat.push_back(stat_h[h[0] + Nchi * h[1]]);
       head_offsets(hoffs, h[0], h[1]);
     }
-    sig_slots = std::max(sig_slots, (int)g.heads.size());
+    sig_slots = std::max(sig_slots, parts ? sig_cap : nh);
     sig_outs = std::max(sig_outs, (int)g.outs.size());
   }
   sig_off.set(std::move(off), s);
@@ -596,9 +600,12 @@ void ConvEngine<R>::sigma(zd* sig, const zd* V, const double* stat_h, double tem
       p4->exec_accum_last(srcs.p, N, g.nsrc, MulAccAccum<R>{accum_tab.p + g.first_src, acc.p, S, N}, -1, (R)1, s,
                           sig_map.d.p + g.first_src, dhD.p, sig_off.d.p + g.first_off, no);
     } else {
-      p4->exec_batch(heads.from(g.first_head), GridStore<R>{srcs.p, S, N}, srcs.p, nh, tmp.p, -1, (R)1, s);
-      contract<R>(acc.p, srcs.p, Fg.p, sig_off.d.p + g.first_off, sig_ta.d.p + g.first_src, sig_tb.d.p + g.first_src,
-                  no, N, s);
+      for (int h0 = 0, part = 0; h0 < nh; h0 += sig_cap, ++part) {
+        p4->exec_batch(heads.from(g.first_head + h0), GridStore<R>{srcs.p, S, N}, srcs.p, std::min(sig_cap, nh - h0),
+                       tmp.p, -1, (R)1, s);
+        contract<R>(acc.p, srcs.p, Fg.p, sig_off.d.p + g.first_off + part, sig_ta.d.p + g.first_src,
+                    sig_tb.d.p + g.first_src, no, N, part > 0, s);
+      }
     }
     p4->exec_batch(GridLoad<R>{acc.p, S, N}, gat.from(g.first_out), acc.p, no, tmp.p, +1, invN, s);
   }
@@ -682,7 +689,7 @@ void ConvEngine<R>::gap(zd* nd, const zd* F, const double* prt, bool singlet, do
   for (int o0 = 0; o0 < nout; o0 += step) {
     const int no = std::min(step, nout - o0);
     if (vft_cached) {
-      contract<R>(acc.p, Vft.p, Ff.p, gap_off.d.p + o0, gap_ta.d.p, gap_tb.d.p, no, N, s);
+      contract<R>(acc.p, Vft.p, Ff.p, gap_off.d.p + o0, gap_ta.d.p, gap_tb.d.p, no, N, false, s);
     } else {
       for (int o = o0; o < o0 + no; ++o)
         for (int c = gap_off.h[o]; c < gap_off.h[o + 1]; ++c)

@@ -799,10 +799,10 @@ struct GatherBatch {
 };
 
 // Products summed over sources: out + o N (o < nout) = sum of A_{ta[c]} B_{tb[c]}
-// over c = off[o] .. off[o + 1] - 1 in turn (grids of N elements)
+// over c = off[o] .. off[o + 1] - 1 in turn (grids of N elements; add: onto out)
 template <typename R>
 void contract(cpx<R>* out, const cpx<R>* A, const cpx<R>* B, const int* off, const int* ta, const int* tb, int nout,
-              long N, hipStream_t s);
+              long N, bool add, hipStream_t s);
 // partner slices of a (Nk, Nw, ...) array: slice tab[4 i + 1] = +-conj slice
 // tab[4 i] (GatherBatch's table; negative: none)
 void partner_copies(zd* a, const int* tab, int n, long NkNw, hipStream_t s);

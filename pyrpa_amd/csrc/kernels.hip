@@ -379,11 +379,11 @@ template void mirror_grid<double>(cpx<double>*, const cpx<double>*, int, int, in
 template <typename R>
 __global__ void __launch_bounds__(TPB)
 k_contract(cpx<R>* __restrict__ out, const cpx<R>* __restrict__ A, const cpx<R>* __restrict__ B,
-           const int* __restrict__ off, const int* __restrict__ ta, const int* __restrict__ tb, long N) {
+           const int* __restrict__ off, const int* __restrict__ ta, const int* __restrict__ tb, long N, int add) {
   const int o = blockIdx.y, c0 = off[o], c1 = off[o + 1];
   for (long e = blockIdx.x * (long)TPB + threadIdx.x; e < N; e += (long)gridDim.x * TPB) {
-    cpx<R> acc = A[ta[c0] * N + e] * B[tb[c0] * N + e];
-    for (int c = c0 + 1; c < c1; ++c) {
+    cpx<R> acc = add ? out[o * N + e] : A[ta[c0] * N + e] * B[tb[c0] * N + e];
+    for (int c = add ? c0 : c0 + 1; c < c1; ++c) {
       const cpx<R> v = A[ta[c] * N + e] * B[tb[c] * N + e];
       acc = acc + v;
     }
@@ -392,9 +392,9 @@ k_contract(cpx<R>* __restrict__ out, const cpx<R>* __restrict__ A, const cpx<R>*
 }
 template <typename R>
 void contract(cpx<R>* out, const cpx<R>* A, const cpx<R>* B, const int* off, const int* ta, const int* tb, int nout,
-              long N, hipStream_t s) {
+              long N, bool add, hipStream_t s) {
   hipLaunchKernelGGL((k_contract<R>), dim3(nblocks(N, TPB, 4096), (unsigned)nout), dim3(TPB), 0, s, out, A, B, off, ta,
-                     tb, N);
+                     tb, N, add ? 1 : 0);
   GMOD_CHECK_LAUNCH();
 }
 
@@ -891,7 +891,7 @@ void sigma_inc_contract(cpx<R>* out, const cpx<R>* Fr, const cpx<R>* Fd, const c
 #define INST(R) \
   template void mul_acc<R>(cpx<R>*, const cpx<R>*, const cpx<R>*, bool, long, hipStream_t); \
   template void contract<R>(cpx<R>*, const cpx<R>*, const cpx<R>*, const int*, const int*, const int*, int, long, \
-                            hipStream_t); \
+                            bool, hipStream_t); \
   template void sigma_ref_contract<R>(cpx<R>*, cpx<R>*, const cpx<R>*, const cpx<R>*, const cpx<R>*, const int*, int, \
                                       int, long, hipStream_t); \
   template void sigma_inc_contract<R>(cpx<R>*, const cpx<R>*, const cpx<R>*, const cpx<R>*, const cpx<R>*, \

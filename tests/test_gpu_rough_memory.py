@@ -39,7 +39,8 @@ def free_bytes(F):
     return f.value
 
 
-@pytest.mark.parametrize("ny,sources", [(506, None), (1936, 4)])  # grids of 26 MB (several a launch) and 101 MB
+# grids of 26 MB (several a launch), 101 MB and 1.2 GB (an output's sources in two parts)
+@pytest.mark.parametrize("ny,sources", [(506, None), (1936, 4), (23184, 3)])
 def test_flex_on_a_rough_mesh(ny, sources):
     import pyrpa_amd.flibs as F
     F.set_precision(0)
