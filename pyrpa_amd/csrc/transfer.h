@@ -29,6 +29,7 @@ class HostCopy {
   friend void copy_to_device(void* dst, const void* src, size_t bytes, hipStream_t s);
   void run(char* dst, const char* src, size_t bytes, bool to_host, hipStream_t s);
   void join();
+  bool owner_ = false;  // of the staging buffers, from run() to join()
   std::vector<std::thread> threads_;
   std::atomic<int> error_{0};
 };

@@ -47,14 +47,15 @@ void release_transfer_buffers() {
 }
 
 void HostCopy::run(char* dst, const char* src, size_t bytes, bool to_host, hipStream_t s) {
+  const size_t n = (bytes + PIECE - 1) / PIECE;
+  const unsigned hw = std::max(2u, std::thread::hardware_concurrency());
+  const int nt = (int)std::min<size_t>(n, std::min<unsigned>(MAX_THREADS, hw / 2));
+  threads_.reserve(nt);
   // both directions wait for what s holds: its kernels write the source, or
   // still use the block that the destination was allocated from
   GMOD_HIP(hipEventRecord(g_before, s));
   GMOD_HIP(hipStreamWaitEvent(g_stream, g_before, 0));
-  g_busy = true;
-  const size_t n = (bytes + PIECE - 1) / PIECE;
-  const unsigned hw = std::max(2u, std::thread::hardware_concurrency());
-  const int nt = (int)std::min<size_t>(n, std::min<unsigned>(MAX_THREADS, hw / 2));
+  g_busy = owner_ = true;
   const int dev = ctx().device;
   auto work = [=](int t) {
     auto ok = [&](hipError_t e) {
@@ -88,7 +89,6 @@ void HostCopy::run(char* dst, const char* src, size_t bytes, bool to_host, hipSt
     while (nheld > 0)
       if (!retire()) return;
   };
-  threads_.reserve(nt);
   for (int t = 0; t < nt; ++t) {
     try {
       threads_.emplace_back(work, t);
@@ -99,10 +99,10 @@ void HostCopy::run(char* dst, const char* src, size_t bytes, bool to_host, hipSt
 }
 
 void HostCopy::join() {
-  if (threads_.empty()) return;
+  if (!owner_) return;
   for (auto& t : threads_) t.join();
   threads_.clear();
-  g_busy = false;
+  g_busy = owner_ = false;
 }
 
 void HostCopy::start(void* dst, const void* src, size_t bytes, hipStream_t s) {
