@@ -102,6 +102,8 @@ void HostCopy::join() {
   if (!owner_) return;
   for (auto& t : threads_) t.join();
   threads_.clear();
+  // a worker that failed leaves its pieces in flight
+  if (error_.load()) (void)hipStreamSynchronize(g_stream);
   g_busy = owner_ = false;
 }
 

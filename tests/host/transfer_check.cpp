@@ -1,7 +1,7 @@
 // Drives transfer.hip's staged copies on the CPU against a small model of the
 // runtime: copies of the library's own stream run as late as they may (when an
 // event recorded behind them or the stream is waited for), other streams run at
-// once, threads can be made to fail.  Prints the failed check.
+// once, threads and copies can be made to fail.  Prints the failed check.
 #include <dlfcn.h>
 #include <pthread.h>
 
@@ -19,7 +19,7 @@ std::mutex g_mu;
 std::deque<Op> g_queue;
 std::vector<std::pair<char*, size_t>> g_pinned;
 int g_own;  // the library's stream is &g_own
-int g_fail_thread = 0, g_staged = 0, g_freed = 0;
+int g_fail_thread = 0, g_fail_copy = -1, g_copies = 0, g_staged = 0, g_freed = 0;
 
 void run_until(void* ev) {  // ev null: all
   while (!g_queue.empty()) {
@@ -68,6 +68,7 @@ hipError_t hipHostFree(void* p) {
 }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t st) {
   std::lock_guard<std::mutex> g(g_mu);
+  if (g_copies++ == g_fail_copy) return hipErrorUnknown;
   if (pinned(d) || pinned(s)) ++g_staged;
   if ((void*)st == &g_own) g_queue.push_back({d, s, n, nullptr});
   else memcpy(d, s, n);
@@ -139,6 +140,29 @@ int main(int argc, char** argv) {
     CHECK(g_freed == 16 && g_pinned.empty());
     g_fail_thread = 0;
     round_trip(big, 2);
+  } else if (what == "failed_copy") {  // an error, nothing left in flight on the buffers, the next copy right
+    const std::vector<char> a = values(big, 1);
+    std::vector<char> d(big);
+    for (int run = 0; run < 8; ++run) {  // with and without threads, a copy in the middle and the last one
+      const bool dir = run & 1;
+      g_fail_thread = run & 2;
+      g_copies = 0;
+      g_fail_copy = run & 4 ? 18 : 9;
+      bool thrown = false;
+      try {
+        if (dir) gmod::copy_to_host(d.data(), a.data(), big, S);
+        else gmod::copy_to_device(d.data(), a.data(), big, S);
+      } catch (gmod::Error&) {
+        thrown = true;
+      }
+      g_fail_copy = -1;
+      g_fail_thread = 0;
+      CHECK(thrown);
+      size_t left = 0;
+      for (auto& o : g_queue) left += o.dst != nullptr;
+      CHECK(left == 0);
+      round_trip(big, 3 + run);
+    }
   } else if (what == "background") {  // another copy meanwhile, and an abandoned one
     const std::vector<char> a = values(big, 1);
     std::vector<char> b(big);

@@ -1,7 +1,7 @@
 """The staged copies between the caller's arrays and the device on the CPU
 (tests/host/transfer_check.cpp): the library's transfer unit with a model of
 the runtime whose copies run as late as they may, around the size where staging
-begins, without threads, and in the background."""
+begins, without threads, with a failing copy, and in the background."""
 import os
 import subprocess
 
@@ -20,7 +20,7 @@ def check(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["sizes", "no_threads", "release", "background"])
+@pytest.mark.parametrize("what", ["sizes", "no_threads", "release", "failed_copy", "background"])
 def test_staged_copies(check, what):
     r = subprocess.run([check, what], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
