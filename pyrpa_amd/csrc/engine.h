@@ -122,7 +122,7 @@ class ConvEngine {
   // Sigma through the accumulating last pass: the sources of one output
   // after their first passes, and the device table of their operand grids
   DBuf<cpx<R>> srcs;
-  DBuf<cpx<R>*> accum_tab;
+  DBuf<cpx<R>*> accum_tab;  // of the increment; sigma() keeps sig_tab from one call to the next
   // the grouped Sigma increment: Y of every output, then Gn = Fr + Fd of every
   // orbital pair (the contraction form: the outputs themselves); ytab_d: per
   // output and pair the reference-vertex grid
@@ -183,6 +183,7 @@ class ConvEngine {
   bool sig_fused = false, sig_unfused = false;
   int sig_slots = 0, sig_outs = 0, sig_cap = 1;
   DualTab<int> sig_off, sig_map, sig_heads, sig_ta, sig_tb, sig_gat;
+  DBuf<cpx<R>*> sig_tab;
   DualTab<double> sig_hstat;
   DualTab<long> sig_hoffs;
   DBuf<int> srcmap_d;

@@ -523,7 +523,7 @@ void ConvEngine<R>::sigma_tables(const double* stat_h, hipStream_t s) {
   std::vector<int> smap, off, heads, ta, tb, gat;
   std::vector<double> hstat;
   std::vector<long> hoffs;
-  accum_tab_h.clear();
+  std::vector<cpx<R>*> fg;
   sig_slots = 0;
   sig_outs = 0;
   for (auto& g : sig_groups) {
@@ -539,7 +539,7 @@ void ConvEngine<R>::sigma_tables(const double* stat_h, hipStream_t s) {
       for (auto& e : g.src[i]) {
         if (parts && c > 0 && c % sig_cap == 0) off.push_back(c);
         const int ab = op.ol[e[0]][1] + No * op.ol[e[1]][1];
-        accum_tab_h.push_back(Fg.p + (long)ab * N);
+        fg.push_back(Fg.p + (long)ab * N);
         smap.push_back(e[2]);
         ta.push_back((e[2] >> 1) % (parts ? sig_cap : nh));
         tb.push_back(ab);
@@ -567,9 +567,9 @@ void ConvEngine<R>::sigma_tables(const double* stat_h, hipStream_t s) {
   sig_ta.set(std::move(ta), s);
   sig_tb.set(std::move(tb), s);
   sig_gat.set(std::move(gat), s);
-  accum_tab.alloc(accum_tab_h.size());
-  accum_tab.upload(accum_tab_h.data(), accum_tab_h.size(), s);
-  GMOD_HIP(hipStreamSynchronize(s));
+  sig_tab.alloc(fg.size());
+  sig_tab.upload(fg.data(), fg.size(), s);
+  GMOD_HIP(hipStreamSynchronize(s));  // fg is released here
 }
 
 template <typename R>
@@ -597,7 +597,7 @@ void ConvEngine<R>::sigma(zd* sig, const zd* V, const double* stat_h, double tem
       p4->exec_head(heads.from(g.first_head), srcs.p, nh, tmp.p, -1, s);
       if (dhD.n < (size_t)nh * S) dhD.alloc((size_t)nh * S);
       slot0_corr(dhD.p, V, sig_hoffs.d.p + 2 * (long)g.first_head, nh, s);
-      p4->exec_accum_last(srcs.p, N, g.nsrc, MulAccAccum<R>{accum_tab.p + g.first_src, acc.p, S, N}, -1, (R)1, s,
+      p4->exec_accum_last(srcs.p, N, g.nsrc, MulAccAccum<R>{sig_tab.p + g.first_src, acc.p, S, N}, -1, (R)1, s,
                           sig_map.d.p + g.first_src, dhD.p, sig_off.d.p + g.first_off, no);
     } else {
       for (int h0 = 0, part = 0; h0 < nh; h0 += sig_cap, ++part) {
