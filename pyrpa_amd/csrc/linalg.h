@@ -34,6 +34,17 @@ void soc_vertex(const zd* chi_in, zd* out, long batch, BatchLayout L, int n, con
 // X = (I + alpha A W)^-1 A  (fchi.f90:319-350, fself.f90:783-816); out may alias nothing
 void rpa_solve(zd* out, BatchLayout Lo, const zd* A, BatchLayout La, long batch, int n, const double* W,
                double alpha, int* err, hipStream_t s);
+// A wavefront per matrix up to 64 rows (a lane per row, and 64 x 64 is what
+// fits twice in the 160 KB of LDS), while the batch is short of the line below:
+// a lane per matrix takes one serial chain of any batch that fits the chip,
+// the wavefronts a time in proportion to the batch.  Lane and wave kernel, us:
+//   n = 1, 20000 matrices 30 and 33; 200000: 30 and 71
+//   n = 4, 6000: 161 and 128; 20000: 212 and 308; 200000: 1035 and 2564
+//   n = 9, 9000: 861 and 684; 16000: 858 and 1137; 48000: 1556 and 3234
+//   n = 16, 12000: 3878 and 3086; 24000: 5249 and 5516; 48000: 6788 and 11089
+//   n = 25, 24000: 17454 and 15054; 48000: 30771 and 29953
+constexpr int EIG_WAVE_MAX = 64;
+inline bool eig_by_wave(long batch, int n) { return n <= EIG_WAVE_MAX && batch <= 9500 + 40L * n * n; }
 // max Re eig(alpha * A * W) per matrix (W = nullptr: identity)  (fchi.f90:373-389)
 void max_re_eig(double* out, const zd* A, BatchLayout La, long batch, int n, const double* W, double alpha,
                 int* err, hipStream_t s);

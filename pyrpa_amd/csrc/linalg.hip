@@ -6,7 +6,7 @@
 //   one lane per element.
 // * dyson / filling_charpoly / green0 / anomalous_f: one lane per (k, i w) with
 //   the No x No matrix held in registers (No <= 8).
-// * max_re_eig: one wavefront per matrix (n <= 64); Hessenberg reduction + shifted complex QR.
+// * max_re_eig: one wavefront per matrix (n <= 64), one lane in large batches; Hessenberg reduction + shifted complex QR.
 #include <cfloat>
 #include <cmath>
 
@@ -1599,14 +1599,10 @@ k_max_re_eig_wave(double* out, const zd* A, BatchLayout La, long batch, int n, c
 #undef HH
 }
 
-// a wavefront has one lane per row, and 64 x 64 is also what fits twice in
-// the 160 KB of LDS; larger matrices run one lane each in the workspace
-constexpr int EIG_WAVE_MAX = 64;
-
 void max_re_eig_ws(double* out, const zd* A, BatchLayout La, long batch, int n, const double* W, double alpha,
                    zd* work, int* err, hipStream_t s) {
   if (batch <= 0) return;
-  if (n <= EIG_WAVE_MAX) {
+  if (eig_by_wave(batch, n)) {
     const size_t shm = ((size_t)n * (n + 1) + (size_t)std::max(n * n, 2 * n)) * sizeof(zd);
     if (shm > 64 * 1024)
       GMOD_HIP(hipFuncSetAttribute((const void*)&k_max_re_eig_wave, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1624,7 +1620,7 @@ void max_re_eig_ws(double* out, const zd* A, BatchLayout La, long batch, int n, 
 void max_re_eig(double* out, const zd* A, BatchLayout La, long batch, int n, const double* W, double alpha,
                 int* err, hipStream_t s) {
   if (batch <= 0) return;
-  DBuf<zd> scratch(n <= EIG_WAVE_MAX ? 0 : batch * (long)(n * n + n));
+  DBuf<zd> scratch(eig_by_wave(batch, n) ? 0 : batch * (long)(n * n + n));
   max_re_eig_ws(out, A, La, batch, n, W, alpha, scratch.p, err, s);
   if (scratch.n) GMOD_HIP(hipStreamSynchronize(s));
 }
