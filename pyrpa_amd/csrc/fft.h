@@ -363,8 +363,7 @@ class FFTPlan {
   void launch(const FFTPassDesc& p, LD ld, ST st, int n, const cpx<R>* tw, R sc, hipStream_t s) const;
   template <class LD, class ST>
   void launch_box(int sg, int i, LD ld, ST st, int n, int sign, R sc, hipStream_t s) const;
-  // pass i runs with the small boxes: the launch would leave CUs idle, or
-  // the pass is not tiled (two work-groups then share a CU)
+  // pass i of n transforms runs with the small boxes (box_take_small)
   bool small_pass(int sg, int i, long n) const;
   int dims_[4];
   int mask_;

@@ -557,18 +557,10 @@ FFTPlan<R>::~FFTPlan() {
   free_tables(dev_s_);
 }
 
-// Quarter-size boxes where whole ones leave CUs idle (1 orbital, 32x32 x 512:
-// 64 boxes, now 256; a plain pass 16.9 -> 13.4 us) and for untiled passes,
-// which need two boxes in a CU's LDS to overlap (27x27x5 x 180: 28 us a grid
-// in a launch of its own, now 22 in a batch of 9); whole boxes elsewhere (see
-// BoxPlan::build: full launches measured slower with smaller boxes).
 template <typename R>
 bool FFTPlan<R>::small_pass(int sg, int i, long n) const {
   if (!box_s_.ok) return false;
-  const BoxArgs& a = (sg == 0 ? box_.fwd : box_.bwd)[i];
-  const BoxArgs& as = (sg == 0 ? box_s_.fwd : box_s_.bwd)[i];
-  if (as.blocks() == a.blocks()) return false;
-  return !a.tiled || a.blocks() * n < persist_;
+  return box_take_small((sg == 0 ? box_.fwd : box_.bwd)[i], (sg == 0 ? box_s_.fwd : box_s_.bwd)[i], n, persist_);
 }
 
 template <typename R>

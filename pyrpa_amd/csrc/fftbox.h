@@ -983,4 +983,19 @@ struct BoxPlan {
   void build(int nx, int ny, int nz, int m, int mask, long budget, size_t lds_bytes, long small = 0);
 };
 
+// Whether a pass over n transforms runs the quarter-size boxes `as` in place of
+// the whole boxes `a` on ncu CUs.
+// A tiled pass: where all of them run at once (a work-group per CU; two where
+// the quarter box is not tiled).  32x32 x 512 FP64, 64 boxes or 256: 17.8 us
+// whole, 12.5 quarter.  A second round costs more than the idle CUs of the
+// whole boxes: 16x16x8 x 512, 128 boxes or 512: 15.1 and 18.6 us; 64x48 x 512,
+// 192 or 768: 17.7 and 26.7; from one whole box per CU on, the same or slower.
+// An untiled pass needs two boxes in a CU's LDS to overlap (27x27x5 x 180: 28
+// us a grid in a launch of its own, 22 in a batch of 9).
+inline bool box_take_small(const BoxArgs& a, const BoxArgs& as, long n, long ncu) {
+  if (as.blocks() == a.blocks()) return false;
+  if (!a.tiled) return true;
+  return a.blocks() * n < ncu && as.blocks() * n <= (as.tiled ? 1 : 2) * ncu;
+}
+
 }  // namespace gmod

@@ -1,0 +1,35 @@
+"""Which box size a pass takes (fftbox.h) against the times of both, each pass
+timed alone: whole boxes where the quarter-size ones need a second round, small
+ones where they all run at once, whole ones on a full chip."""
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PKG = os.path.join(os.path.dirname(HERE), "pyrpa_amd")
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+
+@pytest.fixture(scope="module")
+def passes(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("rule") / "fft_rule")
+    subprocess.run([HIPCC, "-std=c++17", "-O1", "--offload-host-only", "-x", "hip", "-c",
+                    os.path.join(HERE, "host", "fft_rule.cpp"), "-o", exe + ".o"], check=True, timeout=300)
+    subprocess.run([HIPCC, exe + ".o", os.path.join(PKG, "libgmod.so"), "-Wl,-rpath," + PKG, "-o", exe], check=True,
+                   timeout=300)
+    return lambda *a: subprocess.run([exe, *map(str, a)], capture_output=True, text=True, check=True,
+                                     timeout=60).stdout.strip()
+
+
+@pytest.mark.parametrize("prec,dims,mask,n,want", [
+    (0, (32, 32, 1, 512), 7, 1, "s"), (0, (32, 32, 1, 512), 8, 1, "s"), (0, (16, 16, 8, 256), 8, 1, "s"),
+    (0, (64, 64, 1, 256), 7, 1, "s"), (1, (32, 32, 1, 1024), 7, 1, "s"), (1, (16, 16, 16, 256), 8, 1, "s"),
+    (0, (40, 32, 1, 512), 7, 1, "s"), (1, (48, 48, 1, 512), 7, 1, "s"),  # the quarter box is not tiled: two a CU
+    (0, (48, 32, 1, 512), 7, 1, "w"), (0, (16, 16, 8, 512), 7, 1, "w"), (0, (16, 16, 8, 512), 8, 1, "w"),
+    (0, (64, 48, 1, 512), 8, 1, "w"), (0, (16, 16, 1, 4096), 7, 1, "w"), (1, (32, 32, 4, 512), 15, 1, "ww"),
+    (1, (96, 32, 1, 512), 7, 1, "w"), (1, (64, 64, 1, 512), 8, 1, "w"),
+    (0, (16, 16, 4, 256), 15, 2, "ss"), (0, (16, 16, 4, 256), 15, 4, "ww"), (0, (32, 32, 1, 2048), 15, 1, "ww"),
+    (0, (32, 32, 16, 2048), 15, 1, "www")])
+def test_tiled_passes(passes, prec, dims, mask, n, want):
+    assert passes(prec, *dims, mask, n) == want
