@@ -116,6 +116,7 @@ void BoxPlan<R>::build(int nx, int ny, int nz, int m, int mask, long budget, siz
   };
   max_lds_bytes = 0;
   lds_limit = lds_bytes;
+  this->budget = budget;
   auto make_box = [&](const int ext[4], const std::vector<int>& tdims, BoxArgs& a) -> bool {
     a = BoxArgs{};
     long elems = 1;
@@ -560,7 +561,8 @@ FFTPlan<R>::~FFTPlan() {
 template <typename R>
 bool FFTPlan<R>::small_pass(int sg, int i, long n) const {
   if (!box_s_.ok) return false;
-  return box_take_small((sg == 0 ? box_.fwd : box_.bwd)[i], (sg == 0 ? box_s_.fwd : box_s_.bwd)[i], n, persist_);
+  return box_take_small((sg == 0 ? box_.fwd : box_.bwd)[i], (sg == 0 ? box_s_.fwd : box_s_.bwd)[i], n, persist_,
+                        box_.budget);
 }
 
 template <typename R>

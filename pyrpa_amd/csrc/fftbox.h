@@ -975,6 +975,7 @@ struct BoxPlan {
   std::vector<int> tab_host;       // tile tables of the tiled passes
   size_t max_lds_bytes = 0;  // largest box of this plan
   size_t lds_limit = 0;      // the device's per-work-group LDS limit the plan was built for
+  long budget = 0;           // and the largest box, in elements
   // plan the transform of the axes in `mask` of an (nx,ny,nz,m) grid with
   // boxes of at most `budget` elements and `lds_bytes` of LDS
   // (small: fill a box with untransformed points up to this many elements;
@@ -990,12 +991,24 @@ struct BoxPlan {
 // whole, 12.5 quarter.  A second round costs more than the idle CUs of the
 // whole boxes: 16x16x8 x 512, 128 boxes or 512: 15.1 and 18.6 us; 64x48 x 512,
 // 192 or 768: 17.7 and 26.7; from one whole box per CU on, the same or slower.
-// An untiled pass needs two boxes in a CU's LDS to overlap (27x27x5 x 180: 28
-// us a grid in a launch of its own, 22 in a batch of 9).
-inline bool box_take_small(const BoxArgs& a, const BoxArgs& as, long n, long ncu) {
+// An untiled pass: where all of them run at once, two a CU, or by the rounds
+// (whole ones up to four). A round costs a whole box its elements, and two
+// quarter boxes 1.15 of one's (they overlap: 27x27x5 x 180, 28 us a grid in a
+// launch of its own, 22 in a batch of 9) plus 0.15 of the largest box (the waits
+// of a short one): 48x48x12 x 150 FP64 t pass, 576 boxes or 2304: 76.8 us whole,
+// 58.8 quarter; 36x36x5 x 288 FP32, 180 or 540: 27.2 and 44.5; 45x32 x 4096, 512
+// or 2048: 62.1 and 84.8. Of 132 transforms timed alone two take a side that is
+// slower by more than 5 % (96x42x6 x 288 FP32: 127 us whole, 144 quarter;
+// 50x64x4 x 300 FP64 t pass: 60 and 70).
+inline bool box_take_small(const BoxArgs& a, const BoxArgs& as, long n, long ncu, long budget) {
   if (as.blocks() == a.blocks()) return false;
-  if (!a.tiled) return true;
-  return a.blocks() * n < ncu && as.blocks() * n <= (as.tiled ? 1 : 2) * ncu;
+  const long nw = a.blocks() * n, ns = as.blocks() * n;
+  if (a.tiled) return nw < ncu && ns <= (as.tiled ? 1 : 2) * ncu;
+  if (ns <= 2 * ncu) return true;
+  auto rounds = [](long boxes, long slots) {
+    return boxes > 4 * slots ? (double)boxes / (double)slots : (double)((boxes + slots - 1) / slots);
+  };
+  return rounds(ns, 2 * ncu) * (1.15 * as.elems + 0.15 * budget) <= rounds(nw, ncu) * a.elems;
 }
 
 }  // namespace gmod

@@ -17,7 +17,7 @@ static void print(char** v) {
   q.build(nx, ny, nz, m, mask, budget, lds, budget / 4);
   const bool two = q.ok && q.fwd.size() == p.fwd.size();
   for (size_t i = 0; i < p.fwd.size(); ++i)
-    putchar(two && box_take_small(p.fwd[i], q.fwd[i], atol(v[7]), 256) ? 's' : 'w');
+    putchar(two && box_take_small(p.fwd[i], q.fwd[i], atol(v[7]), 256, budget) ? 's' : 'w');
   putchar('\n');
 }
 
