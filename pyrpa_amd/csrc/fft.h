@@ -470,12 +470,14 @@ void FFTPlan<R>::launch_box(int sg, int i, LD ld, ST st, int n, int sign, R sc, 
   const Tables& tb = small ? dev_s_ : dev_;
   const BoxArgs& a = (sg == 0 ? bp.fwd : bp.bwd)[i];
   const size_t shm = (size_t)(a.lds_elems + a.ntwl) * sizeof(cpx<R>);
+  const long tot = a.blocks() * (long)n;
+  if (tot >= (1L << 31)) throw Error("FFT batch of 2^31 boxes or more");
   static bool attr_done = false;  // one per kernel instantiation: allow the device's whole LDS
   if (!attr_done) {
-    GMOD_HIP(hipFuncSetAttribute((const void*)&box_fft_kernel<R, LD, ST, true>,
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)box_.lds_limit));
-    GMOD_HIP(hipFuncSetAttribute((const void*)&box_fft_kernel<R, LD, ST, false>,
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)box_.lds_limit));
+    for (const void* f : {(const void*)&box_fft_kernel<R, LD, ST, BOX_PAIR>,
+                          (const void*)&box_fft_kernel<R, LD, ST, BOX_ONE>,
+                          (const void*)&box_fft_kernel<R, LD, ST, BOX_TILED>})
+      GMOD_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)box_.lds_limit));
     attr_done = true;
   }
   ProfScope ps(sizeof(R) == 4 ? PROF_FFT32 : PROF_FFT,
@@ -483,15 +485,15 @@ void FFTPlan<R>::launch_box(int sg, int i, LD ld, ST st, int n, int sign, R sc, 
   // the pool a pass reads its tables from is the sign's; the power-of-two
   // sub-passes take the sign itself at compile time
   const cpx<R>* tw = tb.tw[sign < 0 ? 0 : 1];
-  const long tot = a.blocks() * (long)n;
-  if (tot >= (1L << 31)) throw Error("FFT batch of 2^31 boxes or more");
-  if (a.tiled)  // persistent work-groups, one per CU, a multiple of 8
-    hipLaunchKernelGGL((box_fft_kernel<R, LD, ST, true>), dim3((unsigned)std::min(tot, persist_)), dim3(BOX_THREADS),
-                       shm, s, ld, st, (const BoxArgs*)(tb.args[sg] + i), tw, (const int*)tb.tabs, sc, sign,
-                       (unsigned)n);
-  else
-    hipLaunchKernelGGL((box_fft_kernel<R, LD, ST, false>), dim3((unsigned)tot), dim3(BOX_THREADS), shm, s, ld, st,
+  auto go = [&](auto kernel, long grid) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(BOX_THREADS), shm, s, ld, st,
                        (const BoxArgs*)(tb.args[sg] + i), tw, (const int*)tb.tabs, sc, sign, (unsigned)n);
+  };
+  switch (box_kind(a, tot, shm, box_.lds_limit, small, persist_)) {
+    case BOX_TILED: go(box_fft_kernel<R, LD, ST, BOX_TILED>, std::min(tot, persist_)); break;  // a multiple of 8 on a full chip
+    case BOX_ONE: go(box_fft_kernel<R, LD, ST, BOX_ONE>, tot); break;
+    case BOX_PAIR: go(box_fft_kernel<R, LD, ST, BOX_PAIR>, tot); break;
+  }
   GMOD_CHECK_LAUNCH();
 }
 

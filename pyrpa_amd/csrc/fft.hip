@@ -704,9 +704,9 @@ int box_host_run(double* data, int nx, int ny, int nz, int m, int mask, int sign
       seen[lb] = 1;
       const BoxOrigin O = box_origin(a, lb);
       box_twiddles_to_lds<R>(lds.data(), a, tw, 0, 1);
-      box_load<R>(lds.data(), HostGridLoad<R>{in, S}, a, O, 0, 1, plan.tab_host.data());
+      box_load<R, 8>(lds.data(), HostGridLoad<R>{in, S}, a, O, 0, 1, plan.tab_host.data());
       for (int j = 0; j < a.nsub; ++j) box_dispatch<R>(lds.data(), a, a.sub[j], tw, 0, 1, sign);
-      box_store<R>(lds.data(), HostGridStore<R>{out, S}, a, O, scale, tw, 0, 1, plan.tab_host.data());
+      box_store<R, 8>(lds.data(), HostGridStore<R>{out, S}, a, O, scale, tw, 0, 1, plan.tab_host.data());
     }
   }
   for (long i = 0; i < N; ++i) { data[2 * i] = (double)g[i].re; data[2 * i + 1] = (double)g[i].im; }

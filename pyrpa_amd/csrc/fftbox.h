@@ -293,7 +293,8 @@ __host__ __device__ __forceinline__ void box_load_tiled(cpx<R>* lds, const LD& l
 }
 
 // ---- phase 1: grid -> LDS (x fastest: coalesced along the grid's contiguous axis)
-template <typename R, class LD>
+// U: loads in flight per thread before the first LDS store
+template <typename R, int U, class LD>
 __host__ __device__ __forceinline__ void box_load(cpx<R>* lds, const LD& ld, const BoxArgs& a, const BoxOrigin& O,
                                                   int tid, int nthr, const int* __restrict__ tabs) {
 #if !defined(__HIP_DEVICE_COMPILE__)
@@ -302,9 +303,6 @@ __host__ __device__ __forceinline__ void box_load(cpx<R>* lds, const LD& ld, con
     return;
   }
 #endif
-  // U loads in flight per thread before the first LDS store (two work-groups
-  // share the CU's registers)
-  constexpr int U = sizeof(R) == 4 ? 8 : 4;
   const int ex = a.box[0], ey = a.box[1], ez = a.box[2];
   for (int e0 = tid; e0 < a.elems; e0 += nthr * U) {
     cpx<R> v[U];
@@ -512,7 +510,9 @@ __host__ __device__ __forceinline__ void box_store_tiled(const cpx<R>* lds, cons
 }
 
 // ---- phase 3: LDS -> grid through the store functor
-template <typename R, class ST>
+// U: elements of a batch; every load a store functor needs (accumulators,
+// operands, gather indices) is issued before the batch's first store
+template <typename R, int U, class ST>
 __host__ __device__ __forceinline__ void box_store(const cpx<R>* lds, const ST& st, const BoxArgs& a,
                                                    const BoxOrigin& O, R scale, const cpx<R>* __restrict__ tw,
                                                    int tid, int nthr, const int* __restrict__ tabs) {
@@ -522,9 +522,6 @@ __host__ __device__ __forceinline__ void box_store(const cpx<R>* lds, const ST& 
     return;
   }
 #endif
-  // batches of U elements: every load a store functor needs (accumulators,
-  // operands, gather indices) is issued before the batch's first store
-  constexpr int U = 2;
   const int ex = a.box[0], ey = a.box[1], ez = a.box[2];
   for (int e0 = tid; e0 < a.elems; e0 += nthr * U) {
     unsigned spv[U], tv[U];
@@ -932,21 +929,28 @@ box_accum_kernel(const cpx<R>* __restrict__ src, long src_stride, int nsrc1, AC 
 // than passed by value: run-time indices into a by-value kernel argument
 // make the compiler copy the whole argument to scratch memory.
 // Bound by the overlap of a box's load, sub-passes and store, not by bytes.
-// TILED: persistent work-groups, one per CU (the prefetch takes the registers
-// of a second one); else a work-group per box, two per CU (4 waves per SIMD),
-// so that one loads or stores while the other transforms.
+// BOX_TILED: persistent work-groups, one per CU (the prefetch takes the registers
+// of a second one).  Else a work-group per box: BOX_PAIR two per CU (4 waves per
+// SIMD), so that one loads or stores while the other transforms; BOX_ONE, for
+// boxes that fill more than half the LDS or are fewer than the CUs, with the
+// loads in flight that a CU's only work-group has to keep (in the kernel of its
+// own: beside the persistent loop it takes 5 % from FP32 tiled passes).  Pair
+// and one: 24x45x6 x 2400 FP32 t pass, boxes of 115 KB, 281 and 245 us;
+// 80x80 x 1250 FP64, 102 KB, 135 and 124; 36x36x5 x 288 FP32, 180 boxes, 32.5
+// and 27.2; 25x25x6 x 800 FP32, 750 boxes of 32 KB, 61 and 67.
 // nitem transforms in one launch: alone, a grid of 16x16x8 x 512 gives 128
 // boxes to 256 CUs (136 bubble products of 4 orbitals: 32 us each, now 21 in
 // batches of 8; their gathers 25 -> 11 us), and 16x16 x 256 eight boxes
 // (spin-orbit bubbles 13.6 -> 1.1 us each).
-template <typename R, class LD, class ST, bool TILED>
-__global__ void __launch_bounds__(BOX_THREADS, TILED ? 2 : 4)
+enum BoxKind { BOX_PAIR, BOX_ONE, BOX_TILED };
+template <typename R, class LD, class ST, BoxKind KIND>
+__global__ void __launch_bounds__(BOX_THREADS, KIND == BOX_PAIR ? 4 : 2)
 box_fft_kernel(LD ld, ST st, const BoxArgs* __restrict__ ap, const cpx<R>* __restrict__ tw,
                const int* __restrict__ tabs, R scale, int sign, unsigned nitem) {
   extern __shared__ unsigned char smem_raw[];
   cpx<R>* lds = reinterpret_cast<cpx<R>*>(smem_raw);
   const BoxArgs& a = *ap;
-  if constexpr (TILED) {
+  if constexpr (KIND == BOX_TILED) {
     box_persistent<R>(lds, ld, st, a, tw, tabs, scale, threadIdx.x, sign, nitem);
   } else {
     const unsigned nb = (unsigned)a.blocks(), it = blockIdx.x / nb;
@@ -956,13 +960,14 @@ box_fft_kernel(LD ld, ST st, const BoxArgs* __restrict__ ap, const cpx<R>* __res
     if (box_skipped(si, a, lb, O)) return;
     const int tid = threadIdx.x;
     box_twiddles_to_lds<R>(lds, a, tw, tid, BOX_THREADS);
-    box_load<R>(lds, BatchOf<LD>::at(ld, it), a, O, tid, BOX_THREADS, tabs);
+    constexpr bool ONE = KIND == BOX_ONE;
+    box_load<R, (ONE ? 2 : 1) * (sizeof(R) == 4 ? 8 : 4)>(lds, BatchOf<LD>::at(ld, it), a, O, tid, BOX_THREADS, tabs);
     __syncthreads();
     for (int i = 0; i < a.nsub; ++i) {
       box_dispatch<R>(lds, a, box_sub_at(a, i), tw, tid, BOX_THREADS, sign);
       __syncthreads();
     }
-    box_store<R>(lds, si, a, O, scale, tw, tid, BOX_THREADS, tabs);
+    box_store<R, ONE ? 8 : 2>(lds, si, a, O, scale, tw, tid, BOX_THREADS, tabs);
   }
 }
 
@@ -1009,6 +1014,12 @@ inline bool box_take_small(const BoxArgs& a, const BoxArgs& as, long n, long ncu
     return boxes > 4 * slots ? (double)boxes / (double)slots : (double)((boxes + slots - 1) / slots);
   };
   return rounds(ns, 2 * ncu) * (1.15 * as.elems + 0.15 * budget) <= rounds(nw, ncu) * a.elems;
+}
+
+// the kernel of a pass of nbox boxes (box_fft_kernel)
+inline BoxKind box_kind(const BoxArgs& a, long nbox, size_t lds_bytes, size_t lds_limit, bool small, long ncu) {
+  if (a.tiled) return BOX_TILED;
+  return 2 * lds_bytes > lds_limit || (!small && nbox <= ncu) ? BOX_ONE : BOX_PAIR;
 }
 
 }  // namespace gmod

@@ -1,5 +1,6 @@
 // fft_rule PREC NX NY NZ M MASK N: the box passes of N transforms on 256 CUs,
-// a letter each: w whole boxes, s small ones
+// a letter each: w whole boxes, s small ones, a capital where untiled boxes
+// run one per CU
 #include <cstdio>
 
 #include "../../pyrpa_amd/csrc/fftbox.h"
@@ -16,8 +17,14 @@ static void print(char** v) {
   p.build(nx, ny, nz, m, mask, budget, lds);
   q.build(nx, ny, nz, m, mask, budget, lds, budget / 4);
   const bool two = q.ok && q.fwd.size() == p.fwd.size();
-  for (size_t i = 0; i < p.fwd.size(); ++i)
-    putchar(two && box_take_small(p.fwd[i], q.fwd[i], atol(v[7]), 256, budget) ? 's' : 'w');
+  const long n = atol(v[7]), ncu = 256;
+  for (size_t i = 0; i < p.fwd.size(); ++i) {
+    const bool small = two && box_take_small(p.fwd[i], q.fwd[i], n, ncu, budget);
+    const BoxArgs& a = small ? q.fwd[i] : p.fwd[i];
+    const size_t shm = (size_t)(a.lds_elems + a.ntwl) * sizeof(cpx<R>);
+    const bool one = box_kind(a, a.blocks() * n, shm, lds, small, ncu) == BOX_ONE;
+    putchar(small ? (one ? 'S' : 's') : (one ? 'W' : 'w'));
+  }
   putchar('\n');
 }
 
