@@ -996,24 +996,21 @@ struct BoxPlan {
 // whole, 12.5 quarter.  A second round costs more than the idle CUs of the
 // whole boxes: 16x16x8 x 512, 128 boxes or 512: 15.1 and 18.6 us; 64x48 x 512,
 // 192 or 768: 17.7 and 26.7; from one whole box per CU on, the same or slower.
-// An untiled pass: where all of them run at once, two a CU, or by the rounds
-// (whole ones up to four). A round costs a whole box its elements, and two
-// quarter boxes 1.15 of one's (they overlap: 27x27x5 x 180, 28 us a grid in a
-// launch of its own, 22 in a batch of 9) plus 0.15 of the largest box (the waits
-// of a short one): 48x48x12 x 150 FP64 t pass, 576 boxes or 2304: 76.8 us whole,
-// 58.8 quarter; 36x36x5 x 288 FP32, 180 or 540: 27.2 and 44.5; 45x32 x 4096, 512
-// or 2048: 62.1 and 84.8. Of 132 transforms timed alone two take a side that is
-// slower by more than 5 % (96x42x6 x 288 FP32: 127 us whole, 144 quarter;
-// 50x64x4 x 300 FP64 t pass: 60 and 70).
+// An untiled pass: where all of them run at once, two a CU, or fill more than
+// five rounds (they overlap: 27x27x5 x 180, 28 us a grid in a launch of its own,
+// 22 in a batch of 9; 100x100x8 x 180 FP32 t pass 178 us whole, 117 quarter).
+// Between, by the rounds: one costs a whole box its elements, and two quarter
+// boxes 1.05 of one's plus 0.175 of the largest box (the waits of a short one):
+// 48x48x12 x 150 FP64 t pass, 576 boxes or 2304: 76.8 us whole, 58.8 quarter;
+// 36x36x5 x 288 FP32, 180 or 540: 27.2 and 44.5; 45x32 x 4096, 512 or 2048: 62.1
+// and 84.8. Of 132 transforms timed alone one takes a side that is slower by
+// more than 5 % (96x42x6 x 288 FP32: 127 us whole, 144 quarter).
 inline bool box_take_small(const BoxArgs& a, const BoxArgs& as, long n, long ncu, long budget) {
   if (as.blocks() == a.blocks()) return false;
   const long nw = a.blocks() * n, ns = as.blocks() * n;
   if (a.tiled) return nw < ncu && ns <= (as.tiled ? 1 : 2) * ncu;
-  if (ns <= 2 * ncu) return true;
-  auto rounds = [](long boxes, long slots) {
-    return boxes > 4 * slots ? (double)boxes / (double)slots : (double)((boxes + slots - 1) / slots);
-  };
-  return rounds(ns, 2 * ncu) * (1.15 * as.elems + 0.15 * budget) <= rounds(nw, ncu) * a.elems;
+  const long rw = (nw + ncu - 1) / ncu, rs = (ns + 2 * ncu - 1) / (2 * ncu);
+  return rs == 1 || rs > 5 || (double)rs * (1.05 * as.elems + 0.175 * budget) <= (double)rw * a.elems;
 }
 
 // the kernel of a pass of nbox boxes (box_fft_kernel)
