@@ -38,13 +38,16 @@ void rpa_solve(zd* out, BatchLayout Lo, const zd* A, BatchLayout La, long batch,
 // fits twice in the 160 KB of LDS), while the batch is short of the line below:
 // a lane per matrix takes one serial chain of any batch that fits the chip,
 // the wavefronts a time in proportion to the batch.  Lane and wave kernel, us:
-//   n = 1, 20000 matrices 30 and 33; 200000: 30 and 71
-//   n = 4, 6000: 161 and 128; 20000: 212 and 308; 200000: 1035 and 2564
-//   n = 9, 9000: 861 and 684; 16000: 858 and 1137; 48000: 1556 and 3234
-//   n = 16, 12000: 3878 and 3086; 24000: 5249 and 5516; 48000: 6788 and 11089
-//   n = 25, 24000: 17454 and 15054; 48000: 30771 and 29953
+//   n = 1, 9000 matrices 11 and 6; 24000: 15 and 11; 48000: 17 and 15
+//   n = 2, 16000: 24 and 21; 24000: 24 and 28; 48000: 26 and 48
+//   n = 5, 6000: 201 and 162; 9000: 202 and 224; 48000: 263 and 1028
+//   n = 9, 9000: 761 and 679; 12000: 769 and 884; 48000: 1123 and 3252
+//   n = 16, 12000: 3303 and 3065; 16000: 3541 and 3933; 48000: 5905 and 11085
+//   n = 25, 24000: 16157 and 15207; 48000: 24739 and 29924
 constexpr int EIG_WAVE_MAX = 64;
-inline bool eig_by_wave(long batch, int n) { return n <= EIG_WAVE_MAX && batch <= 9500 + 40L * n * n; }
+inline bool eig_by_wave(long batch, int n) {
+  return n <= EIG_WAVE_MAX && batch <= (n <= 2 ? 20000 : 7500 + 30L * n * n);
+}
 // max Re eig(alpha * A * W) per matrix (W = nullptr: identity)  (fchi.f90:373-389)
 void max_re_eig(double* out, const zd* A, BatchLayout La, long batch, int n, const double* W, double alpha,
                 int* err, hipStream_t s);

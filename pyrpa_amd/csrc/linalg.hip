@@ -1366,37 +1366,37 @@ __host__ __device__ int zhess_eig(zd* H, int n, zd* w, long st = 1) {
       sigma = abs1(e1 - d) < abs1(e2 - d) ? e1 : e2;
     }
     for (int k = l; k <= hi; ++k) HH(k, k) -= sigma;
-    // QR by Givens on rows (store rotations in the subdiagonal workspace)
-    double cs[64];
-    zd sn[64];
+    // QR sweep by Givens rotations; the columns of rotation k follow the rows
+    // of rotation k + 1, which do not touch them, so one rotation is kept (a
+    // table of them took 0.7 GB of private memory for a lane per matrix)
     const int nrot = hi - l;
     if (nrot > 64) return 2;
-    for (int k = l; k < hi; ++k) {
-      zd x = HH(k, k), y = HH(k + 1, k);
-      double ax = hypot(x.re, x.im), ay = hypot(y.re, y.im);
-      double r = hypot(ax, ay);
-      double c;
-      zd sv;
-      if (r == 0.0) { c = 1.0; sv = zd(0, 0); }
-      else if (ax == 0.0) { c = 0.0; sv = conj(y) * (1.0 / ay); }
-      else { zd ph = x * (1.0 / ax); c = ax / r; sv = ph * conj(y) * (1.0 / r); }
-      cs[k - l] = c;
-      sn[k - l] = sv;
-      for (int j = k; j <= hi; ++j) {
-        zd h1 = HH(k, j), h2 = HH(k + 1, j);
-        HH(k, j) = h1 * c + sv * h2;
-        HH(k + 1, j) = h2 * c - conj(sv) * h1;
+    double pc = 1.0;  // rotation k - 1
+    zd ps(0, 0);
+    for (int k = l; k <= hi; ++k) {
+      double c = 1.0;
+      zd sv(0, 0);
+      if (k < hi) {
+        zd x = HH(k, k), y = HH(k + 1, k);
+        double ax = hypot(x.re, x.im), ay = hypot(y.re, y.im);
+        double r = hypot(ax, ay);
+        if (r == 0.0) { c = 1.0; sv = zd(0, 0); }
+        else if (ax == 0.0) { c = 0.0; sv = conj(y) * (1.0 / ay); }
+        else { zd ph = x * (1.0 / ax); c = ax / r; sv = ph * conj(y) * (1.0 / r); }
+        for (int j = k; j <= hi; ++j) {
+          zd h1 = HH(k, j), h2 = HH(k + 1, j);
+          HH(k, j) = h1 * c + sv * h2;
+          HH(k + 1, j) = h2 * c - conj(sv) * h1;
+        }
       }
-    }
-    for (int k = l; k < hi; ++k) {
-      double c = cs[k - l];
-      zd sv = sn[k - l];
-      int rmax = k + 1 < hi ? k + 1 : hi;
-      for (int i = l; i <= rmax; ++i) {
-        zd h1 = HH(i, k), h2 = HH(i, k + 1);
-        HH(i, k) = h1 * c + h2 * conj(sv);
-        HH(i, k + 1) = h2 * c - h1 * sv;
-      }
+      if (k > l)
+        for (int i = l; i <= k; ++i) {
+          zd h1 = HH(i, k - 1), h2 = HH(i, k);
+          HH(i, k - 1) = h1 * pc + h2 * conj(ps);
+          HH(i, k) = h2 * pc - h1 * ps;
+        }
+      pc = c;
+      ps = sv;
     }
     for (int k = l; k <= hi; ++k) HH(k, k) += sigma;
   }
