@@ -46,7 +46,7 @@ void rpa_solve(zd* out, BatchLayout Lo, const zd* A, BatchLayout La, long batch,
 //   n = 25, 24000: 16157 and 15207; 48000: 24739 and 29924
 constexpr int EIG_WAVE_MAX = 64;
 inline bool eig_by_wave(long batch, int n) {
-  return n <= EIG_WAVE_MAX && batch <= (n <= 2 ? 20000 : 7500 + 30L * n * n);
+  return n <= EIG_WAVE_MAX && batch <= (n == 1 ? 50000 : n == 2 ? 20000 : 7500 + 30L * n * n);
 }
 // max Re eig(alpha * A * W) per matrix (W = nullptr: identity)  (fchi.f90:373-389)
 void max_re_eig(double* out, const zd* A, BatchLayout La, long batch, int n, const double* W, double alpha,

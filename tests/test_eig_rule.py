@@ -19,7 +19,7 @@ def by_wave(tmp_path_factory):
 
 
 @pytest.mark.parametrize("n,batch,wave", [
-    (1, 9000, True), (1, 200000, False), (2, 9000, True), (3, 6000, True), (3, 12000, False), (5, 12000, False), (2, 33, True), (2, 46000, False), (4, 514, True), (4, 2000, True),
+    (1, 9000, True), (1, 24000, True), (1, 200000, False), (2, 9000, True), (3, 6000, True), (3, 12000, False), (5, 12000, False), (2, 33, True), (2, 46000, False), (4, 514, True), (4, 2000, True),
     (4, 20000, False), (6, 6000, True), (6, 46000, False), (9, 514, True), (9, 6000, True), (9, 9000, True), (9, 12000, False),
     (9, 48000, False), (13, 9000, True), (13, 48000, False), (16, 130, True), (16, 9000, True), (16, 12000, True), (16, 24000, False),
     (20, 12000, True), (20, 16000, True), (20, 24000, False), (25, 24000, True), (25, 48000, False), (32, 12000, True), (40, 24000, True), (64, 514, True),

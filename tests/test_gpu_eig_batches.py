@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("over", [0, 1])
 def test_both_sides_of_the_line(n, over):
     import pyrpa_amd.flibs as F
-    nk = (20000 if n <= 2 else 7500 + 30 * n * n) + over
+    nk = (50000 if n == 1 else 7500 + 30 * n * n) + over
     rng = np.random.default_rng(n)
     a = rng.standard_normal((nk, n, n)) + 1j * rng.standard_normal((nk, n, n))
     a[7] = 0.0
