@@ -375,7 +375,7 @@ template void mirror_grid<double>(cpx<double>*, const cpx<double>*, int, int, in
 // again for each output that uses them, from the cache when they fit it.
 // One launch for all outputs; a launch per product wrote the running sum
 // back and read it again each time (the 54 products of a 3-orbital gap step
-// at 20x20x4 x 256: 290 us, now 106 us, 6.7 TB/s).
+// at 20x20x4 x 256: 290 us, now 107 us, 4.2 TB/s of grids counted once).
 template <typename R>
 __global__ void __launch_bounds__(TPB)
 k_contract(cpx<R>* __restrict__ out, const cpx<R>* __restrict__ A, const cpx<R>* __restrict__ B,
@@ -461,7 +461,8 @@ void sum_diff(zd* a, zd* b, long n, hipStream_t s) {
 }
 
 // ------------------------------------------------------------------ reductions
-// Latency-bound (a few MB at most): one launch and one wait per result.  The
+// One launch and one wait per result: latency-bound up to a few MB (the fields
+// of the 4-orbital 16x16x8 x 256 mesh are 67 MB each, bound by their bytes).  The
 // earlier form summed the 1024 partial results of a dot product in one thread
 // of a second launch (90 us, a dependent load per term) and copied the sum
 // back: 110 us on the device, now 15 with the wait.

@@ -747,7 +747,8 @@ k_vertex_gj(const zd* chi_in, zd* chi_out, long batch, long es, const VSparse* _
 // a wavefront, the LU waits for the whole work-group twice.  3 orbitals,
 // 27x27x5 x 90: 1295 us by columns, 719 by rows (registers for three or four
 // waves per SIMD spill: 1173, 1413); spinful 2 orbitals, 16x16 x 128: 740 us
-// with a wavefront per matrix in LDS, 87 by rows.
+// with a wavefront per matrix in LDS, 87 by rows.  Nchi = 4 stays with the
+// register kernel and 10 to 15 (several sites) with the LU: neither was compared.
 template <int N, int KIND>
 __global__ void __launch_bounds__(64 * GJ_WAVES) __attribute__((amdgpu_waves_per_eu(2)))
 k_vertex_rows(const zd* chi_in, zd* chi_out, long batch, long es, const VSparse* __restrict__ spg,
