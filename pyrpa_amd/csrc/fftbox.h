@@ -997,9 +997,10 @@ struct BoxPlan {
 // whole boxes: 16x16x8 x 512, 128 boxes or 512: 15.1 and 18.6 us; 64x48 x 512,
 // 192 or 768: 17.7 and 26.7; from one whole box per CU on, the same or slower.
 // An untiled pass: where all of them run at once, two a CU, or fill more than
-// five rounds (they overlap: 27x27x5 x 180, 28 us a grid in a launch of its own,
-// 22 in a batch of 9; 100x100x8 x 180 FP32 t pass 178 us whole, 117 quarter).
-// Between, by the rounds: one costs a whole box its elements, and two quarter
+// five rounds with nearly three elements a thread (they overlap: 27x27x5 x 180,
+// 28 us a grid in a launch of its own, 22 in a batch of 9; 100x100x8 x 180 FP32
+// t pass 178 us whole, 117 quarter; 128x128 x 1000 FP64 x pass, 1280 elements,
+// 171 and 225).  Else by the rounds: one costs a whole box its elements, and two quarter
 // boxes 1.05 of one's plus 0.175 of the largest box (the waits of a short one):
 // 48x48x12 x 150 FP64 t pass, 576 boxes or 2304: 76.8 us whole, 58.8 quarter;
 // 36x36x5 x 288 FP32, 180 or 540: 27.2 and 44.5; 45x32 x 4096, 512 or 2048: 62.1
@@ -1010,7 +1011,7 @@ inline bool box_take_small(const BoxArgs& a, const BoxArgs& as, long n, long ncu
   const long nw = a.blocks() * n, ns = as.blocks() * n;
   if (a.tiled) return nw < ncu && ns <= (as.tiled ? 1 : 2) * ncu;
   const long rw = (nw + ncu - 1) / ncu, rs = (ns + 2 * ncu - 1) / (2 * ncu);
-  return rs == 1 || rs > 5 || (double)rs * (1.05 * as.elems + 0.175 * budget) <= (double)rw * a.elems;
+  return rs == 1 || (rs > 5 && as.elems >= 1400) || (double)rs * (1.05 * as.elems + 0.175 * budget) <= (double)rw * a.elems;
 }
 
 // the kernel of a pass of nbox boxes (box_fft_kernel)

@@ -37,7 +37,7 @@ def test_tiled_passes(passes, prec, dims, mask, n, want):
 
 @pytest.mark.parametrize("prec,dims,mask,n,want", [
     (1, (18, 18, 1, 90), 7, 1, "s"), (1, (18, 14, 1, 150), 8, 1, "s"), (0, (48, 48, 12, 150), 8, 1, "s"),
-    (1, (80, 80, 4, 240), 8, 1, "s"), (0, (100, 100, 3, 720), 7, 1, "sss"), (0, (27, 27, 5, 180), 15, 9, "ss"),
+    (1, (80, 80, 4, 240), 8, 1, "s"), (0, (100, 100, 3, 720), 7, 1, "sss"), (0, (128, 128, 1, 1000), 1, 1, "W"), (0, (27, 27, 5, 180), 15, 9, "ss"),
     (1, (24, 24, 6, 200), 15, 21, "ws"), (1, (24, 24, 6, 200), 15, 15, "ws"), (0, (50, 64, 4, 300), 8, 1, "W"),
     (1, (36, 36, 5, 288), 8, 1, "W"), (0, (30, 30, 12, 140), 7, 1, "WW"), (1, (45, 32, 1, 4096), 7, 1, "W"),
     (1, (24, 45, 6, 2400), 8, 1, "W"), (0, (80, 80, 1, 1250), 7, 1, "W"), (1, (50, 15, 1, 800), 8, 1, "W"),
