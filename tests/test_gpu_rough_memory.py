@@ -27,7 +27,7 @@ def solve(L, ny):
     hamk = L.gen_ham(klist, HAM, RVEC)
     eig, uni = L.get_eig(hamk)
     olist, site = O.get_chi_orb_list(2, [2])
-    S, C = O.get_scmat(olist, site, 0.5, 0.1)
+    S, C = O.get_scmat(olist, site, 0.1, 0.02)  # below the Stoner instability of free levels
     sig, mu = L.mkself(S, C, kmap, invk, olist, hamk, eig, uni, MU, FILL, TEMP, NW, NX, ny, 1, False, False, eps=0.0,
                        pp=0.5, m_diis=1, scf_loop=2, sw_tail=False)
     return sig, mu
@@ -55,3 +55,19 @@ def test_flex_on_a_rough_mesh(ny, sources):
     assert np.abs(sig - ref[..., :1]).max() <= 1e-10 * np.abs(ref).max()
     grid = 16.0 * NX * ny * 2 * NW
     assert not sources or used <= (8 + 2 + 1 + sources + 4 + 4 + 0.5 + 0.5) * grid, used / grid
+
+
+@pytest.mark.parametrize("ny", [506, 1936])
+def test_increments_on_a_rough_mesh(ny):
+    """FP32 grids of 13 and 50 MB: the reference's transforms and the increments in several launches.  Tolerance of
+    the direct DFT's tests for its FP32 sums: 8 eps sqrt(nx + ny + m)."""
+    import pyrpa_amd.flibs as F
+    ref, mu1 = solve(O, 1)
+    try:
+        F.set_precision(1)
+        sig, mu = solve(F, ny)
+    finally:
+        F.set_precision(0)
+        F.release_memory()
+    tol = 8 * float(np.finfo(np.float32).eps) * np.sqrt(NX + ny + 2 * NW)
+    assert abs(mu - mu1) < tol and np.abs(sig - ref[..., :1]).max() <= tol * np.abs(ref).max()
